@@ -7,14 +7,13 @@
 // are occupied, so it is computed on 64-bit occupancy words and the particle
 // data are moved afterwards in one parallel pass:
 //
-//   1. classify (one thread per cell, or per cell and group of slots when the
-//      cells alone do not fill the chip; coalesced over the cell planes):
-//      in-cell test, domain test, destination (bisection seeded at the cell)
-//      as a neighbour code, occupancy/mover words, and a copy of every
-//      mover's coordinates and fields into a staging area indexed by its
-//      original slot;
+//   1. classify (one thread per cell, or per cell and chunk of 8 slots;
+//      coalesced over the cell planes): in-cell test, domain test,
+//      destination (bisection seeded at the cell) as a neighbour code,
+//      occupancy/mover words, and a copy of every mover's coordinates and
+//      fields into a staging area, packed per cell like the codes;
 //   2. 3^D colour phases (one thread per source cell of the colour): the
-//      reference's slot loop replayed on the occupancy words of the 3^D
+//      reference's slot loop replayed on the free-slot words of the 3^D
 //      neighbourhood (kept in LDS), recording for every slot that received a
 //      particle where that particle came from;
 //   3. scatter (threads as in classify): arrivals copy their staged data
@@ -36,50 +35,91 @@ using namespace jp;
 
 namespace {
 
-constexpr uint8_t kDel = 0xFE;
+// A mover's code is its destination cell in the 3^D neighbourhood: in 3D n =
+// (dx+1) + 3 (dy+1) + 9 (dz+1), in 2D the same with the row pitch of the tiled
+// phases' region (dx+1) + 42 (dy+1), so that a destination's word there is one
+// addition away.  Codes without a bit of 0x80 below: the phases' fast loop
+// takes them.  The centre's code fills the rows up to a multiple of 8.
+constexpr uint8_t kRare = 0x80;  // re-slotted in its own cell (the centre's code), or an
+                                 // arrival that fails the strict test of its destination
 // a mover whose destination is found from its staged position when its cell
 // is processed (far-jump path only: movers that jump more than one cell, and
 // arrivals there that fail the strict test of their new cell)
-constexpr uint8_t kFar = 0xFC;
+constexpr uint8_t kFar = 0xFF;
 constexpr int kFlagFar = 1;       // a mover jumps more than one cell
 constexpr int kFlagRejected = 2;  // split geometry rejected
-constexpr uint8_t kGap = 0x80;  // arrival fails the strict in-cell test of its destination
-// s_waitcnt immediate of gfx9 for vmcnt(0) with expcnt and lgkmcnt left free
-constexpr int kVmcnt0 = 0x0F70;
 
 __device__ inline double dnan() { return __builtin_nan(""); }
 
 struct MoveScratch {
     uint64_t* occ0;  // occupancy before the call
     uint64_t* occ;   // running occupancy
-    uint64_t* mov;   // slots holding a particle that moves when its cell's phase runs
-    uint64_t* arr;   // slots holding a particle that arrived during this call
-    uint64_t* tch;   // slots that received a particle at some point
-    uint8_t* code;   // per slot, 8 per word (word j*C + c): neighbour code / kDel, movers only
-    uint32_t* org;   // per slot: staged index of an arrival's record (layout: org_at)
+    uint64_t* mov;   // slots whose particle leaves or is re-slotted (classify)
+    uint64_t* rar;   // 2D: rare movers (kRare), read by the tiled phases
+    uint64_t* gap;   // rare movers, then also the slots whose arrival the cell re-slots (at
+                     // the end: slots that an arrival was removed from, and some of occ0)
+    uint8_t* code;   // the codes of the staged movers in slot order, 8 per word (word j*C + c)
+    uint16_t* org;   // per slot: where an arrival came from (org_code; layout: org_at)
+    uint32_t* orgf;  // far-jump path: the arrival's record (org: kOrgFar)
     char* stg;       // staged movers (layout: stg_coord; index: stage_index)
-    uint64_t* stm;   // 3D: each cell's staged movers (bit k), written by classify
+    uint64_t* stm;   // each cell's staged movers (bit k), written by classify
     int64_t S;       // slots
-    int64_t stride;  // 3D: record bytes (multiple of 8)
-    int64_t foff;    // 3D: byte offset of the fields in a record; 2D: of the field planes
-                     // (after the interleaved coordinates)
+    int64_t stride;  // record bytes (multiple of 8)
+    int64_t foff;    // byte offset of the fields in a record
 };
+
+// Slots of a cell that hold an arrival of this call.  A slot that was occupied
+// before the call keeps its particle unless that particle is a mover, which
+// leaves its slot when its own cell is processed: every other occupied slot
+// holds an arrival, so no words are kept for arrivals.  (Before its cell is
+// processed no mover has left: there the arrivals are occ & ~occ0.)
+__device__ inline uint64_t arrivals(uint64_t occ, uint64_t occ0, uint64_t mov) {
+    return occ & ~(occ0 & ~mov);
+}
 
 // Position of (cell, slot) in the origin array.  2D: plane-major like the
 // particle data (c + C k).  3D: cell-major (c K + k): each mover of a colour
 // phase stores one origin into a neighbour cell, and cell-major keeps a
 // wavefront's stores inside the few lines of its cells' neighbourhoods
-// (plane-major scatters them over an array larger than the last-level cache:
-// 452 MB at 128^3 with K = 54).
+// (plane-major scatters them over an array as large as the last-level cache).
 template <int D>
 __device__ inline uint32_t org_at(uint32_t c, uint32_t k, uint32_t C, uint32_t K) {
     return D == 2 ? c + C * k : c * K + k;
 }
+// An arrival's origin is a neighbour of its cell: the code of its move and its
+// rank among the source's staged movers fit 13 bits (half the bytes of a
+// record number for the phases' scattered stores and the scatter's reads).
+__device__ inline uint32_t org_code(uint32_t code, uint32_t rank) { return (code << 6) + rank; }
+constexpr uint32_t kOrgFar = 0xFFFFu;  // the record is in orgf
 
 template <int D>
 constexpr int kNB = D == 2 ? 9 : 27;
 template <int D>
 constexpr int kCenter = (kNB<D> - 1) / 2;
+
+constexpr int kPitch2 = 42;  // row length of the tiled 2D phases' region
+// neighbour n (0..3^D-1) <-> code
+template <int D>
+__device__ inline uint32_t code_of(int n) {
+    return D == 2 ? (uint32_t)(n + (kPitch2 - 3) * (n / 3)) : (uint32_t)n;
+}
+template <int D>
+__device__ inline int neighbour_of(uint32_t cd) {
+    return D == 2 ? (int)(cd - (kPitch2 - 3) * (cd / kPitch2)) : (int)cd;
+}
+// offset of a move's destination from its source, in cells (str: the strides
+// of dimensions 1.. in cells)
+template <int D>
+__device__ inline int move_offset(uint32_t cd, int str1, int str2) {
+    if (D == 2) {
+        const int q = (int)(cd / kPitch2);
+        return (int)cd - kPitch2 * q - 1 + str1 * (q - 1);
+    }
+    const int z = (int)(cd / 9), y = (int)(cd / 3) - 3 * z;
+    return (int)cd - 3 * (int)(cd / 3) - 1 + str1 * (y - 1) + str2 * (z - 1);
+}
+template <int D>
+constexpr uint32_t kHere = D == 2 ? kPitch2 + 1 : kCenter<3>;  // code of the cell itself
 
 // colour phase of a cell: offsets (o_1 outer ... o_D inner), 0-based
 template <int D>
@@ -185,54 +225,46 @@ __device__ inline ClassifySlots<D> classify_slots(const Grid<D>& g) {
     }
     return r;
 }
-// The record index of the chunk's first staged mover.  CHUNKS: the counts
-// of the cell's lower chunks, through LDS (every thread of the block calls
-// this once); else the running count of the thread's own cell.
-template <bool CHUNKS>
-__device__ inline int64_t chunk_record(int64_t c, int K, int k0, uint32_t stg, uint64_t staged,
-                                       int (&s_cnt)[8][64]) {
-    if constexpr (CHUNKS) {
-        const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-        s_cnt[w][lane] = __popc(stg);
-        __syncthreads();
-        int base = 0;
-        for (int v = 0; v < w; ++v) base += s_cnt[v][lane];
-        (void)k0;
-        (void)staged;
-        return c * K + base;
-    } else {
-        (void)s_cnt;
-        (void)k0;
-        (void)stg;
-        return c * K + __popcll(staged);
+// The per-cell words of classify.  CHUNKS: each chunk-thread puts its byte of
+// every word into LDS; after the block's barrier the words are whole, give
+// the chunk's record index (the cell's staged movers below it), and each
+// wavefront stores some of them (8 bytes per lane, contiguous; stored byte by
+// byte from the chunks the split classify took 84 us at 512^2, so 78).  Bytes
+// above the last chunk are masked on reading.
+enum { W_OCC = 0, W_MOV, W_STG, W_GAP, W_COUNT };
+struct CellWords {
+    uint64_t w[W_COUNT][64];
+    __device__ inline void put(int t, uint32_t v) {
+        reinterpret_cast<uint8_t*>(&w[t][threadIdx.x & 63])[threadIdx.x >> 6] = (uint8_t)v;
     }
+    __device__ inline uint64_t get(int t) const {
+        const int n = (int)(blockDim.x >> 6);
+        return w[t][threadIdx.x & 63] & (n == 8 ? ~0ull : ((1ull << (8 * n)) - 1));
+    }
+};
+// The codes of the staged movers, packed in slot order: a row of 68 bytes per
+// cell in LDS (17 dwords: the lanes' rows start on different banks), filled
+// with the centre's code first.
+constexpr int kRow = 68;
+template <int D>
+__device__ inline void fill_codes(uint32_t* row, int from, int to) {  // bytes from..to-1
+    for (int b = from >> 2; b < (to >> 2); ++b) row[b] = 0x01010101u * kHere<D>;
 }
-
-// The per-cell words of slot group kb..ke-1 (kb, and ke unless it is K, are
-// multiples of 8): whole words for a single group, else the group's bytes
-// (the last group also writes the zero bytes above K).
-__device__ inline void store_cell_words(const MoveScratch& ms, int64_t c, int kb, int ke, int K,
-                                        uint64_t occ, uint64_t mov) {
-    if (kb == 0 && ke == K) {
-        ms.occ0[c] = occ;
-        ms.occ[c] = occ;
-        ms.mov[c] = mov;
-        ms.arr[c] = 0;
-        ms.tch[c] = 0;
-        return;
-    }
-    uint8_t* __restrict__ o0 = reinterpret_cast<uint8_t*>(ms.occ0 + c);
-    uint8_t* __restrict__ o1 = reinterpret_cast<uint8_t*>(ms.occ + c);
-    uint8_t* __restrict__ mv = reinterpret_cast<uint8_t*>(ms.mov + c);
-    const int b1 = ke == K ? 8 : ke >> 3;
-    for (int b = kb >> 3; b < b1; ++b) {
-        o0[b] = (uint8_t)(occ >> (8 * b));
-        o1[b] = (uint8_t)(occ >> (8 * b));
-        mv[b] = (uint8_t)(mov >> (8 * b));
-    }
-    if (kb == 0) {
-        ms.arr[c] = 0;
-        ms.tch[c] = 0;
+__device__ inline uint64_t code_word(const uint32_t* row, int j) {
+    return (uint64_t)row[2 * j] | ((uint64_t)row[2 * j + 1] << 32);
+}
+template <int D>
+__device__ inline void store_word(const MoveScratch& ms, int64_t c, int t, uint64_t v) {
+    if (t == W_OCC) {
+        ms.occ0[c] = v;
+        ms.occ[c] = v;
+    } else if (t == W_MOV) {
+        ms.mov[c] = v;
+    } else if (t == W_STG) {
+        ms.stm[c] = v;
+    } else {
+        ms.gap[c] = v;
+        if (D == 2) ms.rar[c] = v;
     }
 }
 
@@ -245,7 +277,8 @@ __global__ void __launch_bounds__(kClassifyMax) k_mv_classify(Grid<D> g, CPtr3 c
                                                               int nargs, ArgPtrs args,
                                                               MoveScratch ms, int* flag) {
     constexpr bool CH = D == 2;
-    __shared__ int s_cnt[8][64];
+    __shared__ CellWords s_w;
+    __shared__ uint32_t s_code[(CH ? 64 : kBlock) * kRow / 4];
     const ClassifySlots<D> cs = classify_slots<D, CH>(g);
     if (!CH && !cs.live) return;  // (CH: every thread reaches the block's barrier)
     const int64_t c = cs.live ? cs.c : 0;
@@ -275,8 +308,11 @@ __global__ void __launch_bounds__(kClassifyMax) k_mv_classify(Grid<D> g, CPtr3 c
     const uint64_t occ = !cs.live ? 0ull
                          : (kb == 0 && ke == g.K) ? active_slots(index, c, C, g.K)
                                                   : active_slots_in(index, c, C, kb, ke);
-    uint64_t mov = 0, staged = 0;
+    uint64_t mov = 0, staged = 0, rare = 0;
     uint64_t* __restrict__ cw = reinterpret_cast<uint64_t*>(ms.code) + c;
+    uint32_t* row = s_code + (CH ? threadIdx.x & 63 : threadIdx.x) * (kRow / 4);
+    uint8_t* const crow = reinterpret_cast<uint8_t*>(row);
+    fill_codes<D>(row, kb, CH ? kb + 8 : 64);
     // chunks of slot planes walked in lockstep by the wavefront (coalesced
     // loads and stores across neighbouring cells)
     constexpr int B = 8;
@@ -288,8 +324,8 @@ __global__ void __launch_bounds__(kClassifyMax) k_mv_classify(Grid<D> g, CPtr3 c
 #pragma unroll
             for (int d = 0; d < D; ++d) pb[j][d] = on ? coords.p[d][c + C * (k0 + j)] : 0.0;
         }
-        uint64_t word = 0;
-        uint32_t mv8 = 0, stg = 0;
+        uint32_t cd8[2] = {0, 0};  // the chunk's codes, by slot
+        uint32_t mv8 = 0, stg = 0, rr8 = 0;
 #pragma unroll
         for (int j = 0; j < B; ++j) {
             const int k = k0 + j;
@@ -305,10 +341,8 @@ __global__ void __launch_bounds__(kClassifyMax) k_mv_classify(Grid<D> g, CPtr3 c
             }
             if (inc) continue;
             mv8 |= 1u << j;
-            uint8_t cd;
-            if (!indom) {
-                cd = kDel;
-            } else {
+            if (indom) {  // (else deleted: empty_particle! only)
+                uint32_t cd;
                 int n = 0, mult = 1;
                 bool far = false, inJ = true;
                 int64_t jump = 0;  // cells jumped (largest over the dimensions)
@@ -335,17 +369,40 @@ __global__ void __launch_bounds__(kClassifyMax) k_mv_classify(Grid<D> g, CPtr3 c
                     atomicMax(flag + 1, (int)(jump < (1 << 30) ? jump : (1 << 30)));
                     cd = kFar;
                 } else {
-                    cd = (uint8_t)n;
-                    if (n != kCenter<D> && !inJ) cd |= kGap;
+                    const bool rr = n == kCenter<D> || !inJ;
+                    cd = code_of<D>(n) | (rr ? kRare : 0u);
+                    rr8 |= (uint32_t)rr << j;
                 }
                 stg |= 1u << j;
+                cd8[j >> 2] |= cd << (8 * (j & 3));
             }
-            word |= (uint64_t)cd << (8 * j);
         }
-        if (mv8) cw[(k0 >> 3) * C] = word;
         mov |= (uint64_t)mv8 << k0;
+        rare |= (uint64_t)rr8 << k0;
         // the chunk's staged movers, packed after the cell's earlier ones
-        const int64_t o0 = chunk_record<CH>(c, g.K, k0, stg, staged, s_cnt);
+        if constexpr (CH) {  // (one chunk per thread)
+            s_w.put(W_OCC, (uint32_t)(occ >> k0));
+            s_w.put(W_MOV, mv8);
+            s_w.put(W_STG, stg);
+            s_w.put(W_GAP, rr8);
+            __syncthreads();
+            staged = s_w.get(W_STG) & ((1ull << k0) - 1);
+        }
+        const int r0 = __popcll(staged);
+#pragma unroll
+        for (int j = 0; j < B; ++j)
+            if ((stg >> j) & 1)
+                crow[r0 + __popc(stg & ((1u << j) - 1))] = (uint8_t)(cd8[j >> 2] >> (8 * (j & 3)));
+        const int64_t o0 = c * g.K + r0;
+        if constexpr (CH) {
+            __syncthreads();
+            if (cs.live) {
+                // (one code word per chunk-thread)
+                if (__popcll(s_w.get(W_STG)) > kb) cw[(kb >> 3) * C] = code_word(row, kb >> 3);
+                for (int t = (int)(threadIdx.x >> 6); t < W_COUNT; t += (int)(blockDim.x >> 6))
+                    store_word<D>(ms, c, t, s_w.get(t));
+            }
+        }
         if (cs.live) {
 #pragma unroll
             for (int j = 0; j < B; ++j)
@@ -358,12 +415,13 @@ __global__ void __launch_bounds__(kClassifyMax) k_mv_classify(Grid<D> g, CPtr3 c
         }
         staged |= (uint64_t)stg << k0;
     }
-    if (!cs.live) return;
-    store_cell_words(ms, c, kb, ke, g.K, occ, mov);
-    if constexpr (CH)
-        reinterpret_cast<uint8_t*>(ms.stm + c)[kb >> 3] = (uint8_t)(staged >> kb);
-    else
-        ms.stm[c] = staged;
+    if constexpr (!CH) {
+        store_word<D>(ms, c, W_OCC, occ);
+        store_word<D>(ms, c, W_MOV, mov);
+        store_word<D>(ms, c, W_STG, staged);
+        store_word<D>(ms, c, W_GAP, rare);
+        for (int j = 0; 8 * j < __popcll(staged); ++j) cw[j * C] = code_word(row, j);
+    }
 }
 
 // ------------------------------------------------------------ 2. colour phases
@@ -380,257 +438,266 @@ __device__ inline int64_t nb_cell(const Grid<D>& g, const int64_t* I, int n, boo
     return ok ? lin<D>(g.ni, J) : -1;
 }
 
-// Per thread in LDS: for each cell of the 3^D neighbourhood its occupancy
-// word and cell number (one 16-byte entry), and the cell's code words.  The
-// mover loop is one serial chain per thread with under two wavefronts per
-// SIMD, so it is kept short: per mover one LDS byte read (the code), then one
-// read of the destination's entry, 32-bit slot arithmetic (a move has fewer
-// than 2^32 slots), and this cell's own word in a register.
+// A cell of the 3^D neighbourhood in LDS: its free slots (0 outside the grid
+// and, while a cell's movers are dealt out, for the cell itself) and its number.
+constexpr uint32_t kNoCell = 0xFFFFFFFFu;
 struct alignas(16) NbEntry {
-    uint64_t occ;
-    uint32_t cell;  // 0xFFFFFFFF outside the grid (never a destination)
+    uint64_t free;
+    uint32_t cell;  // kNoCell: arrivals there are not recorded (outside the grid; another tile's)
     uint32_t pad;
 };
 
-// The reference slot loop of cell I in phase `phase`.  `stop`: the far-jump
-// path runs instead (checked after the cell's loads are issued).  FAR (the
-// far-jump path, cells in an order that keeps apart any two that interact):
-// kFar codes are resolved here from the staged positions, and a destination
-// beyond the 3^D neighbourhood is updated in the global words directly.
-template <int D, int BS, typename T, bool FAR>
-__device__ inline void phase_cell(const Grid<D>& g, const MoveScratch& ms, const int64_t* I,
-                                  int phase, bool stop, NbEntry (&s_nb)[kNB<D>][BS],
-                                  uint64_t (&s_cw)[8][BS], int& n_moved, int& n_del,
-                                  int& n_drop, int& n_far) {
-    const int64_t S = lin<D>(g.ni, I);
-    const int tid = threadIdx.x;
-    const int K = g.K;
-    const int64_t C = g.C;
-    const uint32_t S32 = (uint32_t)S, C32 = (uint32_t)C;
-    const uint64_t full = K == 64 ? ~0ull : ((1ull << K) - 1);
-    // everything this cell needs, in one round of independent loads: its
-    // mover/arrival words and code words, and occupancy words of its 3^D
-    // neighbourhood; in 2D also the neighbours' arrival and touched words.
-    // Cells of one colour are 3 apart, so no other thread of this phase reads
-    // or writes these neighbourhood words and the values loaded now are still
-    // current at the end (loading them late waits for this thread's earlier
-    // stores).  In 3D the 26 extra pairs would cost the occupancy they save.
-    constexpr bool kPre = D == 2;
-    uint64_t pend = ms.mov[S];
-    uint64_t arrS = ms.arr[S];
-    const uint64_t tchS = ms.tch[S];
-    const uint64_t stmS = ms.stm[S];  // staged movers (their record index)
-    uint64_t cw[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // movers' code bytes, 8 per word
-    {
-        const uint64_t* __restrict__ cp = reinterpret_cast<const uint64_t*>(ms.code) + S;
-        const int nw = (K + 7) >> 3;
+// The reference slot loop of a cell without rare movers: the n staged movers in
+// slot order, each to the first free slot >= starting_point of its
+// destination, which becomes starting_point.
+//
+// The loop is one serial chain per thread, on one or two wavefronts per SIMD,
+// and a phase lasts as long as its longest chain, so what counts is the
+// instructions per mover.  The codes come packed (no search for the next
+// mover), a dword of four at a time; a destination's entry is one LDS read,
+// issued a mover ahead (the previous mover's result is forwarded when both go
+// to the same cell); the chain itself is a few operations on masks (mask with
+// the slots >= starting_point, isolate the lowest bit, negate it for the next
+// mask).  Rows end with codes of the cell itself, whose entry has no free slot
+// meanwhile: no test for the last mover, and none for a full destination but
+// the one that guards the store.  Nothing else is kept per mover (arrivals
+// follow from the occupancy words at the end): ~32 instructions a mover.  A
+// loop over the mover bits with two dependent LDS reads, arrival words updated
+// per mover and an origin stored for every processing took 105 us for the
+// tiled 2D phases at 512^2 (32^2: 87, 3D 128^3: 30.9 per phase), this one 51
+// (38, 26.6).  Of that, origins stored for the tile's own cells only: 74 -> 58,
+// in 16 bits: 58 -> 51 (scattered stores, each a cache line).
+//
+// at(code): the entry of a code's destination.
+template <int D, bool STATS, typename At>
+__device__ inline void run_movers(int n, const uint32_t* row, const At& at,
+                                  uint16_t* __restrict__ org, uint32_t C32, uint32_t K,
+                                  int& n_moved) {
+    uint64_t ge = ~0ull;  // slots >= starting_point
+    uint32_t cw = row[0], cd = cw & 0xFFu;
+    NbEntry* to = &at(cd);
+    NbEntry* last = to;
+    uint64_t word = to->free, put = word;
+    uint32_t cell = to->cell;
+    for (int i = 0; i < n; i += 4) {
+        const uint32_t cnext = i + 4 < n ? row[(i >> 2) + 1] : 0x01010101u * kHere<D>;
 #pragma unroll
-        for (int j = 0; j < 8; ++j)
-            if (j < nw) cw[j] = cp[j * C];
+        for (int j = 0; j < 4; ++j) {
+            const uint32_t cd1 = j < 3 ? (cw >> (8 * (j + 1))) & 0xFFu : cnext & 0xFFu;
+            NbEntry* const to1 = &at(cd1);
+            const uint64_t word1 = to1->free;
+            const uint32_t cell1 = to1->cell;
+            const uint64_t fw = to == last ? put : word;
+            const uint64_t fr = fw & ge;
+            const uint64_t fb = fr & (0 - fr);
+            put = fw ^ fb;
+            last = to;
+            to->free = put;
+            const bool got = fr != 0;  // else find_free_memory found nothing: dropped
+            ge = got ? 0 - fb : ge;    // starting_point = free_idx
+            if (got & (cell != kNoCell))
+                org[org_at<D>(cell, (uint32_t)__builtin_ctzll(fb), C32, K)] =
+                    (uint16_t)org_code(cd, (uint32_t)(i + j));
+            if (STATS) n_moved += got;
+            to = to1;
+            word = word1;
+            cell = cell1;
+            cd = cd1;
+        }
+        cw = cnext;
     }
-    int64_t nbc[kNB<D>];
-    uint64_t was[kNB<D>], arrN[kNB<D>], tchN[kNB<D>];
-#pragma unroll
-    for (int n = 0; n < kNB<D>; ++n) {
-        bool v;
-        nbc[n] = nb_cell<D>(g, I, n, v);
-        const bool side = kPre && v && n != kCenter<D>;
-        was[n] = v ? ms.occ[nbc[n]] : ~0ull;  // outside the grid: never free
-        arrN[n] = side ? ms.arr[nbc[n]] : 0ull;
-        tchN[n] = side ? ms.tch[nbc[n]] : 0ull;
-    }
-    if (stop || !pend) return;  // far-jump path, or nothing leaves or re-slots here
-#pragma unroll
-    for (int n = 0; n < kNB<D>; ++n) s_nb[n][tid] = NbEntry{was[n], (uint32_t)nbc[n], 0u};
-#pragma unroll
-    for (int j = 0; j < 8; ++j) s_cw[j][tid] = cw[j];
-    uint64_t occC = was[kCenter<D>];  // this cell's occupancy
-    uint64_t selfm = 0;  // slots that received a re-slotted particle of this cell
-    uint64_t selfins = 0;
-    int sp = 0;
-    while (pend) {
-        const int ip = __builtin_ctzll(pend);
-        pend &= pend - 1;
-        const uint64_t bit = 1ull << ip;
-        const uint8_t code = reinterpret_cast<const uint8_t*>(&s_cw[ip >> 3][tid])[ip & 7];
-        // a mover of this cell: its staged record; an arrival: the record
-        // its origin staged
-        uint32_t origin = (uint32_t)stage_index<D>(S, K, stmS & (bit - 1));
-        if (arrS & bit) {  // rare: an arrival of this call moves on
-            origin = ms.org[org_at<D>(S32, (uint32_t)ip, C32, (uint32_t)K)];
-            // wait here, on the rare path: otherwise the loop head waits for
-            // the load on every iteration, and with it (one counter for loads
-            // and stores) for the previous iteration's store
-            __builtin_amdgcn_s_waitcnt(kVmcnt0);
-        }
-        uint8_t cd = (selfm & bit) ? (uint8_t)kCenter<D> : code;
-        occC &= ~bit;  // empty_particle! on the source slot
-        arrS &= ~bit;
-        selfm &= ~bit;
-        if (cd == kDel) {
-            ++n_del;
-            continue;
-        }
-        if constexpr (FAR) {
-            if (cd == kFar) {
-                // the destination from the staged position: bisection seeded
-                // at this cell (FP64), the cell + floor(u) (split, whose staged
-                // offset is renormalised to it here, for the scatter)
-                int64_t J[D];
-                bool near = true, inJ = true;
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    const T q = stg_coord<D, T>(ms, origin, d);
-                    if constexpr (std::is_same<T, float>::value) {
-                        const int sd = (int)floorf(q);
-                        J[d] = I[d] + sd;
-                        stg_coord<D, T>(ms, origin, d) = (float)((double)q - (double)sd);
-                    } else {
-                        J[d] = find_cell(q, g.xv[d], I[d]);
-                        const double xl = g.xv[d].x[J[d]];
-                        inJ = inJ && xl < q && q < xl + g.xv[d].dx[J[d]];
-                    }
-                    near = near && J[d] - I[d] <= 1 && I[d] - J[d] <= 1;
-                }
-                if (near) {  // inside the neighbourhood: the usual path
-                    int nn = 0, mult = 1;
-#pragma unroll
-                    for (int d = 0; d < D; ++d) {
-                        nn += (int)(J[d] - I[d] + 1) * mult;
-                        mult *= 3;
-                    }
-                    cd = (uint8_t)nn;
-                    if (nn != kCenter<D> && !inJ) cd |= kGap;
-                } else {
-                    ++n_far;
-                    const int64_t dcn = lin<D>(g.ni, J);
-                    const uint64_t od = ms.occ[dcn];
-                    const uint64_t fr = ~od & full & (~0ull << sp);
-                    if (!fr) {
-                        ++n_drop;
-                        continue;
-                    }
-                    const int f = __builtin_ctzll(fr);
-                    sp = f;
-                    const uint64_t fb = 1ull << f;
-                    ++n_moved;
-                    ms.org[org_at<D>((uint32_t)dcn, (uint32_t)f, C32, (uint32_t)K)] = origin;
-                    ms.occ[dcn] = od | fb;
-                    atomicOr(reinterpret_cast<unsigned long long*>(ms.arr + dcn),
-                             (unsigned long long)fb);
-                    atomicOr(reinterpret_cast<unsigned long long*>(ms.tch + dcn),
-                             (unsigned long long)fb);
-                    // an arrival that fails the strict test of its new cell is
-                    // looked up again when that cell comes later: in a later
-                    // phase, or later in this one (a jump by a multiple of 3
-                    // cells keeps the colour; cells of a phase go in linear
-                    // order)
-                    const int pj = phase_of<D>(J);
-                    if (!inJ && (pj > phase || (pj == phase && dcn > S))) {
-                        atomicOr(reinterpret_cast<unsigned long long*>(ms.mov + dcn),
-                                 (unsigned long long)fb);
-                        ms.code[((f >> 3) * C + dcn) * 8 + (f & 7)] = kFar;
-                    }
-                    continue;
-                }
-            }
-        }
-        const int n = cd & 0x7F;
-        const NbEntry nb = s_nb[n][tid];
-        const uint32_t dcn = nb.cell;
-        const uint64_t od = n == kCenter<D> ? occC : nb.occ;
-        const uint64_t fr = ~od & full & (~0ull << sp);
-        // (classify only gives destinations inside the grid; testing the cell
-        // number here makes its LDS read go out with the occupancy read)
-        if (!fr || dcn == 0xFFFFFFFFu) {  // find_free_memory found nothing: dropped
-            ++n_drop;
-            continue;
-        }
-        const int f = __builtin_ctzll(fr);
-        sp = f;  // starting_point = free_idx
-        const uint64_t fb = 1ull << f;
-        s_nb[n][tid].occ = od | fb;  // (the centre's LDS copy is not read)
-        ++n_moved;
-        ms.org[org_at<D>(dcn, (uint32_t)f, C32, (uint32_t)K)] = origin;
-        if (n == kCenter<D>) {
-            occC |= fb;
-            arrS |= fb;
-            selfins |= fb;
-            if (f > ip) {  // the slot loop will reach this particle again
-                pend |= fb;
-                selfm |= fb;
-            }
-        } else if (cd & kGap) {
-            // the arrival fails the strict test of its new cell: when that cell's
-            // phase comes later, it is re-slotted there (bisection returns that cell)
-            const int64_t Dc = dcn;
-            int64_t J[D];
-            unlin<D>(g.ni, Dc, J);
-            if (phase_of<D>(J) > phase) {
-                ms.mov[Dc] |= fb;
-                // (the far-jump path looks the destination up again, as the
-                // reference does)
-                ms.code[((f >> 3) * C + Dc) * 8 + (f & 7)] = FAR ? kFar : (uint8_t)kCenter<D>;
-            }
-        }
-    }
-#pragma unroll
-    for (int n = 0; n < kNB<D>; ++n) {
-        if (n == kCenter<D>) continue;
-        const NbEntry nb = s_nb[n][tid];
-        const uint32_t dn = nb.cell;
-        if (dn == 0xFFFFFFFFu) continue;
-        const uint64_t now = nb.occ;
-        if (now != was[n]) {
-            const uint64_t ins = now & ~was[n];
-            ms.occ[dn] = now;
-            if constexpr (kPre) {
-                ms.arr[dn] = arrN[n] | ins;
-                ms.tch[dn] = tchN[n] | ins;
-            } else {
-                // no other thread of the phase touches these words: an atomic
-                // OR without return updates them with no load to wait for (a
-                // load here would also wait for every earlier store)
-                atomicOr(reinterpret_cast<unsigned long long*>(ms.arr + dn),
-                         (unsigned long long)ins);
-                atomicOr(reinterpret_cast<unsigned long long*>(ms.tch + dn),
-                         (unsigned long long)ins);
-            }
-        }
-    }
-    ms.occ[S] = occC;
-    ms.arr[S] = arrS;
-    ms.tch[S] = tchS | selfins;
-    ms.mov[S] = 0;
 }
 
-// one colour phase, one thread per colour cell
-template <int D, int BS>
+// The same for a cell with rare movers (one re-slotted in its own cell, one
+// that its destination will re-slot, an arrival of this call that failed the
+// strict test of this cell), every case handled.  `pend`: slots to visit, on
+// return the visited ones (re-slotted particles met again included); returns
+// the cell's free slots.  later(code, entry, bit): the destination re-slots the
+// arrival when its phase comes later.
+template <int D, bool STATS, typename At, typename Later>
+__device__ inline uint64_t run_rare(uint64_t& pend, uint64_t mov, uint64_t stm,
+                                          uint64_t free, const uint8_t* codes, const At& at,
+                                          const Later& later, uint16_t* org, uint32_t S32,
+                                          uint32_t C32, uint32_t K, int& n_moved, int& n_drop) {
+    uint64_t ge = ~0ull, left = pend, again = 0;
+    while (left) {
+        const int ip = __builtin_ctzll(left);
+        const uint64_t bit = 1ull << ip;
+        left &= left - 1;
+        free |= bit;  // empty_particle! on the source slot
+        uint32_t cd = kHere<D>, origin;
+        if (!(mov & bit)) {  // an arrival (of another cell, or re-slotted here): stays here
+            origin = org[org_at<D>(S32, (uint32_t)ip, C32, K)];
+        } else if (stm & bit) {
+            const int r = __popcll(stm & (bit - 1));
+            cd = codes[r];
+            origin = org_code(cd & 0x7Fu, (uint32_t)r);
+        } else {
+            continue;  // deleted
+        }
+        const uint32_t n = cd & 0x7Fu;
+        const bool here = n == kHere<D>;
+        NbEntry& to = at(n);
+        const uint64_t fw = here ? free : to.free, fr = fw & ge;
+        if (!fr) {  // find_free_memory found nothing
+            if (STATS) ++n_drop;
+            continue;
+        }
+        const uint64_t fb = fr & (0 - fr);
+        const int f = __builtin_ctzll(fb);
+        ge = 0 - fb;
+        if (STATS) ++n_moved;
+        if (to.cell != kNoCell)
+            org[org_at<D>(to.cell, (uint32_t)f, C32, K)] = (uint16_t)origin;
+        if (here) {
+            free ^= fb;
+            if (f > ip) {  // the slot loop reaches it again
+                left |= fb;
+                again |= fb;
+            }
+        } else {
+            to.free = fw ^ fb;
+            if (cd & kRare) later(n, to, fb);
+        }
+    }
+    pend |= again;
+    return free;
+}
+
+// One cell of a phase.  free: its free slots; gap: its word of rare movers and
+// arrivals to re-slot, on return with the slots re-slotted here added.  Returns
+// the free slots after it.
+template <int D, bool STATS, typename At, typename Later>
+__device__ inline uint64_t run_cell(uint64_t mov, uint64_t stm, uint64_t& gap, uint64_t free,
+                                    const uint32_t* row, const At& at, const Later& later,
+                                    uint16_t* __restrict__ org, uint32_t S32, uint32_t C32,
+                                    uint32_t K, int& n_moved, int& n_del, int& n_drop) {
+    if (STATS) n_del += __popcll(mov & ~stm);
+    NbEntry& own = at(kHere<D>);
+    uint64_t after;
+    if (gap) {
+        uint64_t pend = mov | gap;
+        after = run_rare<D, STATS>(pend, mov, stm, free, reinterpret_cast<const uint8_t*>(row),
+                                   at, later, org, S32, C32, K, n_moved, n_drop);
+        gap |= pend & ~mov;
+    } else {
+        own.free = 0;
+        int moved = 0;
+        const int n = __popcll(stm);
+        if (n) run_movers<D, STATS>(n, row, at, org, C32, K, moved);
+        after = free | mov;
+        if (STATS) {
+            n_moved += moved;
+            n_drop += n - moved;
+        }
+    }
+    own.free = after;
+    return after;
+}
+
+__device__ inline void put_codes(uint32_t* row, const uint64_t (&w)[8], int nw) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        if (j < nw) {
+            row[2 * j] = (uint32_t)w[j];
+            row[2 * j + 1] = (uint32_t)(w[j] >> 32);
+        }
+}
+__device__ inline void load_codes(const MoveScratch& ms, uint32_t S32, uint32_t C32, int nw,
+                                  uint64_t (&w)[8]) {
+    const uint64_t* __restrict__ cp = reinterpret_cast<const uint64_t*>(ms.code) + S32;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) w[j] = j < nw ? cp[(int64_t)j * C32] : 0ull;
+}
+
+// one colour phase, one thread per colour cell; the neighbourhood's entries in
+// a column of LDS per thread
+template <int D, int BS, bool STATS>
 __global__ void __launch_bounds__(BS) k_mv_phase(Grid<D> g, MoveScratch ms, Off3 off, int phase,
                                                  const int* __restrict__ flag, jp_stats* st) {
     __shared__ NbEntry s_nb[kNB<D>][BS];
-    __shared__ uint64_t s_cw[8][BS];
-    const int stop = *flag;
-    int n_moved = 0, n_del = 0, n_drop = 0, n_far = 0;
-    int64_t t = blockIdx.x * (int64_t)BS + threadIdx.x, total = 1, ncol[D], I[D];
+    __shared__ uint32_t s_code[BS * kRow / 4];
+    const int stop = *flag;  // far-jump path, or rejected grid: nothing moves here
+    int n_moved = 0, n_del = 0, n_drop = 0;
+    // (a phase has fewer than 2^31 cells: 32-bit divisions)
+    uint32_t t = blockIdx.x * BS + threadIdx.x, ncol[D];
+    int I[D];
+    bool ok = true;
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-        ncol[d] = (g.ni[d] + 2) / 3;
-        total *= ncol[d];
+        ncol[d] = ((uint32_t)g.ni[d] + 2) / 3;
+        const uint32_t q = d < D - 1 ? t / ncol[d] : 0;
+        I[d] = 3 * (int)(t - q * ncol[d]) + off.o[d];
+        ok = ok && I[d] < (int)g.ni[d];
+        t = q;
     }
-    bool ok = t < total;
+    if (ok) {
+        // everything the cell needs, in one round of independent loads (cells
+        // of one colour are 3 apart: no other thread of this phase touches
+        // these neighbourhood words)
+        uint32_t str[D], S32 = 0;
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-        I[d] = 3 * (t % ncol[d]) + off.o[d];
-        t /= ncol[d];
-        ok = ok && I[d] < g.ni[d];
+        for (int d = 0; d < D; ++d) {
+            str[d] = d == 0 ? 1u : str[d - 1] * (uint32_t)g.ni[d - 1];
+            S32 += (uint32_t)I[d] * str[d];
+        }
+        const int tid = threadIdx.x;
+        const uint32_t K = (uint32_t)g.K, C32 = (uint32_t)g.C;
+        const uint64_t full = K == 64 ? ~0ull : ((1ull << K) - 1);
+        const uint64_t mov = ms.mov[S32], stm = ms.stm[S32];
+        uint64_t gap = ms.gap[S32];
+        const int nw = ((int)K + 7) >> 3;
+        uint64_t cw[8], word[kNB<D>];
+        uint32_t cell[kNB<D>], in = 0;
+        load_codes(ms, S32, C32, nw, cw);
+#pragma unroll
+        for (int n = 0; n < kNB<D>; ++n) {
+            bool v = true;
+            uint32_t c = S32;
+            int r = n;
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                const int o = r % 3 - 1;
+                r /= 3;
+                v = v && I[d] + o >= 0 && I[d] + o < (int)g.ni[d];
+                c += (uint32_t)(o * (int)str[d]);
+            }
+            cell[n] = c;
+            word[n] = v ? ms.occ[c] : ~0ull;
+            in |= (uint32_t)v << n;
+        }
+        if (!stop && (mov | gap)) {
+#pragma unroll
+            for (int n = 0; n < kNB<D>; ++n) s_nb[n][tid] = NbEntry{~word[n] & full, cell[n], 0u};
+            uint32_t* const row = s_code + tid * (kRow / 4);
+            put_codes(row, cw, nw);
+            const uint64_t gap0 = gap;
+            auto at = [&](uint32_t cd) -> NbEntry& {
+                return s_nb[D == 2 ? neighbour_of<D>(cd) : (int)cd][tid];
+            };
+            auto later = [&](uint32_t, NbEntry& to, uint64_t fb) {
+                int64_t J[D];
+                unlin<D>(g.ni, (int64_t)to.cell, J);
+                if (phase_of<D>(J) > phase) ms.gap[to.cell] |= fb;
+            };
+            run_cell<D, STATS>(mov, stm, gap, s_nb[kCenter<D>][tid].free, row, at, later, ms.org,
+                               S32, C32, K, n_moved, n_del, n_drop);
+            // all words of the neighbourhood (unchanged ones too: comparing
+            // would hold the old words in registers)
+#pragma unroll
+            for (int n = 0; n < kNB<D>; ++n)
+                if ((in >> n) & 1) {
+                    const NbEntry e = s_nb[n][tid];
+                    ms.occ[e.cell] = ~e.free & full;
+                }
+            if (gap != gap0) ms.gap[S32] = gap;
+        }
     }
-    if (ok)
-        phase_cell<D, BS, double, false>(g, ms, I, phase, stop != 0, s_nb, s_cw, n_moved, n_del,
-                                         n_drop, n_far);
-    stat_add(st, ST_MOVED, n_moved);
-    stat_add(st, ST_DELETED, n_del);
-    stat_add(st, ST_DROPPED, n_drop);
+    if (STATS) {
+        stat_add(st, ST_MOVED, n_moved);
+        stat_add(st, ST_DELETED, n_del);
+        stat_add(st, ST_DROPPED, n_drop);
+    }
 }
 
 // ------------------------------------------------------------ 2'. 2D phases in tiles
@@ -656,10 +723,10 @@ __global__ void __launch_bounds__(BS) k_mv_phase(Grid<D> g, MoveScratch ms, Off3
 // dimension 0, 10 below and 18 above in dimension 1.
 //
 // Tiles overlap, so a halo processing also runs in the tile that owns it;
-// both compute the same slots from the same exact inputs.  Every processing
-// here stores its origins (equal values where tiles overlap), since a later
-// phase of this workgroup reads the origin of an arrival that moves on;
-// counts and final words come from owned cells only.
+// both compute the same slots from the same exact inputs.  Origins, counts and
+// final words come from owned cells only.  (An arrival that is re-slotted has
+// its origin read again, but stays in its cell: in a cell of another tile
+// neither the read nor the store matters.)
 //
 // A pending slot that holds an arrival of this call is always re-slotted in
 // its own cell (an arrival that fails the strict test of its new cell, or a
@@ -677,11 +744,9 @@ __global__ void __launch_bounds__(BS) k_mv_tiles2(Grid<2> g, MoveScratch ms,
     constexpr int RY = TY + kTileHalo1Lo + kTileHalo1Hi;
     constexpr int R = RX * RY;
     static_assert(((RX + 2) / 3) * ((RY + 2) / 3) <= BS, "one cell per thread and phase");
-    __shared__ uint64_t s_occ[R], s_mov[R], s_arr[R], s_tch[R];
-    // the code bytes of the cell each thread is processing: a row of 68
-    // bytes per thread (slot k at byte k; 17 dwords, so the lanes' rows start
-    // on different banks)
-    constexpr int kRow = 68;
+    static_assert(RX == kPitch2, "the codes' row pitch");
+    __shared__ NbEntry s_nb[R];
+    __shared__ uint64_t s_gap[R];
     __shared__ uint32_t s_code[BS * kRow / 4];
     if (*flag) return;  // far jump or rejected grid: nothing moves here
     const int n0 = (int)g.ni[0], n1 = (int)g.ni[1];
@@ -697,166 +762,92 @@ __global__ void __launch_bounds__(BS) k_mv_tiles2(Grid<2> g, MoveScratch ms,
     const int gy0 = ty0 - kTileHalo1Lo > 0 ? ty0 - kTileHalo1Lo : 0;
     const int gy1 = ty1 + kTileHalo1Hi < n1 - 1 ? ty1 + kTileHalo1Hi : n1 - 1;
     const int rw = gx1 - gx0 + 1, rh = gy1 - gy0 + 1;
+    const uint32_t K = (uint32_t)g.K;
+    const uint32_t C32 = (uint32_t)g.C;
+    const uint64_t full = K == 64 ? ~0ull : ((1ull << K) - 1);
     for (int i = threadIdx.x; i < rw * rh; i += BS) {
         const int x = i % rw, y = i / rw;
         const uint32_t c = (uint32_t)(gx0 + x) + (uint32_t)n0 * (uint32_t)(gy0 + y);
         const int r = x + RX * y;
-        s_occ[r] = ms.occ0[c];
-        s_mov[r] = ms.mov[c];
-        s_arr[r] = 0;
-        s_tch[r] = 0;
+        const bool own = tx0 <= gx0 + x && gx0 + x <= tx1 && ty0 <= gy0 + y && gy0 + y <= ty1;
+        s_nb[r] = NbEntry{~ms.occ0[c] & full, own ? c : kNoCell, 0u};
+        s_gap[r] = ms.rar[c];  // (ms.gap: other tiles may have written theirs)
     }
     __syncthreads();
-    const int K = g.K;
-    const uint32_t C32 = (uint32_t)g.C;
-    const uint64_t full = K == 64 ? ~0ull : ((1ull << K) - 1);
-    const int nw = (K + 7) >> 3;
-    const uint8_t* __restrict__ sc = reinterpret_cast<const uint8_t*>(s_code) + threadIdx.x * kRow;
+    const int nw = ((int)K + 7) >> 3;
+    uint32_t* const row = s_code + threadIdx.x * (kRow / 4);
     int n_moved = 0, n_del = 0, n_drop = 0;
     // the colour-p cells whose processing is exact in the region: x = vx +
-    // 3i (i < cx), y = vy + 3j (j < cy)
-    auto box = [&](int p, int& vx, int& vy, int& cx, int& cy) {
+    // 3i (i < cx), y = vy + 3j (j < cy); this thread's one of them
+    auto my_cell = [&](int p, int& x, int& y) {
         const int ax = gx0 == 0 ? 0 : gx0 - cone_lo(p, 0) + 1;
         const int bx = gx1 == n0 - 1 ? n0 - 1 : gx1 - cone_hi(p, 0) - 1;
         const int ay = gy0 == 0 ? 0 : gy0 - cone_lo(p, 1) + 1;
         const int by = gy1 == n1 - 1 ? n1 - 1 : gy1 - cone_hi(p, 1) - 1;
-        vx = ax + (p / 3 - ax % 3 + 3) % 3;
-        vy = ay + (p % 3 - ay % 3 + 3) % 3;
-        cx = vx <= bx ? (bx - vx) / 3 + 1 : 0;
-        cy = vy <= by ? (by - vy) / 3 + 1 : 0;
+        const int vx = ax + (p / 3 - ax % 3 + 3) % 3;
+        const int vy = ay + (p % 3 - ay % 3 + 3) % 3;
+        const int cx = vx <= bx ? (bx - vx) / 3 + 1 : 0;
+        const int cy = vy <= by ? (by - vy) / 3 + 1 : 0;
+        const int t = threadIdx.x;
+        if (t >= cx * cy) return false;
+        x = vx + 3 * (t % cx);
+        y = vy + 3 * (t / cx);
+        return true;
     };
-    auto load_codes = [&](uint32_t S32, uint64_t (&w)[8]) {
-        const uint64_t* __restrict__ cp = reinterpret_cast<const uint64_t*>(ms.code) + S32;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) w[j] = j < nw ? cp[(int64_t)j * C32] : 0ull;
-    };
-    auto cell_at = [&](int vx, int vy, int cx, int t) {
-        return (uint32_t)(vx + 3 * (t % cx)) + (uint32_t)n0 * (uint32_t)(vy + 3 * (t / cx));
-    };
-    // the code words of each thread's first cell of a phase are loaded one
-    // phase ahead, so that they are in flight during the phase before
-    uint64_t nxt[8];
-    {
-        int vx, vy, cx, cy;
-        box(0, vx, vy, cx, cy);
-        if ((int)threadIdx.x < cx * cy) load_codes(cell_at(vx, vy, cx, threadIdx.x), nxt);
-    }
-    for (int p = 0; p < kNB<2>; ++p) {
-        const int col0 = p / 3, col1 = p % 3;
-        int vx, vy, cx, cy;
-        box(p, vx, vy, cx, cy);
-        if ((int)threadIdx.x < cx * cy) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if (j < nw) {
-                    s_code[threadIdx.x * (kRow / 4) + 2 * j] = (uint32_t)nxt[j];
-                    s_code[threadIdx.x * (kRow / 4) + 2 * j + 1] = (uint32_t)(nxt[j] >> 32);
-                }
-        }
-        if (p + 1 < kNB<2>) {
-            int wx, wy, dx_, dy_;
-            box(p + 1, wx, wy, dx_, dy_);
-            if ((int)threadIdx.x < dx_ * dy_) load_codes(cell_at(wx, wy, dx_, threadIdx.x), nxt);
-        }
-        const int t = threadIdx.x;  // at most one cell of the colour per thread
-        uint64_t pend = 0;
-        int x = 0, y = 0, r = 0;
-        if (t < cx * cy) {
-            x = vx + 3 * (t % cx);
-            y = vy + 3 * (t / cx);
-            r = (x - gx0) + RX * (y - gy0);
-            pend = s_mov[r];
-        }
-        if (pend) {
-            const bool own = tx0 <= x && x <= tx1 && ty0 <= y && y <= ty1;
+    // the words and code words of a phase's cell are loaded one phase ahead,
+    // so that they are in flight during the phase before
+    uint64_t nxt[8], mov = 0, stm = 0;
+    int x = 0, y = 0;
+    auto fetch = [&](int p) {
+        const bool ok = my_cell(p, x, y);
+        if (ok) {
             const uint32_t S32 = (uint32_t)x + (uint32_t)n0 * (uint32_t)y;
-            // neighbours inside the grid (bit n)
-            uint32_t ingm = 0;
-#pragma unroll
-            for (int n = 0; n < kNB<2>; ++n) {
-                const int jx = x + n % 3 - 1, jy = y + n / 3 - 1;
-                ingm |= (uint32_t)(jx >= 0 && jx < n0 && jy >= 0 && jy < n1) << n;
-            }
-            uint64_t occC = s_occ[r], arrS = s_arr[r], tchS = s_tch[r];
-            uint64_t free_sp = full;  // slots >= starting_point
-            // a mover of this cell: its packed record, the cell's staged
-            // movers below it (the loop visits the cell's own movers in slot
-            // order, each once; the deleted ones are not staged)
-            uint32_t rec = S32 * (uint32_t)K;
-            while (pend) {
-                const int ip = __builtin_ctzll(pend);
-                pend &= pend - 1;
-                uint32_t cd = sc[ip];
-                const uint64_t bit = 1ull << ip;
-                occC &= ~bit;  // empty_particle! on the source slot
-                uint32_t origin = rec;
-                rec += (!(arrS & bit) && cd != kDel) ? 1u : 0u;
-                if (arrS & bit) {  // rare: an arrival of this call is re-slotted
-                    origin = ms.org[org_at<2>(S32, (uint32_t)ip, C32, (uint32_t)K)];
-                    // waited for here, on the rare path: a wait at the loop
-                    // head would also wait for the loop's origin stores (one
-                    // counter for vector loads and stores)
-                    __builtin_amdgcn_s_waitcnt(kVmcnt0);
-                    arrS &= ~bit;
-                    cd = kCenter<2>;
-                }
-                if (cd == kDel) {
-                    if (STATS) n_del += own;
-                    continue;
-                }
-                const int n = cd & 0x7F;
-                const int q3 = (n * 11) >> 5;  // n / 3 for n < 9
-                const int dx = n - 3 * q3 - 1, dy = q3 - 1;
-                int rn = r + dx + RX * dy;  // inside the region when in the grid
-                rn = rn < 0 ? 0 : (rn > R - 1 ? R - 1 : rn);
-                const uint64_t ol = s_occ[rn];
-                const bool centre = n == kCenter<2>;
-                // outside the grid: never free
-                const uint64_t od = centre ? occC : (((ingm >> n) & 1) ? ol : ~0ull);
-                const uint64_t fr = ~od & free_sp;
-                if (!fr) {  // find_free_memory found nothing: dropped
-                    if (STATS) n_drop += own;
-                    continue;
-                }
-                const int f = __builtin_ctzll(fr);
-                const uint64_t fb = 1ull << f;
-                free_sp = full & (~0ull << f);  // starting_point = free_idx
-                if (STATS) n_moved += own;
-                const uint32_t dcn = S32 + (uint32_t)(dx + n0 * dy);
-                ms.org[org_at<2>(dcn, (uint32_t)f, C32, (uint32_t)K)] = origin;
-                if (centre) {
-                    occC |= fb;
-                    arrS |= fb;
-                    tchS |= fb;
-                    if (f > ip) pend |= fb;  // the slot loop reaches it again
-                } else {
-                    s_occ[rn] = od | fb;
-                    atomicOr(reinterpret_cast<unsigned long long*>(&s_arr[rn]),
+            load_codes(ms, S32, C32, nw, nxt);
+            mov = ms.mov[S32];
+            stm = ms.stm[S32];
+        }
+        return ok;
+    };
+    bool mine = fetch(0);
+    for (int p = 0; p < kNB<2>; ++p) {
+        const int px = x, py = y;
+        const bool live = mine;
+        const uint64_t mov_p = mov, stm_p = stm;
+        if (live) put_codes(row, nxt, nw);
+        if (p + 1 < kNB<2>) mine = fetch(p + 1);
+        const int r = (px - gx0) + RX * (py - gy0);
+        uint64_t gap = live ? s_gap[r] : 0ull;
+        if (live && (mov_p | gap)) {
+            const uint32_t S32 = (uint32_t)px + (uint32_t)n0 * (uint32_t)py;
+            const int col0 = p / 3, col1 = p % 3;
+            const uint64_t gap0 = gap;
+            NbEntry* const nb0 = s_nb + (r - 1 - RX);
+            auto at = [&](uint32_t cd) -> NbEntry& { return nb0[cd]; };
+            auto later = [&](uint32_t cd, NbEntry& to, uint64_t fb) {
+                const int n = neighbour_of<2>(cd), dx = n % 3 - 1, dy = n / 3 - 1;
+                if (((col0 + dx + 3) % 3) * 3 + (col1 + dy + 3) % 3 > p)
+                    atomicOr(reinterpret_cast<unsigned long long*>(&s_gap[&to - s_nb]),
                              (unsigned long long)fb);
-                    atomicOr(reinterpret_cast<unsigned long long*>(&s_tch[rn]),
-                             (unsigned long long)fb);
-                    // an arrival that fails the strict test of its new cell is
-                    // re-slotted there when that cell's phase comes later
-                    if ((cd & kGap) && ((col0 + dx + 3) % 3) * 3 + (col1 + dy + 3) % 3 > p)
-                        atomicOr(reinterpret_cast<unsigned long long*>(&s_mov[rn]),
-                                 (unsigned long long)fb);
-                }
+            };
+            int mv = 0, dl = 0, dr = 0;
+            run_cell<2, STATS>(mov_p, stm_p, gap, s_nb[r].free, row, at, later, ms.org, S32, C32,
+                               K, mv, dl, dr);
+            if (gap != gap0) s_gap[r] = gap;
+            if (STATS && tx0 <= px && px <= tx1 && ty0 <= py && py <= ty1) {
+                n_moved += mv;
+                n_del += dl;
+                n_drop += dr;
             }
-            s_occ[r] = occC;
-            s_arr[r] = arrS;
-            s_tch[r] = tchS;
-            s_mov[r] = 0;
         }
         __syncthreads();
     }
     const int ow = tx1 - tx0 + 1, oh = ty1 - ty0 + 1;
     for (int i = threadIdx.x; i < ow * oh; i += BS) {
-        const int x = i % ow, y = i / ow;
-        const uint32_t c = (uint32_t)(tx0 + x) + (uint32_t)n0 * (uint32_t)(ty0 + y);
-        const int r = (tx0 - gx0) + x + RX * ((ty0 - gy0) + y);
-        ms.occ[c] = s_occ[r];
-        ms.arr[c] = s_arr[r];
-        ms.tch[c] = s_tch[r];
+        const int cx = i % ow, cy = i / ow;
+        const uint32_t c = (uint32_t)(tx0 + cx) + (uint32_t)n0 * (uint32_t)(ty0 + cy);
+        const int r = (tx0 - gx0) + cx + RX * ((ty0 - gy0) + cy);
+        ms.occ[c] = ~s_nb[r].free & full;
+        if (s_gap[r]) ms.gap[c] = s_gap[r];
     }
     if (STATS) {
         stat_add(st, ST_MOVED, n_moved);
@@ -904,29 +895,38 @@ __global__ void __launch_bounds__(kBlock) k_mv_scatter(Grid<D> g, TPtr3<D, T> co
     // the first chunk's origins go out with the cell's words: unguarded loads
     // (slot clamped to K - 1, values used for arrivals only), one round trip
     // fewer than loading them after the arrival bits are known
-    uint32_t o0[8];
+    uint16_t o0[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         const int k = kb + j < g.K ? kb + j : g.K - 1;
         o0[j] = ms.org[org_at<D>((uint32_t)c, (uint32_t)k, (uint32_t)C, (uint32_t)g.K)];
     }
-    const uint64_t arr = ms.arr[c], occ = ms.occ[c], occ0 = ms.occ0[c], tch = ms.tch[c];
-    const uint64_t work = arr | (~arr & ~occ & (occ0 | tch));
+    const uint64_t occ = ms.occ[c], occ0 = ms.occ0[c], gap = ms.gap[c];
+    const uint64_t arr = arrivals(occ, occ0, ms.mov[c]);
+    const uint64_t work = arr | (~occ & (occ0 | gap));  // arrivals, emptied slots
     if (!(work >> kb)) return;
+    const int str1 = (int)g.ni[0], str2 = (int)(g.ni[0] * g.ni[1]);
     for (int k0 = kb; k0 < ke; k0 += 8) {
         const uint32_t wb = (uint32_t)(work >> k0) & 0xFFu;
         if (!wb) continue;
         const uint32_t ab = (uint32_t)(arr >> k0) & 0xFFu;
         uint32_t o[8];
-        if (k0 == kb) {
 #pragma unroll
-            for (int j = 0; j < 8; ++j) o[j] = o0[j];
-        } else {
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t at = org_at<D>((uint32_t)c, (uint32_t)(k0 + j), (uint32_t)C,
+                                          (uint32_t)g.K);
+            o[j] = k0 == kb ? (uint32_t)o0[j] : ((ab >> j) & 1) ? (uint32_t)ms.org[at] : 0u;
+        }
+        // the record numbers: of the source cell, its rank-th
 #pragma unroll
-            for (int j = 0; j < 8; ++j)
-                o[j] = ((ab >> j) & 1) ? ms.org[org_at<D>((uint32_t)c, (uint32_t)(k0 + j),
-                                                          (uint32_t)C, (uint32_t)g.K)]
-                                       : 0u;
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t src = (uint32_t)c - (uint32_t)move_offset<D>((o[j] >> 6) & 0x7Fu, str1,
+                                                                        str2);
+            if (((ab >> j) & 1) && o[j] == kOrgFar)
+                o[j] = ms.orgf[org_at<D>((uint32_t)c, (uint32_t)(k0 + j), (uint32_t)C,
+                                         (uint32_t)g.K)];
+            else
+                o[j] = src * (uint32_t)g.K + (o[j] & 63u);
         }
         if constexpr (REC16) {
             float u0[8], u1[8];
@@ -990,11 +990,187 @@ __global__ void __launch_bounds__(kBlock) k_mv_scatter(Grid<D> g, TPtr3<D, T> co
 // jump of the grid's size makes every level one cell (the serial order).
 constexpr int kFarBlock = 256;
 
+template <int D>
+__device__ inline void far_origin(const MoveScratch& ms, uint32_t c, uint32_t k, uint32_t C,
+                                  uint32_t K, uint32_t record) {
+    const uint32_t at = org_at<D>(c, k, C, K);
+    ms.orgf[at] = record;
+    ms.org[at] = (uint16_t)kOrgFar;
+}
+
+// The reference slot loop of cell I in phase `phase` on the far-jump path
+// (cells in an order that keeps apart any two that interact): kFar codes are
+// resolved here from the staged positions, and a destination beyond the 3^D
+// neighbourhood is updated in the global words directly.
+template <int D, int BS, typename T>
+__device__ inline void far_cell(const Grid<D>& g, const MoveScratch& ms, const int64_t* I,
+                                int phase, NbEntry (&s_nb)[kNB<D>][BS],
+                                uint32_t (&s_code)[BS * kRow / 4], int& n_moved, int& n_del,
+                                int& n_drop, int& n_far) {
+    const int64_t S = lin<D>(g.ni, I);
+    const int tid = threadIdx.x;
+    const int K = g.K;
+    const int64_t C = g.C;
+    const uint32_t S32 = (uint32_t)S, C32 = (uint32_t)C;
+    const uint64_t full = K == 64 ? ~0ull : ((1ull << K) - 1);
+    // everything this cell needs, in one round of independent loads: its
+    // words, its code words and the occupancy words of its 3^D neighbourhood
+    const uint64_t gapS = ms.gap[S];
+    uint64_t pend = ms.mov[S] | gapS;
+    const uint64_t pend0 = pend, occ0S = ms.occ0[S];
+    const uint64_t stmS = ms.stm[S];  // staged movers (their record index)
+    uint64_t cw[8];
+    load_codes(ms, S32, C32, (K + 7) >> 3, cw);
+    int64_t nbc[kNB<D>];
+    uint64_t was[kNB<D>];
+#pragma unroll
+    for (int n = 0; n < kNB<D>; ++n) {
+        bool v;
+        nbc[n] = nb_cell<D>(g, I, n, v);
+        was[n] = v ? ms.occ[nbc[n]] : ~0ull;  // outside the grid: never free
+    }
+    if (!pend) return;  // nothing leaves or re-slots here
+#pragma unroll
+    for (int n = 0; n < kNB<D>; ++n)
+        s_nb[n][tid] = NbEntry{~was[n] & full, nbc[n] < 0 ? 0xFFFFFFFFu : (uint32_t)nbc[n], 0u};
+    uint32_t* const row = s_code + tid * (kRow / 4);
+    put_codes(row, cw, (K + 7) >> 3);
+    uint64_t occC = was[kCenter<D>];  // this cell's occupancy
+    uint64_t arrS = occC & ~occ0S;  // slots holding an arrival
+    uint64_t selfm = 0;  // slots that received a re-slotted particle of this cell
+    uint64_t again = 0;  // those the loop reaches (pending from then on)
+    int sp = 0;
+    while (pend) {
+        const int ip = __builtin_ctzll(pend);
+        pend &= pend - 1;
+        const uint64_t bit = 1ull << ip;
+        // a mover of this cell: its staged record and code; an arrival: the
+        // record its origin staged, and (unless it was re-slotted here) the
+        // destination from its position
+        const bool arrival = (arrS & bit) != 0;
+        const int rank = __popcll(stmS & (bit - 1));
+        uint32_t origin = S32 * (uint32_t)K + (uint32_t)rank;
+        uint32_t cd = kFar;
+        if (arrival)
+            origin = ms.orgf[org_at<D>(S32, (uint32_t)ip, C32, (uint32_t)K)];
+        else if (stmS & bit)
+            cd = reinterpret_cast<const uint8_t*>(row)[rank];
+        if (selfm & bit) cd = kHere<D>;
+        occC &= ~bit;  // empty_particle! on the source slot
+        arrS &= ~bit;
+        selfm &= ~bit;
+        if (!arrival && !(stmS & bit)) {
+            ++n_del;
+            continue;
+        }
+        if (cd == kFar) {
+            // the destination from the staged position: bisection seeded
+            // at this cell (FP64), the cell + floor(u) (split, whose staged
+            // offset is renormalised to it here, for the scatter)
+            int64_t J[D];
+            bool near = true, inJ = true;
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                const T q = stg_coord<D, T>(ms, origin, d);
+                if constexpr (std::is_same<T, float>::value) {
+                    const int sd = (int)floorf(q);
+                    J[d] = I[d] + sd;
+                    stg_coord<D, T>(ms, origin, d) = (float)((double)q - (double)sd);
+                } else {
+                    J[d] = find_cell(q, g.xv[d], I[d]);
+                    const double xl = g.xv[d].x[J[d]];
+                    inJ = inJ && xl < q && q < xl + g.xv[d].dx[J[d]];
+                }
+                near = near && J[d] - I[d] <= 1 && I[d] - J[d] <= 1;
+            }
+            if (near) {  // inside the neighbourhood: the usual path
+                int nn = 0, mult = 1;
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    nn += (int)(J[d] - I[d] + 1) * mult;
+                    mult *= 3;
+                }
+                cd = code_of<D>(nn);
+                if (nn != kCenter<D> && !inJ) cd |= kRare;
+            } else {
+                ++n_far;
+                const int64_t dcn = lin<D>(g.ni, J);
+                const uint64_t od = ms.occ[dcn];
+                const uint64_t fr = ~od & full & (~0ull << sp);
+                if (!fr) {
+                    ++n_drop;
+                    continue;
+                }
+                const int f = __builtin_ctzll(fr);
+                sp = f;
+                const uint64_t fb = 1ull << f;
+                ++n_moved;
+                far_origin<D>(ms, (uint32_t)dcn, (uint32_t)f, C32, (uint32_t)K, origin);
+                ms.occ[dcn] = od | fb;
+                // an arrival that fails the strict test of its new cell is
+                // looked up again when that cell comes later: in a later
+                // phase, or later in this one (a jump by a multiple of 3
+                // cells keeps the colour; cells of a phase go in linear
+                // order)
+                const int pj = phase_of<D>(J);
+                if (!inJ && (pj > phase || (pj == phase && dcn > S)))
+                    atomicOr(reinterpret_cast<unsigned long long*>(ms.gap + dcn),
+                             (unsigned long long)fb);
+                continue;
+            }
+        }
+        const int n = neighbour_of<D>(cd & 0x7Fu);
+        const NbEntry nb = s_nb[n][tid];
+        const uint32_t dcn = nb.cell;
+        const uint64_t fr = (n == kCenter<D> ? ~occC & full : nb.free) & (~0ull << sp);
+        if (!fr) {  // find_free_memory found nothing: dropped
+            ++n_drop;
+            continue;
+        }
+        const int f = __builtin_ctzll(fr);
+        sp = f;  // starting_point = free_idx
+        const uint64_t fb = 1ull << f;
+        s_nb[n][tid].free = nb.free & ~fb;  // (the centre's LDS copy is not read)
+        ++n_moved;
+        far_origin<D>(ms, dcn, (uint32_t)f, C32, (uint32_t)K, origin);
+        if (n == kCenter<D>) {
+            occC |= fb;
+            arrS |= fb;
+            if (f > ip) {  // the slot loop will reach this particle again
+                pend |= fb;
+                selfm |= fb;
+                again |= fb;
+            }
+        } else if (cd & kRare) {
+            // the arrival fails the strict test of its new cell: when that cell's
+            // phase comes later, it is re-slotted there (bisection returns that cell)
+            const int64_t Dc = dcn;
+            int64_t J[D];
+            unlin<D>(g.ni, Dc, J);
+            if (phase_of<D>(J) > phase) {
+                // (its destination is looked up again, as the reference does)
+                ms.gap[Dc] |= fb;
+            }
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < kNB<D>; ++n) {
+        if (n == kCenter<D>) continue;
+        const NbEntry nb = s_nb[n][tid];
+        const uint32_t dn = nb.cell;
+        if (dn == 0xFFFFFFFFu) continue;
+        const uint64_t now = ~nb.free & full;
+        if (now != was[n]) ms.occ[dn] = now;
+    }
+    ms.occ[S] = occC;
+    if (again & ~pend0) ms.gap[S] = gapS | again;
+}
+
 template <int D, typename T>
 __global__ void __launch_bounds__(kFarBlock) k_mv_far(Grid<D> g, MoveScratch ms,
                                                       int* __restrict__ flag, jp_stats* st) {
     __shared__ NbEntry s_nb[kNB<D>][kFarBlock];
-    __shared__ uint64_t s_cw[8][kFarBlock];
+    __shared__ uint32_t s_code[kFarBlock * kRow / 4];
     const int fl = flag[0];
     if (!fl) return;
     const int R = flag[1];
@@ -1046,8 +1222,8 @@ __global__ void __launch_bounds__(kFarBlock) k_mv_far(Grid<D> g, MoveScratch ms,
                     ok = ok && I[d] < g.ni[d];
                 }
                 if (ok)
-                    phase_cell<D, kFarBlock, T, true>(g, ms, I, ph, false, s_nb, s_cw, n_moved,
-                                                      n_del, n_drop, n_far);
+                    far_cell<D, kFarBlock, T>(g, ms, I, ph, s_nb, s_code, n_moved, n_del,
+                                              n_drop, n_far);
             }
             __syncthreads();
         }
@@ -1069,7 +1245,8 @@ __global__ void __launch_bounds__(kClassifyMax)
     k_mv_classify_split(Grid<D> g, TPtr3<D, float> off, const uint8_t* __restrict__ index,
                         int nargs, ArgPtrs args, MoveScratch ms, int* flag,
                         const SplitGeom* __restrict__ geo) {
-    __shared__ int s_cnt[8][64];
+    __shared__ CellWords s_w;
+    __shared__ uint32_t s_code[64 * kRow / 4];
     const ClassifySlots<D> cs = classify_slots<D, true>(g);
     if (geo->bad) {  // grid rejected: the later kernels of this move return at once
         if (blockIdx.x == 0 && threadIdx.x == 0) atomicOr(flag, kFlagRejected);
@@ -1080,11 +1257,11 @@ __global__ void __launch_bounds__(kClassifyMax)
     const int64_t C = g.C;
     int64_t I[D];
     unlin<D>(g.ni, c, I);
-    const uint64_t occ = !cs.live ? 0ull
-                         : (kb == 0 && ke == g.K) ? active_slots(index, c, C, g.K)
-                                                  : active_slots_in(index, c, C, kb, ke);
-    uint64_t mov = 0, staged = 0;
+    const uint64_t occ = cs.live ? active_slots_in(index, c, C, kb, ke) : 0ull;
     uint64_t* __restrict__ cw = reinterpret_cast<uint64_t*>(ms.code) + c;
+    uint32_t* row = s_code + (threadIdx.x & 63) * (kRow / 4);
+    uint8_t* const crow = reinterpret_cast<uint8_t*>(row);
+    fill_codes<D>(row, kb, kb + 8);
     constexpr int B = 8;
     const double* __restrict__ f0 = nargs ? args.p[0] : nullptr;
     for (int k0 = kb; k0 < ke; k0 += B) {
@@ -1100,7 +1277,7 @@ __global__ void __launch_bounds__(kClassifyMax)
             for (int d = 0; d < D; ++d) ub[j][d] = on ? off.p[d][c + C * (k0 + j)] : 0.0f;
             fb[j] = (on && f0) ? f0[c + C * (k0 + j)] : 0.0;
         }
-        uint64_t word = 0;
+        uint32_t cd8[2] = {0, 0};  // the chunk's codes, by slot
         uint32_t mv8 = 0, stg = 0;
 #pragma unroll
         for (int j = 0; j < B; ++j) {
@@ -1124,28 +1301,40 @@ __global__ void __launch_bounds__(kClassifyMax)
             }
             if (stay && !out) continue;
             mv8 |= 1u << j;
-            uint8_t cd;
-            if (out) {
-                cd = kDel;
-            } else if (far) {  // staged as it is: the far-jump path renormalises it
+            if (out) continue;  // deleted
+            uint32_t cd;
+            if (far) {  // staged as it is: the far-jump path renormalises it
                 atomicOr(flag, kFlagFar);
                 atomicMax(flag + 1, jump);
                 cd = kFar;
-                stg |= 1u << j;
             } else {
-                cd = (uint8_t)n;
+                cd = code_of<D>(n);
 #pragma unroll
                 for (int d = 0; d < D; ++d)  // the staged value: the offset in the new cell
                     ub[j][d] = (float)((double)ub[j][d] - (double)s[d]);
-                stg |= 1u << j;
             }
-            word |= (uint64_t)cd << (8 * j);
+            stg |= 1u << j;
+            cd8[j >> 2] |= cd << (8 * (j & 3));
         }
-        if (mv8) cw[(k0 >> 3) * C] = word;
-        mov |= (uint64_t)mv8 << k0;
         // the chunk's staged movers, packed after the cell's earlier ones
-        const int64_t o0 = chunk_record<true>(c, g.K, k0, stg, staged, s_cnt);
+        // (one chunk per thread)
+        s_w.put(W_OCC, (uint32_t)(occ >> k0));
+        s_w.put(W_MOV, mv8);
+        s_w.put(W_STG, stg);
+        __syncthreads();
+        const int r0 = __popcll(s_w.get(W_STG) & ((1ull << k0) - 1));
+#pragma unroll
+        for (int j = 0; j < B; ++j)
+            if ((stg >> j) & 1)
+                crow[r0 + __popc(stg & ((1u << j) - 1))] = (uint8_t)(cd8[j >> 2] >> (8 * (j & 3)));
+        const int64_t o0 = c * g.K + r0;
+        __syncthreads();
         if (cs.live) {
+            // (one code word per chunk-thread)
+            if (__popcll(s_w.get(W_STG)) > kb) cw[(kb >> 3) * C] = code_word(row, kb >> 3);
+            for (int w = (int)(threadIdx.x >> 6); w < W_COUNT; w += (int)(blockDim.x >> 6))
+                store_word<D>(ms, c, w, w == W_GAP ? 0ull  // no ties: floor(u) is never the cell
+                                                   : s_w.get(w));
             if (D == 2 && nargs == 1) {  // 16-byte records (the scatter reads them whole)
 #pragma unroll
                 for (int j = 0; j < B; ++j)
@@ -1164,11 +1353,7 @@ __global__ void __launch_bounds__(kClassifyMax)
                 stage_args<D>(c, C, k0, stg, o0, nargs, args, ms, 1);
             }
         }
-        staged |= (uint64_t)stg << k0;
     }
-    if (!cs.live) return;
-    store_cell_words(ms, c, kb, ke, g.K, occ, mov);
-    reinterpret_cast<uint8_t*>(ms.stm + c)[kb >> 3] = (uint8_t)(staged >> kb);
 }
 
 ArgPtrs argptrs(double* const* a, int n) {
@@ -1202,10 +1387,11 @@ int run_move(jp_ctx* ctx, const jp_cellgrid* gc, T* const* coords, uint8_t* inde
     const size_t o_occ0 = off; off = align_up(off + C * 8, 256);
     const size_t o_occ = off;  off = align_up(off + C * 8, 256);
     const size_t o_mov = off;  off = align_up(off + C * 8, 256);
-    const size_t o_arr = off;  off = align_up(off + C * 8, 256);
-    const size_t o_tch = off;  off = align_up(off + C * 8, 256);
+    const size_t o_gap = off;  off = align_up(off + C * 8, 256);
+    const size_t o_rar = off;  off = align_up(off + (D == 2 ? C * 8 : 0), 256);
     const size_t o_code = off; off = align_up(off + (size_t)C * 64, 256);
-    const size_t o_org = off;  off = align_up(off + (size_t)S * 4, 256);
+    const size_t o_org = off;  off = align_up(off + (size_t)S * 2, 256);
+    const size_t o_orgf = off; off = align_up(off + (size_t)S * 4, 256);
     const size_t o_stm = off;  off = align_up(off + C * 8, 256);
     ms.S = S;
     ms.foff = (int64_t)align_up(sizeof(T) * D, 8);
@@ -1218,10 +1404,11 @@ int run_move(jp_ctx* ctx, const jp_cellgrid* gc, T* const* coords, uint8_t* inde
     ms.occ0 = (uint64_t*)(base + o_occ0);
     ms.occ = (uint64_t*)(base + o_occ);
     ms.mov = (uint64_t*)(base + o_mov);
-    ms.arr = (uint64_t*)(base + o_arr);
-    ms.tch = (uint64_t*)(base + o_tch);
+    ms.gap = (uint64_t*)(base + o_gap);
+    ms.rar = (uint64_t*)(base + o_rar);
     ms.code = (uint8_t*)(base + o_code);
-    ms.org = (uint32_t*)(base + o_org);
+    ms.org = (uint16_t*)(base + o_org);
+    ms.orgf = (uint32_t*)(base + o_orgf);
     ms.stm = (uint64_t*)(base + o_stm);
     ms.stg = base + o_stg;
 
@@ -1290,8 +1477,11 @@ int run_move(jp_ctx* ctx, const jp_cellgrid* gc, T* const* coords, uint8_t* inde
             o.o[d] = r % 3;
             r /= 3;
         }
-        k_mv_phase<D, BS><<<(unsigned)((total + BS - 1) / BS), BS, 0, ctx->stream>>>(g, ms, o, ph,
-                                                                                    flag, st);
+        const unsigned nb = (unsigned)((total + BS - 1) / BS);
+        if (st)
+            k_mv_phase<D, BS, true><<<nb, BS, 0, ctx->stream>>>(g, ms, o, ph, flag, st);
+        else
+            k_mv_phase<D, BS, false><<<nb, BS, 0, ctx->stream>>>(g, ms, o, ph, flag, st);
         if ((rc = launched())) return rc;
     }
     k_mv_far<D, T><<<1, kFarBlock, 0, ctx->stream>>>(g, ms, flag, st);
