@@ -6,6 +6,7 @@
 #include "jp_inject2.hpp"
 
 #include <cmath>
+#include <type_traits>
 
 using namespace jp;
 
@@ -52,127 +53,277 @@ __global__ void __launch_bounds__(kBlock) k_init(Grid<D> g, Ptr3 coords, uint8_t
 }
 
 // ============================================================ particle2grid
-// _particle2grid! (src/Interpolations/particle_to_grid.jl:37-199): one thread
-// per node, exact reference accumulation order (cells with the last dim
-// outermost, slots ascending).  mode 0: wF/w (2D scalar), 1: wF*inv(w).
-template <int D, int NF>
-__global__ void __launch_bounds__(kBlock) k_p2g(Grid<D> g, int nf_rt, ArgPtrs F, ArgPtrs Fp,
-                                                CPtr3 coords, const uint64_t* __restrict__ occw,
-                                                int mode) {
-    // NF == 1: one field, accumulator kept in a register; NF == 0: nf_rt fields
-    const int nf = NF == 1 ? 1 : nf_rt;
-    int64_t nn[D];
-    int64_t NN = 1;
+// The reference's weight of a particle at distance d = sqrt(s) from a node is
+// 1 / (d d), with the square root, the product and the quotient each correctly
+// rounded.  weights() gives the same bits as sqrt(s), d * d and
+// 1.0 / (d d) for kSafeLo <= s < kSafeHi, where nothing overflows, underflows
+// or is denormal, without the scaling and special-case selects of the general
+// operations: the square root by Goldschmidt's iteration from the hardware
+// estimate and two residual corrections, the quotient from the square of the
+// refined reciprocal root by one Newton step and a residual correction (each
+// last step rounds a result already within an ulp: P. Markstein, IBM J. Res.
+// Dev. 34, 1990).  23 instructions, one of them a slow one, instead of 36 with
+// two.
+constexpr uint32_t kSafeLo = (1023u - 480u) << 20;  // high words of 2^-480, 2^480
+constexpr uint32_t kSafeHi = (1023u + 480u) << 20;
+// B of them side by side, step by step: each is one chain of dependent
+// operations.
+template <int B>
+__device__ inline void weights(const double (&s)[B], double (&wi)[B]) {
+    double g[B], h[B], e[B];
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-        nn[d] = g.ni[d] + 1;
-        NN *= nn[d];
+    for (int j = 0; j < B; ++j) h[j] = __builtin_amdgcn_rsq(s[j]);
+#pragma unroll
+    for (int j = 0; j < B; ++j) g[j] = s[j] * h[j];
+#pragma unroll
+    for (int j = 0; j < B; ++j) h[j] = 0.5 * h[j];
+#pragma unroll
+    for (int j = 0; j < B; ++j) e[j] = fma(-h[j], g[j], 0.5);
+#pragma unroll
+    for (int j = 0; j < B; ++j) g[j] = fma(g[j], e[j], g[j]);
+#pragma unroll
+    for (int j = 0; j < B; ++j) h[j] = fma(h[j], e[j], h[j]);
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+        for (int j = 0; j < B; ++j) e[j] = fma(-g[j], g[j], s[j]);
+#pragma unroll
+        for (int j = 0; j < B; ++j) g[j] = fma(e[j], h[j], g[j]);  // the second: sqrt(s)
     }
-    int64_t node = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    if (node >= NN) return;
-    int64_t N[D];
-    {
-        int64_t r = node;
 #pragma unroll
-        for (int d = 0; d < D; ++d) {
-            N[d] = r % nn[d];
-            r /= nn[d];
-        }
+    for (int j = 0; j < B; ++j) {
+        g[j] = g[j] * g[j];
+        h[j] = (4.0 * h[j]) * h[j];
     }
-    double xn[D];
 #pragma unroll
-    for (int d = 0; d < D; ++d) xn[d] = g.xv[d].x[N[d]];
-    double w = 0.0;
-    double wF[JP_MAX_ARGS];
-    for (int f = 0; f < nf; ++f) wF[f] = 0.0;
+    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+        for (int j = 0; j < B; ++j) e[j] = fma(-g[j], h[j], 1.0);
+#pragma unroll
+        for (int j = 0; j < B; ++j) h[j] = fma(e[j], h[j], h[j]);
+    }
+#pragma unroll
+    for (int j = 0; j < B; ++j) wi[j] = h[j];
+}
+__device__ inline double weight_any(double s) {
+    const double dist = sqrt(s);
+    return 1.0 / (dist * dist);
+}
+
+// _particle2grid! (src/Interpolations/particle_to_grid.jl:37-199), exact
+// reference accumulation order (cells with the last dim outermost, slots
+// ascending).  mode 0: wF/w (2D scalar), 1: wF*inv(w).
+//
+// A thread walks R + 1 layers of cells along the last dimension for a column
+// of R nodes (3D: for PY = 2 columns next to each other in y), two nodes of a
+// column at a time: a layer adds to the node below it, which is then done, and
+// to the node above it.  A particle is loaded once for all of the column's
+// nodes that it touches.  A thread per node reads every particle 2^D times, all
+// of it past the L2 (a plane sweep of the resident wavefronts is far larger),
+// which bounds it at 5 TB/s; columns read it 2 (R + 1) / R times in 2D and
+// 3 (R + 1) / R in 3D.
+//
+// A chunk of B slot planes is straight-line code: every lane computes the
+// weights of B slots side by side (garbage for empty slots), then adds those
+// of its active slots in order; a chunk that no lane of the wavefront needs
+// is skipped.  One range check for the chunk: if any active slot's s lies
+// outside weights()'s range, the chunk's weights come from the general
+// operations.  The next chunk's loads are in flight meanwhile, unguarded (all
+// lanes are on the same slot plane: coalesced across neighbouring cells).
+// NF fields per launch, accumulators in registers.  A thread per node with a
+// branch per slot and the general operations took 190 us at 512^2 (now 157),
+// 49 at 32^2 (31), 192 at 389 x 211 with three fields (77) and 1470 at 61 x 47
+// x 74 with two (383).
+template <int NF>
+struct P2gFields {
+    double* F[NF];
+    const double* Fp[NF];
+};
+template <int D, int NF, int PY>
+__global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 2))) k_p2g(Grid<D> g, P2gFields<NF> fields, CPtr3 coords,
+                                                const uint64_t* __restrict__ occw, int mode,
+                                                int R, int64_t threads) {
+    static_assert(D == 3 || PY == 1, "patches along y in 3D only");
+    int64_t t = blockIdx.x * (int64_t)kBlock + threadIdx.x;
+    if (t >= threads) return;
+    constexpr int L = D - 1;  // the dimension walked along
+    constexpr int NY = D == 3 ? PY : 1;
+    const int64_t n0 = g.ni[0] + 1, n1 = g.ni[1] + 1;
+    // node column: x index i, first y index (3D), first index z along L
+    const int64_t i = t % n0;
+    t /= n0;
+    const int64_t ny = (n1 + PY - 1) / PY;
+    const int64_t y0 = D == 3 ? (t % ny) * PY : 0;
+    const int64_t z0 = (D == 3 ? t / ny : t) * R;
+    const double xn = g.xv[0].x[i];
+    double yn[NY];
+#pragma unroll
+    for (int m = 0; m < NY; ++m)
+        yn[m] = D == 3 ? g.xv[1].x[y0 + m < n1 ? y0 + m : n1 - 1] : 0.0;
     const int64_t C = g.C;
-    constexpr int NC = 1 << D;
-    // the (up to) 2^D cells around the node, last dim outermost, and their
-    // occupancy words (one round of loads)
-    int64_t cell[NC];
-    uint64_t bits[NC];
-#pragma unroll
-    for (int q = 0; q < NC; ++q) {
-        int64_t I[D];
-        bool ok = true;
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            I[d] = N[d] + (((q >> d) & 1) ? 0 : -1);
-            ok = ok && (I[d] >= 0 && I[d] < g.ni[d]);
-        }
-        cell[q] = ok ? lin<D>(g.ni, I) : 0;
-        bits[q] = ok ? occw[cell[q]] : 0ull;
-    }
-    // Reference order: cells, then slots ascending.  The (cell, chunk of B
-    // slots) sequence is walked with the next chunk's loads in flight while
-    // the current one is accumulated; all lanes of a wavefront are on the same
-    // slot plane, so every load is coalesced across neighbouring cells.
-    constexpr int B = D == 2 ? 8 : 4;  // two chunk buffers stay in registers
-    const int nk = (g.K + B - 1) / B;
-    const int total = NC * nk;
-    auto chunk = [&](int t, int64_t& c, uint32_t& bq, int& k0) __attribute__((always_inline)) {
-        const int q = t / nk;
-        k0 = (t - q * nk) * B;
-        c = cell[0];
-        uint64_t bw = bits[0];
-#pragma unroll
-        for (int u = 1; u < NC; ++u) {
-            c = q == u ? cell[u] : c;
-            bw = q == u ? bits[u] : bw;
-        }
-        bq = (uint32_t)(bw >> k0) & ((1u << B) - 1);
+    constexpr int NU = 2 * (D == 3 ? PY + 1 : 1);  // cells of a layer, in order
+    constexpr int B = 4, V = D + NF;
+    struct Chunk {
+        double v[B][V];
+        uint32_t on;  // active slots of the chunk
+        int u;        // cell of the layer
     };
-    auto load = [&](int t, double (&pv)[B][D + 1]) __attribute__((always_inline)) {
-        int64_t c;
-        uint32_t bq;
-        int k0;
-        chunk(t, c, bq, k0);
+    // accumulators of the nodes below ([m][0]) and above ([m][1]) the layer
+    double w[NY][2], wF[NY][2][NF];
 #pragma unroll
-        for (int j = 0; j < B; ++j) {
-            const bool on = (bq >> j) & 1;
-            const int64_t e = c + C * (k0 + j);
+    for (int m = 0; m < NY; ++m)
 #pragma unroll
-            for (int d = 0; d < D; ++d) pv[j][d] = on ? coords.p[d][e] : 0.0;
-            pv[j][D] = on ? Fp.p[0][e] : 0.0;
+        for (int h = 0; h < 2; ++h) {
+            w[m][h] = 0.0;
+#pragma unroll
+            for (int f = 0; f < NF; ++f) wF[m][h][f] = 0.0;
+        }
+    int64_t cell[NU];
+    uint64_t bits[NU];
+    auto layer = [&](int64_t z, int64_t (&c)[NU], uint64_t (&b)[NU]) __attribute__((always_inline)) {
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            const int64_t x = i - 1 + (u & 1), y = y0 - 1 + (u >> 1);
+            bool ok = x >= 0 && x < g.ni[0] && z >= 0 && z < g.ni[L];
+            if (D == 3) ok = ok && y >= 0 && y < g.ni[1];
+            c[u] = !ok ? 0 : x + g.ni[0] * (D == 3 ? y + g.ni[1] * z : z);
+            b[u] = ok ? occw[c[u]] : 0ull;
         }
     };
-    auto accumulate = [&](int t, const double (&pv)[B][D + 1]) __attribute__((always_inline)) {
-        int64_t c;
-        uint32_t bq;
-        int k0;
-        chunk(t, c, bq, k0);
-#pragma unroll
-        for (int j = 0; j < B; ++j) {
-            if (!((bq >> j) & 1)) continue;
-            double a = xn[0] - pv[j][0];
-            double s = a * a;
-#pragma unroll
-            for (int d = 1; d < D; ++d) {
-                double b = xn[d] - pv[j][d];
-                s = s + b * b;
-            }
-            const double dist = sqrt(s);
-            const double wi = 1.0 / (dist * dist);
-            w += wi;
-            wF[0] = fma(wi, pv[j][D], wF[0]);
-            for (int f = 1; f < nf; ++f) wF[f] = fma(wi, Fp.p[f][c + C * (k0 + j)], wF[f]);
-        }
-    };
-    double b0[B][D + 1], b1[B][D + 1];
-    load(0, b0);
+    int64_t cell1[NU];
+    uint64_t bits1[NU];
+    layer(z0 - 1, cell1, bits1);
 #pragma unroll 1
-    for (int t = 0; t < total; t += 2) {
-        if (t + 1 < total) load(t + 1, b1);
-        accumulate(t, b0);
-        if (t + 1 >= total) break;
-        if (t + 2 < total) load(t + 2, b0);
-        accumulate(t + 1, b1);
-    }
-    if (mode == 0) {
-        F.p[0][node] = wF[0] / w;
-    } else {
-        double iw = 1.0 / w;
-        for (int f = 0; f < nf; ++f) F.p[f][node] = wF[f] * iw;
+    for (int r = 0; r <= R; ++r) {
+        const int64_t z = z0 - 1 + r;  // the layer's cells; nodes z (below) and z + 1 (above)
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            cell[u] = cell1[u];
+            bits[u] = bits1[u];
+        }
+        double zn[2];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const int64_t zi = z + h;
+            zn[h] = g.xv[L].x[zi < 0 ? 0 : (zi > g.ni[L] ? g.ni[L] : zi)];
+        }
+        // wait for the layer's words and nodes here: a wait inside the chunk
+        // loop would be one for all loads in flight
+#pragma unroll
+        for (int u = 0; u < NU; ++u) asm volatile("" : "+v"(bits[u]));
+        asm volatile("" : "+v"(zn[0]), "+v"(zn[1]));
+        if (r < R) layer(z + 1, cell1, bits1);
+        // chunk by chunk through the layer's cells: cell u, slot plane k up to
+        // the wavefront's last occupied one (all uniform over the wavefront),
+        // the lane's cell and remaining occupancy bits
+        int last[NU], chunks = 0;
+#pragma unroll
+        for (int v = 0; v < NU; ++v) {
+            int top = 0;
+            for (uint64_t any = bits[v]; __any(any != 0); any >>= B) top += B;
+            last[v] = top > 0 ? top : B;
+            chunks += last[v] / B;
+        }
+        int u = 0, k = 0, end = last[0];
+        int64_t c = cell[0];
+        uint64_t left = bits[0];
+        auto advance = [&]() __attribute__((always_inline)) {
+            k += B;
+            left >>= B;
+            if (k < end || u == NU - 1) return;
+            ++u;
+            k = 0;
+#pragma unroll
+            for (int v = 1; v < NU; ++v) {
+                c = u == v ? cell[v] : c;
+                left = u == v ? bits[v] : left;
+                end = u == v ? last[v] : end;
+            }
+        };
+        // (always the same number of loads, also past the last chunk, so that
+        // the wait for one buffer leaves the other's loads in flight)
+        auto read = [&](Chunk& ch) __attribute__((always_inline)) {
+            ch.on = (uint32_t)left & ((1u << B) - 1);
+            ch.u = u;
+#pragma unroll
+            for (int j = 0; j < B; ++j) {
+                const int64_t plane = C * (k + j < g.K ? k + j : g.K - 1);
+#pragma unroll
+                for (int d = 0; d < D; ++d) ch.v[j][d] = coords.p[d][plane + c];
+#pragma unroll
+                for (int f = 0; f < NF; ++f) ch.v[j][D + f] = fields.Fp[f][plane + c];
+            }
+        };
+        auto add = [&](const Chunk& ch) __attribute__((always_inline)) {
+#pragma unroll
+            for (int m = 0; m < NY; ++m) {
+                if (D == 3 && (ch.u >> 1) != m && (ch.u >> 1) != m + 1) continue;
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    if (h == 0 ? r == 0 : r == R) continue;  // another thread's node
+                    double s[B], wi[B];
+                    uint32_t far = 0;
+#pragma unroll
+                    for (int j = 0; j < B; ++j) {
+                        const double a = xn - ch.v[j][0];
+                        s[j] = a * a;
+                        if (D == 3) {
+                            const double b = yn[m] - ch.v[j][1];
+                            s[j] = s[j] + b * b;
+                        }
+                        const double e = zn[h] - ch.v[j][L];
+                        s[j] = s[j] + e * e;
+                        const uint32_t off = (uint32_t)__double2hiint(s[j]) - kSafeLo;
+                        far = ((ch.on >> j) & 1) && off > far ? off : far;
+                    }
+                    weights<B>(s, wi);
+                    if (__any(far >= kSafeHi - kSafeLo)) {
+#pragma unroll
+                        for (int j = 0; j < B; ++j) wi[j] = weight_any(s[j]);
+                    }
+#pragma unroll
+                    for (int j = 0; j < B; ++j) {
+                        if (!((ch.on >> j) & 1)) continue;
+                        w[m][h] += wi[j];
+#pragma unroll
+                        for (int f = 0; f < NF; ++f)
+                            wF[m][h][f] = fma(wi[j], ch.v[j][D + f], wF[m][h][f]);
+                    }
+                }
+            }
+        };
+        Chunk a, b;
+        read(a);
+#pragma unroll 1
+        for (int n = 0; n < chunks; n += 2) {
+            advance();
+            read(b);
+            add(a);
+            advance();
+            read(a);
+            add(b);
+        }
+        // the nodes below are done; those above are below the next layer
+#pragma unroll
+        for (int m = 0; m < NY; ++m) {
+            if (r > 0 && z <= g.ni[L] && (D == 2 || y0 + m < n1)) {
+                const int64_t node = i + n0 * (D == 3 ? y0 + m + n1 * z : z);
+                if (mode == 0) {
+                    fields.F[0][node] = wF[m][0][0] / w[m][0];
+                } else {
+                    const double iw = 1.0 / w[m][0];
+#pragma unroll
+                    for (int f = 0; f < NF; ++f) fields.F[f][node] = wF[m][0][f] * iw;
+                }
+            }
+            w[m][0] = w[m][1];
+            w[m][1] = 0.0;
+#pragma unroll
+            for (int f = 0; f < NF; ++f) {
+                wF[m][0][f] = wF[m][1][f];
+                wF[m][1][f] = 0.0;
+            }
+        }
     }
 }
 
@@ -644,10 +795,6 @@ int run_p2g(jp_ctx* ctx, const jp_cellgrid* g, int nf, double* const* F, const d
             const double* const* coords, const uint8_t* index, int mode,
             uint64_t* occ_fixed = nullptr) {
     Grid<D> G = to_grid<D>(g);
-    int64_t NN = 1;
-    for (int d = 0; d < D; ++d) NN *= G.ni[d] + 1;
-    ArgPtrs Fa = argptrs(F, nf);
-    ArgPtrs Fpa = argptrs(const_cast<double* const*>(Fp), nf);
     int rc;
     uint64_t* occ = occ_fixed;
     if (!occ) {
@@ -655,13 +802,38 @@ int run_p2g(jp_ctx* ctx, const jp_cellgrid* g, int nf, double* const* F, const d
         occ = static_cast<uint64_t*>(ctx->scratch);
     }
     if ((rc = occ_words(ctx, index, G.C, G.K, occ))) return rc;
-    if (nf == 1)
-        k_p2g<D, 1><<<blocks_for(NN), kBlock, 0, ctx->stream>>>(G, nf, Fa, Fpa, cptr3(coords, D),
-                                                                occ, mode);
-    else
-        k_p2g<D, 0><<<blocks_for(NN), kBlock, 0, ctx->stream>>>(G, nf, Fa, Fpa, cptr3(coords, D),
-                                                                occ, mode);
-    JP_LAUNCHED(ctx);
+    constexpr int PY = D == 3 ? 2 : 1;
+    int64_t cols = G.ni[0] + 1;  // node columns
+    if (D == 3) cols *= (G.ni[1] + 1 + PY - 1) / PY;
+    // nodes per thread: as many (a power of two, up to 16) as leave about 9
+    // wavefronts for every 16 SIMDs.  Longer columns read less, fewer
+    // wavefronts leave SIMDs idle; R = 1, 2, 4, 8 at 512^2 (4116 wavefronts
+    // with R = 1): 187, 180, 157, 190 us; 389 x 211, three fields (1292): 104,
+    // 77, 118, 216; 61 x 47 x 74, two fields (1744): 509, 383, 542, 965; 32^2
+    // (18): 31, 51, 91, 172.
+    int R = 1;
+    while (R < 16 && cols * ((G.ni[D - 1] + 2 * R) / (2 * R)) >= (int64_t)576 * 64) R *= 2;
+    const int64_t threads = cols * ((G.ni[D - 1] + R) / R);
+    // up to three fields per launch (their sums are independent: every launch
+    // computes the same weights); four would spill
+    for (int f = 0; f < nf;) {
+        const int m = nf - f < 3 ? nf - f : 3;
+        auto launch = [&](auto n) {
+            constexpr int NF = decltype(n)::value;
+            P2gFields<NF> a;
+            for (int i = 0; i < NF; ++i) {
+                a.F[i] = F[f + i];
+                a.Fp[i] = Fp[f + i];
+            }
+            k_p2g<D, NF, PY><<<blocks_for(threads), kBlock, 0, ctx->stream>>>(
+                G, a, cptr3(coords, D), occ, mode, R, threads);
+        };
+        if (m == 1) launch(std::integral_constant<int, 1>{});
+        else if (m == 2) launch(std::integral_constant<int, 2>{});
+        else launch(std::integral_constant<int, 3>{});
+        JP_LAUNCHED(ctx);
+        f += m;
+    }
     return finish(ctx);
 }
 
