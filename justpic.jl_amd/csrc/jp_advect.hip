@@ -4,16 +4,18 @@
 // (backtracking.jl, backtracking_MQS.jl, backtracking_LinP.jl) on gfx950, FP64
 // drop-in, 2D and 3D, Euler / RK2 / RK4.
 //
-// The linear scheme (advection!): one workgroup per tile of cells with each
-// velocity component's window of nodes, and its axis windows, staged in LDS;
-// one thread per cell walks the cell's slots in lockstep chunks of planes
-// (k_advect_tile).  A stage point outside a window sends the particle's whole
-// step to the slot path (inline in 2D, a flagged pass in 3D).  The
-// slot path (k_advect_slot, and the MQS / LinP schemes): one thread per
-// slot, the velocity gathered from global memory.  A bracket lookup costs one
-// guess (uniform spacing estimate) and one strict test against the stored
-// axis, with the reference search for everything else (ties, refined axes).
+// One workgroup per tile of cells with each velocity component's window of
+// nodes, and its axis windows, staged in LDS; the wavefronts walk the cells'
+// slots in lockstep chunks of planes (k_advect_tile, all three schemes).  A
+// particle with a stage point outside a window is advected on the slot path
+// after the tile's others.  The slot path (also k_advect_slot): the velocity
+// gathered from global memory.  A bracket lookup costs one guess (uniform
+// spacing estimate; in the windows of refined axes a short search from the
+// particle's cell) and one strict test against the stored axis, with the
+// reference search for everything else (ties).
 #include "jp_ctx.hpp"
+
+#include <type_traits>
 
 using namespace jp;
 
@@ -64,10 +66,12 @@ constexpr int kMQS = 1;     // interp_velocity2particle_MQS (advection_MQS.jl:10
 constexpr int kLinP = 2;    // interp_velocity2particle_LinP (advection_LinP.jl:104-131)
 
 // column-major view of one velocity component (k = 0 in 2D)
+template <typename Int>
 struct FView {
+    using I = Int;
     const double* __restrict__ F;
-    int64_t n0, n1;
-    __device__ double at(int64_t i, int64_t j, int64_t k) const { return F[i + n0 * (j + n1 * k)]; }
+    Int n0, n1;
+    __device__ double at(Int i, Int j, Int k) const { return F[i + n0 * (j + n1 * k)]; }
 };
 
 // half * (t - half)^2 * (muladd(-2, v1, v0) + v2) (src/Interpolations/MQS.jl:13)
@@ -81,9 +85,9 @@ __device__ inline double mqs_corr(double t, double v0, double v1, double v2) {
 // the cell (ta < 1/2) or right of it, then the lerp along the plane's second
 // axis (MQS.jl:2-27, 73-98, 126-152).  Rows 0 and 1 take their extra node
 // from (i-1 | i+2, jb0, kb0) and (i-1 | i+2, jb1, kb1).
-__device__ inline double mqs_x4(const FView& F, double v0, double v1, double v2, double v3,
-                                double ta, double tb, int64_t i, int64_t jb0, int64_t kb0,
-                                int64_t jb1, int64_t kb1) {
+template <class FV, class I = typename FV::I>
+__device__ inline double mqs_x4(const FV& F, double v0, double v1, double v2, double v3,
+                                double ta, double tb, I i, I jb0, I kb0, I jb1, I kb1) {
     const double lb = lerp1(ta, v0, v1), lt = lerp1(ta, v2, v3);
     const bool left = ta < 0.5;
     const double cb = left ? mqs_corr(ta, F.at(i - 1, jb0, kb0), v0, v1)
@@ -95,8 +99,9 @@ __device__ inline double mqs_x4(const FView& F, double v0, double v1, double v2,
 
 // MQS along y (MQS.jl:29-55, 100-124): columns (v00, v01), (v10, v11) lerped
 // along y with the correction through the node below or above, then along x.
-__device__ inline double mqs_y4(const FView& F, double v0, double v1, double v2, double v3,
-                                double t1, double t2, int64_t i, int64_t j, int64_t k) {
+template <class FV, class I = typename FV::I>
+__device__ inline double mqs_y4(const FV& F, double v0, double v1, double v2, double v3,
+                                double t1, double t2, I i, I j, I k) {
     const double ll = lerp1(t2, v0, v2), lr = lerp1(t2, v1, v3);
     const bool below = t2 < 0.5;
     const double cl = below ? mqs_corr(t2, F.at(i, j - 1, k), v0, v2)
@@ -111,15 +116,15 @@ __device__ inline double mqs_y4(const FView& F, double v0, double v1, double v2,
 // plane k (MQS.jl:58-64 pass the same i, j, k); z combines two MQS-x
 // evaluations of the (x, z) planes of rows j and j+1 along y, both with extra
 // nodes of row j (MQS.jl:67-71, 126-152).
-template <int D>
-__device__ inline double mqs(const FView& F, int c, const int64_t (&k0)[D], const double* q,
+template <int D, class FV, class I = typename FV::I>
+__device__ inline double mqs(const FV& F, int c, const I (&k0)[D], const double* q,
                              const double (&t)[D]) {
-    const int64_t i = k0[0], j = k0[1];
+    const I i = k0[0], j = k0[1], o = 0;
     if constexpr (D == 2) {
-        return c == 0 ? mqs_x4(F, q[0], q[1], q[2], q[3], t[0], t[1], i, j, 0, j + 1, 0)
-                      : mqs_y4(F, q[0], q[1], q[2], q[3], t[0], t[1], i, j, 0);
+        return c == 0 ? mqs_x4(F, q[0], q[1], q[2], q[3], t[0], t[1], i, j, o, j + 1, o)
+                      : mqs_y4(F, q[0], q[1], q[2], q[3], t[0], t[1], i, j, o);
     } else {
-        const int64_t k = k0[2];
+        const I k = k0[2];
         if (c == 0) {
             const double bot = mqs_x4(F, q[0], q[1], q[2], q[3], t[0], t[1], i, j, k, j + 1, k);
             const double top = mqs_x4(F, q[4], q[5], q[6], q[7], t[0], t[1], i, j, k, j + 1, k);
@@ -138,18 +143,18 @@ __device__ inline double mqs(const FView& F, int c, const int64_t (&k0)[D], cons
 
 // LinP's pressure-point value of component c (advection_LinP.jl:208-391):
 // the corner index moves by one along c when p is past the cell's middle
-// (offset_LinP); each row of three nodes along c around it (index clamped to
-// the array) is averaged pairwise as (a + b)/2 onto the two pressure points;
+// (offset_LinP); each row of three nodes along c around it (the reference
+// clamps their indices to the array: no effect for the interior corners this
+// is called for) is averaged pairwise as (a + b)/2 onto the two pressure points;
 // the rows run over the other axes (augment_offset: x and y components in
 // axis order, the z component with y before x); y and z components swap the
 // middle pairs (swap_F); t is measured from the corner moved by +-dx_c/2
 // (correct_xci_to_pressure_point).
-template <int D>
-__device__ inline double linp(const FView& F, const int64_t (&nn)[D], int c,
-                              const int64_t (&k0)[D], const double (&xc)[D],
+template <int D, class FV, class I = typename FV::I>
+__device__ inline double linp(const FV& F, int c, const I (&k0)[D], const double (&xc)[D],
                               const double (&dxi)[D], const double (&idx)[D],
                               const double (&p)[D]) {
-    int64_t b[D];
+    I b[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) b[d] = k0[d] + ((d == c && p[d] > xc[d] + dxi[d] / 2.0) ? 1 : 0);
     constexpr int nrow = D == 2 ? 2 : 4;
@@ -159,11 +164,11 @@ __device__ inline double linp(const FView& F, const int64_t (&nn)[D], int c,
         double val[3];
 #pragma unroll
         for (int e = 0; e < 3; ++e) {
-            int64_t id[3] = {0, 0, 0};
+            I id[3] = {0, 0, 0};
             int other = 0;
 #pragma unroll
             for (int d = 0; d < D; ++d) {
-                int64_t o;
+                int o;
                 if (d == c) {
                     o = e - 1;
                 } else {
@@ -171,8 +176,7 @@ __device__ inline double linp(const FView& F, const int64_t (&nn)[D], int c,
                     o = (r >> bit) & 1;
                     ++other;
                 }
-                const int64_t v = b[d] + o;
-                id[d] = v < 0 ? 0 : (v > nn[d] - 1 ? nn[d] - 1 : v);
+                id[d] = b[d] + o;
             }
             val[e] = F.at(id[0], id[1], id[2]);
         }
@@ -244,15 +248,12 @@ __device__ inline double interp_slot(const AxisGuess<D>& Gs, const Vel<D>& vg,
     if constexpr (S == kLinear) {
         return vl;
     } else {
-        int64_t nn[D];
         bool interior = true;
 #pragma unroll
-        for (int d = 0; d < D; ++d) {
-            nn[d] = vg.ax[c][d].n;
-            interior = interior && k[d] >= 1 && k[d] <= nn[d] - 3;
-        }
+        for (int d = 0; d < D; ++d)
+            interior = interior && k[d] >= 1 && k[d] <= vg.ax[c][d].n - 3;
         if (!interior) return vl;
-        const FView Fv{F, n0, n1};
+        const FView<int64_t> Fv{F, n0, n1};
         if constexpr (S == kMQS) {
             return mqs<D>(Fv, c, k, q, t);
         } else {
@@ -264,7 +265,7 @@ __device__ inline double interp_slot(const AxisGuess<D>& Gs, const Vel<D>& vg,
                 dxi[d] = A.dx[k[d]];
                 idx[d] = A.idx[k[d]];
             }
-            const double vp = linp<D>(Fv, nn, c, k, xc, dxi, idx, p);
+            const double vp = linp<D>(Fv, c, k, xc, dxi, idx, p);
             const double A = 2.0 / 3.0;
             return A * vl + (1.0 - A) * vp;
         }
@@ -367,16 +368,18 @@ __global__ void __launch_bounds__(kBlock) k_advect_slot(Grid<D> g, Vel<D> vg, VP
     for (int d = 0; d < D; ++d) coords.p[d][e] = out[d];
 }
 
-// The linear scheme with the velocity staged in LDS: one workgroup per tile
-// of cells (2D 64x4, 3D 16x4x4), one thread per cell walking the cell's slot
-// planes in lockstep chunks (a wavefront covers whole 128-byte runs of a
-// plane).  Each
+// The velocity staged in LDS: one workgroup per tile of cells (2D 64x4, 3D
+// 16x4x4), one thread per cell walking the cell's slot planes in lockstep
+// chunks (a wavefront covers whole 128-byte runs of a plane).  Each
 // component's window holds the nodes from two below the tile's first bracket
 // to kWinPad - 2 beyond its end, which covers the RK stage points of a step of
-// up to one cell; its axis coordinates and inverse spacings are staged too.
-// A bracket, and the corner values, come from the window when they lie in it
-// and from global memory otherwise, with the same tests and the same values
-// as the slot kernel, so the results are identical.
+// up to one cell and the extra nodes of MQS and LinP around them; its axis
+// coordinates and inverse spacings are staged too.  A bracket, and the nodal
+// values, come from the window when they lie in it and from global memory
+// otherwise, with the same tests and the same values as the slot kernel, so
+// the results are identical.  Bound by FP64 issue and LDS reads: RK2 98 us at
+// 512^2, RK4 594 us at 61 x 47 x 74; MQS RK2 88 us at 300 x 431 (the slot
+// kernel, which gathers its stencils from global memory: 191).
 template <int D>
 struct F64Tile;
 template <>
@@ -397,36 +400,71 @@ struct F64Win {
 };
 
 // window entries past the end of an axis hold NaN (no bracket test passes)
-template <int D>
+template <int D, int S>
 struct TileLds {
     double v[D][F64Win<D>::size()];
     double x[D][D][F64Win<D>::axis()];
     double idx[D][D][F64Win<D>::axis()];
+    double dx[S == kLinP ? D : 1][D][S == kLinP ? F64Win<D>::axis() : 1];
 };
+// where the windows sit: first node of component c along d, and the window
+// position of the bracket that the tile's first cell guesses
+template <int D>
+struct TileWin {
+    int64_t lo[D][D];
+    int seed[D][D];
+};
+
+// The bracket k of p in a window of W axis nodes x (inverse spacings idx) and
+// its node xl; false if it does not hold p strictly: the uniform-spacing
+// guess, or (REF: a refined axis) up to two steps from `seed`, the particle's
+// cell's own position.
+template <bool REF>
+__device__ inline bool window_bracket(double p, const double* x, const double* idx, int W,
+                                      int seed, int& k, double& xl) {
+    if constexpr (!REF) {
+        const double g = (p - x[0]) * idx[0];
+        k = g >= 0.0 ? (g < (double)(W - 2) ? (int)g : W - 2) : 0;
+    } else {
+        k = seed < W - 2 ? seed : W - 2;
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            k += (p > x[k + 1] ? 1 : 0) - (p < x[k] ? 1 : 0);
+            k = k < 0 ? 0 : (k > W - 2 ? W - 2 : k);
+        }
+    }
+    xl = x[k];
+    const double xr = x[k + 1];
+    return xl < p && p < xr;
+}
 
 // Component c at p from the window, if every axis brackets p strictly inside
 // it (that bracket is the axis's only one, the one the slot kernel finds, and
-// it lies inside the component's grid); false otherwise.
-template <int D>
-__device__ inline bool interp_tile_f64(const TileLds<D>& L, int c, const double (&p)[D],
-                                       double& v) {
+// it lies inside the component's grid) and the window holds the scheme's
+// nodes around it; false otherwise.  cell: the particle's cell in the tile.
+template <int D, int S, bool REF>
+__device__ inline bool interp_tile_f64(const TileLds<D, S>& L, const TileWin<D>& wn,
+                                       const Vel<D>& vg, int c, const int (&cell)[D],
+                                       const double (&p)[D], double& v) {
+    using WN = F64Win<D>;
     int w[D];
     double t[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-        const double g = (p[d] - L.x[c][d][0]) * L.idx[c][d][0];
-        int k = g >= 0.0 ? (g < (double)(F64Win<D>::w(d) - 2) ? (int)g : F64Win<D>::w(d) - 2) : 0;
-        const double xl = L.x[c][d][k], xr = L.x[c][d][k + 1];
-        if (!(xl < p[d] && p[d] < xr)) return false;
+        int k;
+        double xl;
+        if (!window_bracket<REF>(p[d], L.x[c][d], L.idx[c][d], WN::w(d),
+                                 REF ? wn.seed[c][d] + cell[d] : 0, k, xl))
+            return false;
         w[d] = k;
         t[d] = (p[d] - xl) * L.idx[c][d][k];
     }
-    const int b = w[0] + F64Win<D>::w(0) * (w[1] + (D == 3 ? F64Win<D>::w(1) * w[D - 1] : 0));
+    const int b = w[0] + WN::w(0) * (w[1] + (D == 3 ? WN::w(1) * w[D - 1] : 0));
     double q[1 << D];
 #pragma unroll
     for (int r = 0; r < (1 << D); ++r) {
-        const int o = (r & 1) + ((r >> 1) & 1) * F64Win<D>::w(0) +
-                      (D == 3 ? ((r >> 2) & 1) * F64Win<D>::w(0) * F64Win<D>::w(1) : 0);
+        const int o = (r & 1) + ((r >> 1) & 1) * WN::w(0) +
+                      (D == 3 ? ((r >> 2) & 1) * WN::w(0) * WN::w(1) : 0);
         q[r] = L.v[c][b + o];
     }
     double vl = lerp1(t[1], lerp1(t[0], q[0], q[1]), lerp1(t[0], q[2], q[3]));
@@ -434,24 +472,52 @@ __device__ inline bool interp_tile_f64(const TileLds<D>& L, int c, const double 
         const double hi = lerp1(t[1], lerp1(t[0], q[4], q[5]), lerp1(t[0], q[6], q[7]));
         vl = lerp1(t[2], vl, hi);
     }
+    if constexpr (S != kLinear) {
+        bool interior = true, held = true;
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            const int64_t k = wn.lo[c][d] + w[d];
+            interior = interior && k >= 1 && k <= vg.ax[c][d].n - 3;
+            held = held && w[d] >= 1 && w[d] <= WN::w(d) - 3;
+        }
+        if (interior) {
+            if (!held) return false;
+            const FView<int> Fv{L.v[c], WN::w(0), WN::w(1)};
+            if constexpr (S == kMQS) {
+                vl = mqs<D>(Fv, c, w, q, t);
+            } else {
+                double xc[D], dxi[D], idx[D];
+#pragma unroll
+                for (int d = 0; d < D; ++d) {
+                    xc[d] = L.x[c][d][w[d]];
+                    dxi[d] = L.dx[c][d][w[d]];
+                    idx[d] = L.idx[c][d][w[d]];
+                }
+                const double vp = linp<D>(Fv, c, w, xc, dxi, idx, p);
+                const double A = 2.0 / 3.0;
+                vl = A * vl + (1.0 - A) * vp;
+            }
+        }
+    }
     v = vl;
     return true;
 }
 
-// B: slot planes per chunk; FLAGS: particles whose step leaves the windows
-// are flagged (flags[slot], written for every slot of the tile's planes) for
-// k_advect_flagged instead of being advected inline, and the workgroup
-// records whether it flagged any (any[workgroup])
-template <int D, int M, int B, bool FLAGS>
-__global__ void __launch_bounds__(kBlock) k_advect_tile(Grid<D> g, Vel<D> vg, VPtrs<D> V,
+// B: slot planes per chunk.  A particle whose step leaves the windows (or
+// sits on a node) is marked in its cell's word and advected as k_advect_slot
+// does after the tile's other particles: inside the chunk loop that path costs
+// the loop's occupancy (2D RK2 169 registers, two wavefronts per SIMD instead
+// of four: 165 us against 98 at 512^2), and a flag per slot with a pass of its
+// own costs a launch.
+template <int D, int M, int S, int B>
+__global__ void __launch_bounds__(kBlock, D == 2 ? 4 : 2) k_advect_tile(Grid<D> g, Vel<D> vg, VPtrs<D> V,
                                                         Ptr3 coords,
                                                         const uint8_t* __restrict__ index,
-                                                        uint8_t* __restrict__ flags,
-                                                        uint8_t* __restrict__ any, RKParams P,
-                                                        int span) {
+                                                        RKParams P, int span) {
     using TL = F64Tile<D>;
     using WN = F64Win<D>;
-    __shared__ TileLds<D> L;
+    __shared__ TileLds<D, S> L;
+    __shared__ unsigned long long s_miss[kBlock];  // per cell: slots to do on the slot path
     int64_t t0[D];
     {
         int64_t b = blockIdx.x;
@@ -465,21 +531,55 @@ __global__ void __launch_bounds__(kBlock) k_advect_tile(Grid<D> g, Vel<D> vg, VP
     const int kb = blockIdx.y * span;
     const int ke = kb + span < g.K ? kb + span : g.K;
     const int tid = threadIdx.x;
-    // window origins: two nodes below the guessed bracket of the tile's first
-    // vertex (only where the window sits depends on the guess, not a result)
-    int64_t wlo[D][D];
+    // window origins: two nodes below the bracket of the tile's first vertex
+    // (only where the window sits depends on it, not a result).  On the
+    // staggered grids that is the cell's own number, refined or not; other
+    // axes search.
+    TileWin<D> wn;
+    {
+        // (all loads before the first test: one round trip, not one per axis)
+        double xt[D], xa[D][D], xb[D][D];
+        bool ok = true;
 #pragma unroll
-    for (int c = 0; c < D; ++c)
+        for (int d = 0; d < D; ++d) xt[d] = g.xv[d].x[t0[d]];
 #pragma unroll
-        for (int d = 0; d < D; ++d) {
-            const Axis& A = vg.ax[c][d];
-            const double x = g.xv[d].x[t0[d]];
-            const int64_t last = A.n - 2;
-            int64_t gk = (int64_t)((x - A.x[0]) * A.idx[0]);
-            gk = gk < 0 ? 0 : (gk > last ? last : gk);
-            wlo[c][d] = gk - 2 < 0 ? 0 : gk - 2;
+        for (int c = 0; c < D; ++c)
+#pragma unroll
+            for (int d = 0; d < D; ++d) {  // (an axis has more nodes than the grid cells)
+                xa[c][d] = vg.ax[c][d].x[t0[d]];
+                xb[c][d] = vg.ax[c][d].x[t0[d] + 1];
+            }
+#pragma unroll
+        for (int c = 0; c < D; ++c)
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                ok = ok && xa[c][d] <= xt[d] && xt[d] <= xb[c][d];
+                wn.lo[c][d] = t0[d];
+            }
+        if (!ok) {
+#pragma unroll 1
+            for (int c = 0; c < D; ++c)
+#pragma unroll 1
+                for (int d = 0; d < D; ++d) {
+                    const Axis A = vg.ax[c][d];
+                    const double x0 = A.x[0], xn = A.x[A.n - 1], x = g.xv[d].x[t0[d]];
+                    const int64_t k = find_cell(x < x0 ? x0 : (x > xn ? xn : x), A, t0[d]);
+#pragma unroll
+                    for (int q = 0; q < D * D; ++q)
+                        if (q == c * D + d) wn.lo[q / D][q % D] = k;
+                }
         }
+#pragma unroll
+        for (int c = 0; c < D; ++c)
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                const int64_t k = wn.lo[c][d];
+                wn.lo[c][d] = k - 2 < 0 ? 0 : k - 2;
+                wn.seed[c][d] = (int)(k - wn.lo[c][d]);
+            }
+    }
     const double qnan = __builtin_nan("");
+    bool off = false;  // an axis of the windows is not uniform
 #pragma unroll
     for (int c = 0; c < D; ++c) {
         const double* __restrict__ F = V.v[c];
@@ -489,7 +589,7 @@ __global__ void __launch_bounds__(kBlock) k_advect_tile(Grid<D> g, Vel<D> vg, VP
             bool ok = true;
 #pragma unroll
             for (int d = 0; d < D; ++d) {
-                const int64_t kk = wlo[c][d] + r % WN::w(d);
+                const int64_t kk = wn.lo[c][d] + r % WN::w(d);
                 r /= WN::w(d);
                 ok = ok && kk < vg.ax[c][d].n;
                 node += kk * stride;
@@ -501,12 +601,22 @@ __global__ void __launch_bounds__(kBlock) k_advect_tile(Grid<D> g, Vel<D> vg, VP
         for (int d = 0; d < D; ++d)
             for (int w = tid; w < WN::w(d); w += kBlock) {
                 const Axis& A = vg.ax[c][d];
-                const int64_t kk = wlo[c][d] + w;
-                L.x[c][d][w] = kk < A.n ? A.x[kk] : qnan;
+                const int64_t kk = wn.lo[c][d] + w;
+                const double x = kk < A.n ? A.x[kk] : qnan;
+                L.x[c][d][w] = x;
                 L.idx[c][d][w] = kk < A.n - 1 ? A.idx[kk] : qnan;
+                // (false for NaN)
+                off = off || fabs((x - A.x[wn.lo[c][d]]) * A.idx[wn.lo[c][d]] - (double)w) > 1e-4;
+                if constexpr (S == kLinP) L.dx[c][d][w] = kk < A.n - 1 ? A.dx[kk] : qnan;
             }
     }
-    __syncthreads();
+    // one refined axis in the windows: brackets start from the particle's cell
+    // (the uniform-spacing guess of a window of ~70 refined nodes misses, and
+    // every miss is a step on the slot path: 284 us at 389 x 211 with RK4, 85
+    // with the search; for uniform axes the guess is the shorter way, and a
+    // spacing off by 1e-4 misses too rarely to matter)
+    s_miss[tid] = 0;
+    const bool refined = __builtin_amdgcn_readfirstlane(__syncthreads_or(off ? 1 : 0)) != 0;
     // the cell of thread t of the tile and whether it is in the grid
     auto cell_of = [&](int t, int64_t (&J)[D]) {
         bool in = true;
@@ -523,15 +633,10 @@ __global__ void __launch_bounds__(kBlock) k_advect_tile(Grid<D> g, Vel<D> vg, VP
     const bool inside = cell_of(tid, I);
     const int64_t c = inside ? lin<D>(g.ni, I) : 0;
     const int64_t C = g.C;
-    // the step from the windows; if any stage point leaves a window (or sits
-    // on a node), the whole step again on the slot kernel's path: inline
-    // (2D), or in the flagged pass that follows (3D, where inlining it
-    // doubles the registers)
+    // the step from the windows
     bool win = true;
-    auto interp = [&](const double (&p)[D], double (&v)[D]) {
-#pragma unroll
-        for (int cc = 0; cc < D; ++cc) win = interp_tile_f64<D>(L, cc, p, v[cc]) && win;
-    };
+    int cell[D];  // of the particle, in the tile
+
     // a thread outside the grid owns no particle but still takes work
     const uint64_t act = !inside ? 0ull
                                  : ((kb == 0 && ke == g.K) ? active_slots(index, c, C, g.K)
@@ -545,106 +650,72 @@ __global__ void __launch_bounds__(kBlock) k_advect_tile(Grid<D> g, Vel<D> vg, VP
     __shared__ uint16_t s_items[kBlock / 64][B * 64];
     uint16_t* items = s_items[tid >> 6];
     const int lane = tid & 63, wbase = tid & ~63;
-    bool missed = false;
-    for (int k0 = kb; k0 < ke; k0 += B) {
-        if constexpr (FLAGS) {  // every slot of the chunk: no miss yet
+    auto chunks = [&](auto ref) {
+        auto interp = [&](const double (&p)[D], double (&v)[D]) {
 #pragma unroll
-            for (int j = 0; j < B; ++j)
-                if (inside && k0 + j < ke) flags[c + C * (k0 + j)] = 0;
-        }
-        int n = 0;
+            for (int cc = 0; cc < D; ++cc)
+                win = interp_tile_f64<D, S, decltype(ref)::value>(L, wn, vg, cc, cell, p, v[cc]) &&
+                      win;
+        };
+        for (int k0 = kb; k0 < ke; k0 += B) {
+            int n = 0;
 #pragma unroll
-        for (int j = 0; j < B; ++j) {
-            const bool a = k0 + j < 64 && ((act >> (k0 + j)) & 1);
-            const uint64_t bal = __ballot(a);
-            const int below = (int)__builtin_amdgcn_mbcnt_hi(
-                (uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-            if (a) items[n + below] = (uint16_t)((j << 6) | lane);
-            n += __popcll(bal);
-        }
-        if (!n) continue;
-        // this lane's entries lane, lane + 64, ...: positions loaded first
-        double pq[B][D];
-        int dq[B];
+            for (int j = 0; j < B; ++j) {
+                const bool a = k0 + j < 64 && ((act >> (k0 + j)) & 1);
+                const uint64_t bal = __ballot(a);
+                const int below = (int)__builtin_amdgcn_mbcnt_hi(
+                    (uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+                if (a) items[n + below] = (uint16_t)((j << 6) | lane);
+                n += __popcll(bal);
+            }
+            if (!n) continue;
+            // this lane's entries lane, lane + 64, ...: positions loaded first
+            double pq[B][D];
+            int dq[B];
 #pragma unroll
-        for (int q = 0; q < B; ++q) {
-            const int item = lane + 64 * q;
-            dq[q] = item < n ? items[item] : -1;
-            int64_t J[D];
-            cell_of(wbase + (dq[q] & 63), J);
-            const int64_t e = lin<D>(g.ni, J) + C * (k0 + (dq[q] >> 6));
+            for (int q = 0; q < B; ++q) {
+                const int item = lane + 64 * q;
+                dq[q] = item < n ? items[item] : -1;
+                int64_t J[D];
+                cell_of(wbase + (dq[q] & 63), J);
+                const int64_t e = lin<D>(g.ni, J) + C * (k0 + (dq[q] >> 6));
 #pragma unroll
-            for (int d = 0; d < D; ++d) pq[q][d] = dq[q] >= 0 ? coords.p[d][e] : 0.0;
-        }
-#pragma unroll
-        for (int q = 0; q < B; ++q) {
-            if (dq[q] < 0) break;
-            int64_t J[D];
-            cell_of(wbase + (dq[q] & 63), J);
-            const int64_t e = lin<D>(g.ni, J) + C * (k0 + (dq[q] >> 6));
-            double out[D];
-            win = true;
-            advect_rk<D, M>(P, pq[q], out, interp);
-            if (!win) {
-                if constexpr (FLAGS) {
-                    flags[e] = 1;  // the flagged pass advects it
-                    missed = true;
-                    continue;
-                } else {
-                    AxisGuess<D> Gs;
-                    axis_guess<D>(vg, Gs);
-                    advect_slot<D, M>(Gs, vg, V, P, pq[q], J, out);
-                }
+                for (int d = 0; d < D; ++d) pq[q][d] = dq[q] >= 0 ? coords.p[d][e] : 0.0;
             }
 #pragma unroll
-            for (int d = 0; d < D; ++d) coords.p[d][e] = out[d];
-        }
-    }
-    if constexpr (FLAGS) {
-        const int m = __syncthreads_or(missed ? 1 : 0);
-        if (tid == 0) any[blockIdx.x + (int64_t)gridDim.x * blockIdx.y] = m ? 1 : 0;
-    }
-}
-
-// the flagged particles of the tiled kernel: the same grid of tiles and slot
-// groups, a workgroup returning at once unless its tile flagged some; then
-// one thread per cell of the tile walks its slots, advecting the flagged ones
-// as k_advect_slot does
-template <int D, int M>
-__global__ void __launch_bounds__(kBlock) k_advect_flagged(Grid<D> g, Vel<D> vg, VPtrs<D> V,
-                                                           Ptr3 coords,
-                                                           const uint8_t* __restrict__ flags,
-                                                           const uint8_t* __restrict__ any,
-                                                           RKParams P, int span) {
-    using TL = F64Tile<D>;
-    if (!any[blockIdx.x + (int64_t)gridDim.x * blockIdx.y]) return;
-    int64_t I[D];
-    {
-        int64_t b = blockIdx.x;
-        int r = threadIdx.x;
-        bool in = true;
+            for (int q = 0; q < B; ++q) {
+                if (dq[q] < 0) break;
+                int64_t J[D];
+                cell_of(wbase + (dq[q] & 63), J);
+                const int64_t e = lin<D>(g.ni, J) + C * (k0 + (dq[q] >> 6));
+                double out[D];
+                win = true;
 #pragma unroll
-        for (int d = 0; d < D; ++d) {
-            const int64_t nt = (g.ni[d] + TL::n[d] - 1) / TL::n[d];
-            I[d] = (b % nt) * TL::n[d] + r % TL::n[d];
-            b /= nt;
-            r /= TL::n[d];
-            in = in && I[d] < g.ni[d];
+                for (int d = 0; d < D; ++d) cell[d] = (int)(J[d] - t0[d]);
+                advect_rk<D, M>(P, pq[q], out, interp);
+                if (!win) {
+                    atomicOr(&s_miss[wbase + (dq[q] & 63)], 1ull << (k0 + (dq[q] >> 6)));
+                    continue;
+                }
+#pragma unroll
+                for (int d = 0; d < D; ++d) coords.p[d][e] = out[d];
+            }
         }
-        if (!in) return;
-    }
-    const int kb = blockIdx.y * span;
-    const int ke = kb + span < g.K ? kb + span : g.K;
-    const int64_t c = lin<D>(g.ni, I);
+    };
+    if (refined) chunks(std::true_type{});
+    else chunks(std::false_type{});
+    __syncthreads();
+    uint64_t miss = inside ? s_miss[tid] : 0;
+    if (!miss) return;
     AxisGuess<D> Gs;
     axis_guess<D>(vg, Gs);
-    for (int k = kb; k < ke; ++k) {
-        const int64_t e = c + g.C * (int64_t)k;
-        if (!flags[e]) continue;
+    while (miss) {
+        const int64_t e = c + C * __builtin_ctzll(miss);
+        miss &= miss - 1;
         double p0[D], out[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) p0[d] = coords.p[d][e];
-        advect_slot<D, M>(Gs, vg, V, P, p0, I, out);
+        advect_slot<D, M, S>(Gs, vg, V, P, p0, I, out);
 #pragma unroll
         for (int d = 0; d < D; ++d) coords.p[d][e] = out[d];
     }
@@ -742,35 +813,17 @@ Vel<D> to_vel(const jp_velgrid* vg) {
 template <int D, int M, int S>
 int launch(jp_ctx* ctx, const Grid<D>& G, const Vel<D>& vg, const VPtrs<D>& V, Ptr3 cp,
            const uint8_t* index, const RKParams& P) {
-    if constexpr (S == kLinear) {
-        if (!ctx->opt_advect_slots) {
-            int64_t tiles = 1;
-            for (int d = 0; d < D; ++d)
-                tiles *= (G.ni[d] + F64Tile<D>::n[d] - 1) / F64Tile<D>::n[d];
-            // slot groups when the tiles alone leave the chip under-filled
-            const int span = slot_span(ctx, tiles, G.K, 2048);
-            const dim3 grid((unsigned)tiles, (unsigned)((G.K + span - 1) / span));
-            if constexpr (D == 2) {
-                k_advect_tile<D, M, 8, false><<<grid, kBlock, 0, ctx->stream>>>(
-                    G, vg, V, cp, index, nullptr, nullptr, P, span);
-                JP_LAUNCHED(ctx);
-            } else {
-                // scratch: a flag per slot | a flag per workgroup
-                const size_t nf = ((size_t)G.C * G.K + 255) & ~(size_t)255;
-                const size_t nwg = (size_t)grid.x * grid.y;
-                int rc = ensure_scratch(ctx, nf + nwg);
-                if (rc) return rc;
-                uint8_t* flags = static_cast<uint8_t*>(ctx->scratch);
-                uint8_t* any = flags + nf;
-                k_advect_tile<D, M, 4, true><<<grid, kBlock, 0, ctx->stream>>>(
-                    G, vg, V, cp, index, flags, any, P, span);
-                JP_LAUNCHED(ctx);
-                k_advect_flagged<D, M><<<grid, kBlock, 0, ctx->stream>>>(G, vg, V, cp, flags,
-                                                                        any, P, span);
-                JP_LAUNCHED(ctx);
-            }
-            return JP_OK;
-        }
+    if (!ctx->opt_advect_slots) {
+        int64_t tiles = 1;
+        for (int d = 0; d < D; ++d)
+            tiles *= (G.ni[d] + F64Tile<D>::n[d] - 1) / F64Tile<D>::n[d];
+        // slot groups when the tiles alone leave the chip under-filled
+        const int span = slot_span(ctx, tiles, G.K, 2048);
+        const dim3 grid((unsigned)tiles, (unsigned)((G.K + span - 1) / span));
+        k_advect_tile<D, M, S, D == 2 ? 8 : 4><<<grid, kBlock, 0, ctx->stream>>>(G, vg, V, cp,
+                                                                                index, P, span);
+        JP_LAUNCHED(ctx);
+        return JP_OK;
     }
     dim3 grid((unsigned)row_blocks<D>(G), (unsigned)G.K);
     k_advect_slot<D, M, S><<<grid, kBlock, 0, ctx->stream>>>(G, vg, V, cp, index, P);
