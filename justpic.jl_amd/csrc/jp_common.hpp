@@ -240,18 +240,42 @@ __device__ inline uint64_t active_slots_in(const uint8_t* __restrict__ index, in
     return bits;
 }
 
-// Nearest-neighbour search of the injection on squared distances.
-// wave_argmin: lexicographic minimum of (s, order) over the wavefront.
+// Minimum over the wavefront by data-parallel-primitive shifts (no LDS round
+// trips): within rows of 16 lanes, then across the rows; lane 63 holds it.
+__device__ inline uint32_t wave_min(uint32_t v) {
+    constexpr int kId = -1;
+    auto step = [&](uint32_t o) { v = o < v ? o : v; };
+    step((uint32_t)__builtin_amdgcn_update_dpp(kId, (int)v, 0x111, 0xf, 0xf, false));  // row_shr 1
+    step((uint32_t)__builtin_amdgcn_update_dpp(kId, (int)v, 0x112, 0xf, 0xf, false));  // 2
+    step((uint32_t)__builtin_amdgcn_update_dpp(kId, (int)v, 0x114, 0xf, 0xf, false));  // 4
+    step((uint32_t)__builtin_amdgcn_update_dpp(kId, (int)v, 0x118, 0xf, 0xf, false));  // 8
+    step((uint32_t)__builtin_amdgcn_update_dpp(kId, (int)v, 0x142, 0xa, 0xf, false));  // bcast 15
+    step((uint32_t)__builtin_amdgcn_update_dpp(kId, (int)v, 0x143, 0xc, 0xf, false));  // bcast 31
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// Nearest-neighbour search of the injection on squared distances (not
+// negative, not NaN: their bits order them).  wave_argmin: lexicographic
+// minimum of (s, order) over the wavefront; every lane must call it.
 __device__ inline void wave_argmin(double& best, int& border) {
-#pragma unroll
-    for (int sh = 32; sh >= 1; sh >>= 1) {
-        const double ob = __shfl_xor(best, sh, 64);
-        const int oo = __shfl_xor(border, sh, 64);
-        if (ob < best || (ob == best && oo < border)) {
-            best = ob;
-            border = oo;
+    const uint64_t b = (uint64_t)__double_as_longlong(best);
+    const uint32_t hi = (uint32_t)(b >> 32), lo = (uint32_t)b;
+    const uint32_t mh = wave_min(hi);
+    uint64_t at = __ballot(hi == mh);
+    if (at & (at - 1)) {  // several lanes: the low words, then the order
+        const uint32_t ml = wave_min(hi == mh ? lo : ~0u);
+        at = __ballot(hi == mh && lo == ml);
+        if (at & (at - 1)) {
+            const uint32_t mo = wave_min(hi == mh && lo == ml ? (uint32_t)border : ~0u);
+            best = __longlong_as_double((long long)(((uint64_t)mh << 32) | ml));
+            border = (int)mo;
+            return;
         }
     }
+    const int l = __builtin_ctzll(at);
+    const uint32_t bl = (uint32_t)__builtin_amdgcn_readlane((int)lo, l);
+    best = __longlong_as_double((long long)(((uint64_t)mh << 32) | bl));
+    border = __builtin_amdgcn_readlane(border, l);
 }
 
 // The reference takes the first element (in order) of minimal distance
@@ -278,10 +302,13 @@ __device__ inline void resolve_ties(const double (&s9)[NB], double best, int& bo
     border = min(border, o);
 }
 
-// a neighbour cell whose squared bound exceeds best (1 + 2^-40) cannot hold
-// an element within the tie range above (the margin covers the rounding of
-// the bound)
-constexpr double kPrune = 1.0 + 0x1p-40;
+// The same with one element per lane, s at `order` (0x7fffffff: none).
+__device__ inline void resolve_ties_at(double s, int order, double best, int& border) {
+    const bool near = order != 0x7fffffff && s > best && s <= best * (1.0 + 0x1p-50);
+    if (!__any(near)) return;
+    const uint32_t o = wave_min(near && sqrt(s) == sqrt(best) ? (uint32_t)order : 0x7fffffffu);
+    border = min(border, (int)o);
+}
 
 // Appends c to the list segment of its wavefront and colour without atomics:
 // segment (q, wave) holds up to 64 cells at seg[(q*nwave + wave)*64 + i] and

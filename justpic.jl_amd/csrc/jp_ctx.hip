@@ -188,17 +188,15 @@ int occ_words(jp_ctx* ctx, const uint8_t* index, int64_t C, int K, uint64_t* occ
     return JP_OK;
 }
 
-int inject_lists(jp_ctx* ctx, int64_t C, int nq, int64_t cap, size_t box_bytes, InjectLists& L) {
-    // scratch: totals | counts | segments | lists | occupancy words | boxes | states
+int inject_lists(jp_ctx* ctx, int64_t C, int nq, int64_t cap, bool ordered, InjectLists& L) {
+    // scratch: totals | counts | segments | lists | occupancy words | states
     L.nwave = (C + 63) / 64;
     const size_t a = 256;
     const size_t b = a + (((size_t)nq * L.nwave * 4 + 255) & ~(size_t)255);
     const size_t c = b + (size_t)nq * L.nwave * 64 * 4;
     const size_t d = c + (((size_t)nq * cap * 4 + 255) & ~(size_t)255);
     const size_t e = d + (((size_t)C * 8 + 255) & ~(size_t)255);
-    const size_t f = e + ((box_bytes + 255) & ~(size_t)255);
-    const size_t h = f + (size_t)C * 4;
-    int rc = ensure_scratch(ctx, h);
+    int rc = ensure_scratch(ctx, e + (size_t)C * 4);
     if (rc) return rc;
     char* base = static_cast<char*>(ctx->scratch);
     L.total = reinterpret_cast<int32_t*>(base);
@@ -206,8 +204,9 @@ int inject_lists(jp_ctx* ctx, int64_t C, int nq, int64_t cap, size_t box_bytes, 
     L.seg = reinterpret_cast<int32_t*>(base + b);
     L.list = reinterpret_cast<int32_t*>(base + c);
     L.occ = reinterpret_cast<uint64_t*>(base + d);
-    L.box = box_bytes ? static_cast<void*>(base + e) : nullptr;
-    L.state = reinterpret_cast<uint32_t*>(base + f);
+    uint32_t* const per_cell = reinterpret_cast<uint32_t*>(base + e);
+    L.state = ordered ? per_cell : nullptr;
+    L.out = ordered ? nullptr : per_cell;
     L.cap = cap;
     return JP_OK;
 }

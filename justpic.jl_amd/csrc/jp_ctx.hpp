@@ -155,10 +155,11 @@ struct InjectLists {
     int64_t nwave;
     int64_t cap;
     uint64_t* occ;  // occupancy word of every cell
-    void* box;      // 2*D planes of C: per-cell min, max of each coordinate (2D)
-    uint32_t* state;  // per cell, written by the scan: 1 listed, 0 not (ordered 2D injection)
+    // per cell, written by the scan, one of the two null:
+    uint32_t* state;  // ordered 2D injection: 1 listed, 0 not
+    uint32_t* out;    // colour launches: a particle lies outside the cell's box
 };
-int inject_lists(jp_ctx* ctx, int64_t C, int nq, int64_t cap, size_t box_bytes, InjectLists& L);
+int inject_lists(jp_ctx* ctx, int64_t C, int nq, int64_t cap, bool ordered, InjectLists& L);
 int join_segments(jp_ctx* ctx, int nq, const InjectLists& L);
 // workgroups (4 wavefronts each) of persistent wavefronts for a work list of
 // at most n entries: one wavefront per entry up to 4096

@@ -4,6 +4,7 @@
 // jp_move.hip).
 #include "jp_ctx.hpp"
 #include "jp_inject2.hpp"
+#include "jp_inject_cells.hpp"
 
 #include <cmath>
 #include <type_traits>
@@ -374,12 +375,14 @@ __global__ void __launch_bounds__(kBlock) k_inject_scan(Grid<D> g, CPtr3 coords,
     int64_t I[D];
     unlin<D>(g.ni, valid ? c : 0, I);
     int num = 0;
+    bool out = false;  // a particle outside the cell's box (or NaN)
     int cnt_q[1 << D] = {};  // ANYQ: particles strictly inside quadrants 1..2^D-1
     if (valid) {
-        double lo[D], hq[D];
+        double lo[D], hi[D], hq[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             lo[d] = g.xv[d].x[I[d]];
+            hi[d] = g.xv[d].x[I[d] + 1];
             hq[d] = g.xv[d].dx[I[d]] / 2.0;
         }
         // quadrant c11: vertex + dq*0 (src/Particles/injection.jl:442-448)
@@ -390,12 +393,6 @@ __global__ void __launch_bounds__(kBlock) k_inject_scan(Grid<D> g, CPtr3 coords,
             q1[d] = q0[d] + hq[d];
         }
         const uint64_t act = active_slots(index, c, g.C, g.K);
-        double bl[D], bh[D];  // box of the cell's particles (NaN coordinates ignored)
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            bl[d] = __builtin_inf();
-            bh[d] = -__builtin_inf();
-        }
         constexpr int B = 16;  // slots per chunk; lanes share the slot plane (coalesced)
         for (int k0 = 0; k0 < g.K; k0 += B) {
             double pb[B][D];
@@ -412,10 +409,7 @@ __global__ void __launch_bounds__(kBlock) k_inject_scan(Grid<D> g, CPtr3 coords,
 #pragma unroll
                 for (int d = 0; d < D; ++d) {
                     inside = inside & (q0[d] < pb[j][d] && pb[j][d] < q1[d]);
-                    if (D == 2 && on) {
-                        bl[d] = fmin(bl[d], pb[j][d]);
-                        bh[d] = fmax(bh[d], pb[j][d]);
-                    }
+                    out = out || (on && !(lo[d] <= pb[j][d] && pb[j][d] <= hi[d]));
                 }
                 num += inside ? 1 : 0;
                 if constexpr (ANYQ) {
@@ -434,14 +428,7 @@ __global__ void __launch_bounds__(kBlock) k_inject_scan(Grid<D> g, CPtr3 coords,
             }
         }
         L.occ[c] = act;
-        if (D == 2 && L.box) {
-            double* __restrict__ bx = static_cast<double*>(L.box);
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                bx[(2 * d) * g.C + c] = bl[d];
-                bx[(2 * d + 1) * g.C + c] = bh[d];
-            }
-        }
+        if (L.out) L.out[c] = out ? 1u : 0u;
     }
     bool want = valid && num < min_q;
     if constexpr (ANYQ) {
@@ -453,292 +440,6 @@ __global__ void __launch_bounds__(kBlock) k_inject_scan(Grid<D> g, CPtr3 coords,
 #pragma unroll
     for (int d = 0; d < D; ++d) col = col * 2 + (int)(I[d] & 1);
     wave_segment<D == 2 ? 4 : 8>(want, col, (int32_t)c, c >> 6, L.nwave, L.seg, L.cnt);
-}
-
-// _inject_particles! (src/Particles/injection.jl:68-131) with one wavefront per
-// listed cell: lane k owns slot k of the cell (K <= 64).  Quadrant counts are
-// ballots; injected particles fill the free slots in ascending order, and the
-// nearest-neighbour search of index_min_distance (:330-393) evaluates the
-// 3^D x K candidates lane-parallel, keeping the reference's first-occurrence
-// tie rule (strict '<' in loop order: neighbour cell, then slot) through a
-// (distance, order) argmin.
-//
-// PHASE: _inject_particles_phase! (src/Particles/injection.jl:233-325): every
-// short quadrant is topped up (`continue` past a full one, :278), the new
-// particle takes its nearest neighbour's phase, and each arg is interpolated
-// from its field (cell-centred or nodal) and clamped to the corner extrema.
-struct PhaseInj {
-    double* phases;
-    const double* fields[JP_MAX_ARGS];
-    uint32_t centred;  // bit a: fields[a] is cell-centred (dims ni), else nodal (ni + 1)
-    Axis xc[3];        // centre axes (particles.xci with di.center)
-};
-
-// Julia's min / max on Float64 (NaN-propagating, -0.0 below 0.0) and clamp
-__device__ inline double jl_min(double x, double y) {
-    if (x != x || y != y) return x != x ? x : y;
-    return (x < y || (x == y && signbit(x) && !signbit(y))) ? x : y;
-}
-__device__ inline double jl_max(double x, double y) {
-    if (x != x || y != y) return x != x ? x : y;
-    return (x > y || (x == y && !signbit(x) && signbit(y))) ? x : y;
-}
-
-// _grid2particle at corner cell idx of F (dims nn), t = (p - x0) * inv(di),
-// clamped to the extrema of the 2^D corner values (src/Particles/
-// injection.jl:299-314, cell_field :395-409)
-template <int D>
-__device__ double g2p_clamped(const double* __restrict__ F, const int64_t (&nn)[D],
-                              const int64_t (&idx)[D], const double (&p)[D],
-                              const double (&x0)[D], const double (&inv)[D]) {
-    double v[1 << D], t[D];
-#pragma unroll
-    for (int q = 0; q < (1 << D); ++q) {
-        int64_t o = 0, stride = 1;
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            o += (idx[d] + ((q >> d) & 1)) * stride;
-            stride *= nn[d];
-        }
-        v[q] = F[o];
-    }
-#pragma unroll
-    for (int d = 0; d < D; ++d) t[d] = (p[d] - x0[d]) * inv[d];
-    double r = lerp1(t[1], lerp1(t[0], v[0], v[1]), lerp1(t[0], v[2], v[3]));
-    if constexpr (D == 3)
-        r = lerp1(t[2], r, lerp1(t[1], lerp1(t[0], v[4], v[5]), lerp1(t[0], v[6], v[7])));
-    double lo = v[0], hi = v[0];
-#pragma unroll
-    for (int q = 1; q < (1 << D); ++q) {
-        lo = jl_min(lo, v[q]);
-        hi = jl_max(hi, v[q]);
-    }
-    return r > hi ? hi : (r < lo ? lo : r);
-}
-
-template <int D, bool PHASE = false>
-__global__ void __launch_bounds__(kBlock) k_inject_wave(Grid<D> g, Ptr3 coords, uint8_t* index,
-                                                        int nargs, ArgPtrs args, int min_q,
-                                                        uint64_t seed, uint64_t counter,
-                                                        const int32_t* __restrict__ list,
-                                                        const int32_t* __restrict__ count,
-                                                        jp_stats* st, PhaseInj pi) {
-    const int lane = threadIdx.x & 63;
-    // persistent wavefronts over the colour's list (every wavefront exits once
-    // the list is exhausted)
-    const int64_t nwv = (int64_t)gridDim.x * (kBlock / 64);
-    const int64_t total = *count;
-    int64_t n_inj = 0, n_orph = 0;
-    for (int64_t w = blockIdx.x * (int64_t)(kBlock / 64) + (threadIdx.x >> 6); w < total;
-         w += nwv) {
-    const int64_t c = list[w];
-    const int64_t C = g.C;
-    const int K = g.K;
-    const uint64_t full = K == 64 ? ~0ull : ((1ull << K) - 1);
-    int64_t I[D];
-    unlin<D>(g.ni, c, I);
-    constexpr int NQ = D == 2 ? 4 : 8;
-    constexpr int NB = D == 2 ? 9 : 27;
-    constexpr int CENTER = (NB - 1) / 2;
-    double xv[D], dq[D];
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-        xv[d] = g.xv[d].x[I[d]];
-        dq[d] = g.xv[d].dx[I[d]] / 2.0;
-    }
-    // this cell's slots, one per lane, kept current in registers
-    const bool own = lane < K;
-    const int64_t e = c + C * lane;
-    bool act = own && index[e];
-    double p[D];
-#pragma unroll
-    for (int d = 0; d < D; ++d) p[d] = act ? coords.p[d][e] : 0.0;
-    // 2D: the neighbour cells' masks and coordinates, loaded once for all of
-    // this cell's searches (they do not change while it injects: the cells
-    // of one colour are two apart); 3D loads them per search, in batches
-    uint8_t m9[D == 2 ? NB : 1];
-    double q9[D == 2 ? NB : 1][D];
-    if constexpr (D == 2) {
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-            int64_t J[D];
-            bool ok = own && u != CENTER;
-            int r = u;
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                J[d] = I[d] + (r % 3) - 1;
-                r /= 3;
-                ok = ok && J[d] >= 0 && J[d] < g.ni[d];
-            }
-            const int64_t e2 = ok ? lin<D>(g.ni, J) + C * lane : 0;
-            m9[u] = ok ? index[e2] : (uint8_t)0;
-#pragma unroll
-            for (int d = 0; d < D; ++d) q9[u][d] = ok ? coords.p[d][e2] : 0.0;
-        }
-    }
-    for (int q = 0; q < NQ; ++q) {
-        double vert[D];
-#pragma unroll
-        for (int d = 0; d < D; ++d) vert[d] = xv[d] + dq[d] * (double)((q >> d) & 1);
-        bool inside = act;
-#pragma unroll
-        for (int d = 0; d < D; ++d) inside = inside & (vert[d] < p[d] && p[d] < vert[d] + dq[d]);
-        int num = __popcll(__ballot(inside));
-        if (num >= min_q) {
-            if constexpr (PHASE) continue;
-            break;
-        }
-        uint64_t freeS = ~__ballot(act) & full;
-        bool done = false;
-        while (freeS) {
-            const int ip = __builtin_ctzll(freeS);
-            freeS &= freeS - 1;
-            ++num;
-            double pn[D];
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                const double r = uniform53(seed, (uint64_t)c, ip, d, 2, counter);
-                pn[d] = vert[d] + dq[d] * fma(0.95, r, 0.05);
-            }
-            const int64_t enew = c + C * ip;
-            if (lane == ip) {
-                act = true;
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    p[d] = pn[d];
-                    coords.p[d][enew] = pn[d];
-                }
-                index[enew] = 1;
-            }
-            // index_min_distance over the 3^D neighbourhood
-            double best = __builtin_inf();
-            int border = 0x7fffffff;
-            constexpr int NBB = 9;  // neighbour cells per batch: masks, then coordinates
-#pragma unroll
-            for (int nb0 = 0; nb0 < NB; nb0 += NBB) {
-                bool a[NBB];
-                int64_t e2[NBB];
-#pragma unroll
-                for (int u = 0; u < NBB; ++u) {
-                    const int nb = nb0 + u;
-                    int64_t J[D];
-                    bool ok = own;
-                    int r = nb;
-#pragma unroll
-                    for (int d = 0; d < D; ++d) {
-                        J[d] = I[d] + (r % 3) - 1;
-                        r /= 3;
-                        ok = ok && J[d] >= 0 && J[d] < g.ni[d];
-                    }
-                    e2[u] = ok ? lin<D>(g.ni, J) + C * lane : 0;
-                    a[u] = ok;
-                }
-                // masks and coordinates of the batch in one round of loads
-                // (an empty slot holds NaN coordinates and is masked out below)
-                uint8_t m[NBB];
-                double pq[NBB][D];
-#pragma unroll
-                for (int u = 0; u < NBB; ++u) {
-                    const bool other = a[u] && nb0 + u != CENTER;
-                    if constexpr (D == 2) {
-                        m[u] = other ? m9[nb0 + u] : (uint8_t)0;
-#pragma unroll
-                        for (int d = 0; d < D; ++d) pq[u][d] = other ? q9[nb0 + u][d] : p[d];
-                    } else {
-                        m[u] = other ? index[e2[u]] : (uint8_t)0;
-#pragma unroll
-                        for (int d = 0; d < D; ++d)
-                            pq[u][d] = other ? coords.p[d][e2[u]] : p[d];
-                    }
-                }
-#pragma unroll
-                for (int u = 0; u < NBB; ++u)
-                    a[u] = (nb0 + u == CENTER) ? (act && lane != ip) : (m[u] != 0);
-#pragma unroll
-                for (int u = 0; u < NBB; ++u) {
-                    if (!a[u]) continue;
-                    bool hasnan = false;
-#pragma unroll
-                    for (int d = 0; d < D; ++d) hasnan = hasnan || (pq[u][d] != pq[u][d]);
-                    if (D == 2 && hasnan) continue;
-                    double du = pq[u][0] - pn[0];
-                    double s = du * du;
-#pragma unroll
-                    for (int d = 1; d < D; ++d) {
-                        double dv = pq[u][d] - pn[d];
-                        s = s + dv * dv;
-                    }
-                    const double dd = sqrt(s);
-                    if (dd < best) {
-                        best = dd;
-                        border = (nb0 + u) * 64 + lane;
-                    }
-                }
-            }
-#pragma unroll
-            for (int m = 32; m >= 1; m >>= 1) {
-                const double ob = __shfl_xor(best, m, 64);
-                const int oo = __shfl_xor(border, m, 64);
-                if (ob < best || (ob == best && oo < border)) {
-                    best = ob;
-                    border = oo;
-                }
-            }
-            if (border == 0x7fffffff) ++n_orph;
-            if (lane == ip && border != 0x7fffffff) {
-                int64_t J[D];
-                int r = border >> 6;
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    J[d] = I[d] + (r % 3) - 1;
-                    r /= 3;
-                }
-                const int64_t esrc = lin<D>(g.ni, J) + C * (border & 63);
-                if constexpr (PHASE)
-                    pi.phases[enew] = pi.phases[esrc];
-                else
-                    for (int a = 0; a < nargs; ++a) args.p[a][enew] = args.p[a][esrc];
-            }
-            if constexpr (PHASE) {
-                if (lane == ip) {
-                    // args from fields: nodal at this cell's corners, cell-centred at
-                    // the shifted index clamped to 1..ni-1 (1-based)
-                    int64_t nnv[D], nnc[D], ic[D], Iv[D];
-                    double xc0[D], ivc[D], xv0[D], ivv[D];
-#pragma unroll
-                    for (int d = 0; d < D; ++d) {
-                        nnv[d] = g.ni[d] + 1;
-                        nnc[d] = g.ni[d];
-                        Iv[d] = I[d];
-                        xv0[d] = xv[d];
-                        ivv[d] = g.xv[d].idx[I[d]];
-                        int64_t k = pn[d] < xv[d] + dq[d] ? I[d] - 1 : I[d];
-                        k = k > g.ni[d] - 2 ? g.ni[d] - 2 : (k < 0 ? 0 : k);
-                        ic[d] = k;
-                        xc0[d] = pi.xc[d].x[k];
-                        ivc[d] = pi.xc[d].idx[k];
-                    }
-                    for (int a = 0; a < nargs; ++a)
-                        args.p[a][enew] = ((pi.centred >> a) & 1)
-                                              ? g2p_clamped<D>(pi.fields[a], nnc, ic, pn, xc0, ivc)
-                                              : g2p_clamped<D>(pi.fields[a], nnv, Iv, pn, xv0, ivv);
-                }
-            }
-            // later searches of this wavefront read what lane ip just wrote
-            __threadfence_block();
-            ++n_inj;
-            if (num >= min_q) {
-                done = true;
-                break;
-            }
-        }
-        (void)done;
-    }
-    }  // work list
-    if (lane == 0) {
-        stat_add(st, ST_INJECTED, n_inj);
-        stat_add(st, ST_ORPHAN, n_orph);
-    }
 }
 
 // ============================================================ host side
@@ -848,6 +549,23 @@ int run_g2p(jp_ctx* ctx, const jp_cellgrid* g, double* Fp, const double* F,
 }
 
 template <int D>
+InjectCells<D> inject_cells(const Grid<D>& G, double* const* coords, uint8_t* index, int nargs,
+                            double* const* args, int min_q, uint64_t seed, uint64_t counter,
+                            jp_stats* st) {
+    InjectCells<D> a{};
+    a.g = G;
+    for (int d = 0; d < D; ++d) a.x[d] = coords[d];
+    a.index = index;
+    a.nargs = nargs;
+    a.args = argptrs(args, nargs);
+    a.min_q = min_q;
+    a.seed = seed;
+    a.counter = counter;
+    a.st = st;
+    return a;
+}
+
+template <int D>
 int run_inject(jp_ctx* ctx, const jp_cellgrid* gc, double* const* coords, uint8_t* index,
                int nargs, double* const* args, int min_xcell, uint64_t seed, uint64_t counter,
                jp_stats* stats) {
@@ -860,16 +578,13 @@ int run_inject(jp_ctx* ctx, const jp_cellgrid* gc, double* const* coords, uint8_
     int64_t cap = 1;
     for (int d = 0; d < D; ++d) cap *= (G.ni[d] + 1) / 2;
     InjectLists L;
-    if ((rc = inject_lists(ctx, G.C, NQ, cap, 0, L))) return rc;
     const bool two = D == 2 && nargs <= 1;  // the 2D kernel (k_inject2)
     const bool ordered = two && inject2_ordered(ctx);
-    if (!ordered) L.state = nullptr;
+    if ((rc = inject_lists(ctx, G.C, NQ, cap, ordered, L))) return rc;
     k_inject_scan<D><<<blocks_for(G.C), kBlock, 0, ctx->stream>>>(G, cptr3(coords, D), index,
                                                                   min_q, L);
     JP_LAUNCHED(ctx);
     if ((rc = join_segments(ctx, NQ, L))) return rc;
-    Ptr3 cp = ptr3(coords, D);
-    ArgPtrs ap = argptrs(args, nargs);
     jp_stats* st = stats ? dstats(ctx) : nullptr;
     if constexpr (D == 2) {
         if (two) {
@@ -887,13 +602,9 @@ int run_inject(jp_ctx* ctx, const jp_cellgrid* gc, double* const* coords, uint8_
             if ((rc = launch_inject2<false>(ctx, a, L, cap))) return rc;
         }
     }
-    // colour index of a phase: offsets (o_1 outer ... o_D inner); persistent
-    // wavefronts, one listed cell at a time each
-    for (int ph = 0; ph < NQ && !two; ++ph) {
-        k_inject_wave<D><<<(unsigned)inject_blocks(ctx, cap), kBlock, 0, ctx->stream>>>(
-            G, cp, index, nargs, ap, min_q, seed, counter, L.list + (int64_t)ph * cap,
-            L.total + ph, st, PhaseInj{});
-        JP_LAUNCHED(ctx);
+    if (!two) {
+        InjectCells<D> a = inject_cells<D>(G, coords, index, nargs, args, min_q, seed, counter, st);
+        if ((rc = launch_inject_cells<D, false, false>(ctx, a, L, cap))) return rc;
     }
     if ((rc = stats_end(ctx, stats))) return rc;
     if (ordered && stats && (rc = inject_wait_report(ctx))) return rc;
@@ -915,26 +626,18 @@ int run_inject_phase(jp_ctx* ctx, const jp_cellgrid* gc, const jp_axis* xc,
     int64_t cap = 1;
     for (int d = 0; d < D; ++d) cap *= (G.ni[d] + 1) / 2;
     InjectLists L;
-    if ((rc = inject_lists(ctx, G.C, NQ, cap, 0, L))) return rc;
-    L.state = nullptr;  // colour launches only
+    if ((rc = inject_lists(ctx, G.C, NQ, cap, false, L))) return rc;
     k_inject_scan<D, true><<<blocks_for(G.C), kBlock, 0, ctx->stream>>>(G, cptr3(coords, D),
                                                                         index, min_q, L);
     JP_LAUNCHED(ctx);
     if ((rc = join_segments(ctx, NQ, L))) return rc;
-    PhaseInj pi{};
-    pi.phases = phases;
-    pi.centred = centred;
-    for (int a = 0; a < nargs; ++a) pi.fields[a] = fields[a];
-    for (int d = 0; d < D; ++d) pi.xc[d] = Axis{xc[d].x, xc[d].dx, xc[d].inv_dx, xc[d].n};
-    Ptr3 cp = ptr3(coords, D);
-    ArgPtrs ap = argptrs(args, nargs);
-    jp_stats* st = stats ? dstats(ctx) : nullptr;
-    for (int ph = 0; ph < NQ; ++ph) {
-        k_inject_wave<D, true><<<(unsigned)inject_blocks(ctx, cap), kBlock, 0, ctx->stream>>>(
-            G, cp, index, nargs, ap, min_q, seed, counter, L.list + (int64_t)ph * cap,
-            L.total + ph, st, pi);
-        JP_LAUNCHED(ctx);
-    }
+    InjectCells<D> a = inject_cells<D>(G, coords, index, nargs, args, min_q, seed, counter,
+                                       stats ? dstats(ctx) : nullptr);
+    a.pi.phases = phases;
+    a.pi.centred = centred;
+    for (int f = 0; f < nargs; ++f) a.pi.fields[f] = fields[f];
+    for (int d = 0; d < D; ++d) a.pi.xc[d] = Axis{xc[d].x, xc[d].dx, xc[d].inv_dx, xc[d].n};
+    if ((rc = launch_inject_cells<D, false, true>(ctx, a, L, cap))) return rc;
     if ((rc = stats_end(ctx, stats))) return rc;
     return finish(ctx);
 }

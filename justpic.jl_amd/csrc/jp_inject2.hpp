@@ -53,7 +53,6 @@ struct Inject2 {
     Grid<2> g;
     double* x[2];      // FP64 form: coordinates
     float* u[2];       // split form: offsets in cell units
-    double h[2];       // split form: uniform vertex spacing
     uint8_t* index;
     double* arg;       // the field moved with the particles, or null
     int min_q;         // particles wanted per quadrant
@@ -142,6 +141,8 @@ __global__ void __launch_bounds__(kBlock) k_inject2(Inject2 a) {
     const uint64_t full = K == 64 ? ~0ull : ((1ull << K) - 1);
     const bool slot = lane < K;
     const bool has_arg = a.arg != nullptr;
+    // split form: the uniform vertex spacing
+    const double h[2] = {SPLIT ? g.xv[0].dx[0] : 0.0, SPLIT ? g.xv[1].dx[0] : 0.0};
     int64_t n_inj = 0, n_orph = 0;
     for (int64_t w = blockIdx.x * (int64_t)(kBlock / 64) + (threadIdx.x >> 6); w < total;
          w += nwv) {
@@ -317,9 +318,9 @@ __global__ void __launch_bounds__(kBlock) k_inject2(Inject2 a) {
                 double sq;
                 if constexpr (SPLIT) {
                     const double r0 =
-                        ((double)(nb % 3 - 1) + (double)q[nb][0] - (double)pn[0]) * a.h[0];
+                        ((double)(nb % 3 - 1) + (double)q[nb][0] - (double)pn[0]) * h[0];
                     const double r1 =
-                        ((double)(nb / 3 - 1) + (double)q[nb][1] - (double)pn[1]) * a.h[1];
+                        ((double)(nb / 3 - 1) + (double)q[nb][1] - (double)pn[1]) * h[1];
                     sq = r0 * r0 + r1 * r1;
                 } else {
                     if (q[nb][0] != q[nb][0] || q[nb][1] != q[nb][1]) continue;  // 2D NaN skip

@@ -11,6 +11,7 @@
 // (README.md:42-44).
 #include "jp_ctx.hpp"
 #include "jp_inject2.hpp"
+#include "jp_inject_cells.hpp"
 #include "jp_splitmath.hpp"
 
 #include <algorithm>
@@ -538,12 +539,7 @@ __global__ void __launch_bounds__(kBlock) k_inj_scan_split(Grid<D> g, FPtr3 off,
     int num = 0;
     if (valid) {
         const uint64_t act = active_slots(index, c, g.C, g.K);
-        float bl[D], bh[D];  // box of the cell's offsets
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            bl[d] = __builtin_inff();
-            bh[d] = -__builtin_inff();
-        }
+        bool out = false;  // an offset outside the cell (or NaN)
         constexpr int B = 16;
         for (int k0 = 0; k0 < g.K; k0 += B) {
             float ub[B][D];
@@ -560,23 +556,13 @@ __global__ void __launch_bounds__(kBlock) k_inj_scan_split(Grid<D> g, FPtr3 off,
 #pragma unroll
                 for (int d = 0; d < D; ++d) {
                     inside = inside & (0.0f < ub[j][d] && ub[j][d] < 0.5f);
-                    if (D == 2 && on) {
-                        bl[d] = fminf(bl[d], ub[j][d]);
-                        bh[d] = fmaxf(bh[d], ub[j][d]);
-                    }
+                    out = out || (on && !(0.0f <= ub[j][d] && ub[j][d] <= 1.0f));
                 }
                 num += inside ? 1 : 0;
             }
         }
         L.occ[c] = act;
-        if (D == 2 && L.box) {
-            float* __restrict__ bx = static_cast<float*>(L.box);
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                bx[(2 * d) * g.C + c] = bl[d];
-                bx[(2 * d + 1) * g.C + c] = bh[d];
-            }
-        }
+        if (L.out) L.out[c] = out ? 1u : 0u;
     }
     if (valid && L.state) L.state[c] = num < min_q ? 1u : 0u;
     int col = 0;
@@ -584,151 +570,6 @@ __global__ void __launch_bounds__(kBlock) k_inj_scan_split(Grid<D> g, FPtr3 off,
     for (int d = 0; d < D; ++d) col = col * 2 + (int)(I[d] & 1);
     wave_segment<D == 2 ? 4 : 8>(valid && num < min_q, col, (int32_t)c, c >> 6, L.nwave, L.seg,
                                  L.cnt);
-}
-
-template <int D>
-__global__ void __launch_bounds__(kBlock) k_inj_wave_split(Grid<D> g, SGrid<D> sg, FPtr3 off,
-                                                           uint8_t* index, int nargs, ArgPtrs args,
-                                                           int min_q, uint64_t seed,
-                                                           uint64_t counter,
-                                                           const int32_t* __restrict__ list,
-                                                           const int32_t* __restrict__ count,
-                                                           jp_stats* st) {
-    const int lane = threadIdx.x & 63;
-    // persistent wavefronts over the colour's list (every wavefront exits once
-    // the list is exhausted)
-    const int64_t nwv = (int64_t)gridDim.x * (kBlock / 64);
-    const int64_t total = *count;
-    int64_t n_inj = 0, n_orph = 0;
-    for (int64_t w = blockIdx.x * (int64_t)(kBlock / 64) + (threadIdx.x >> 6); w < total;
-         w += nwv) {
-    const int64_t c = list[w];
-    const int64_t C = g.C;
-    const int K = g.K;
-    const uint64_t full = K == 64 ? ~0ull : ((1ull << K) - 1);
-    int64_t I[D];
-    unlin<D>(g.ni, c, I);
-    constexpr int NQ = D == 2 ? 4 : 8;
-    constexpr int NB = D == 2 ? 9 : 27;
-    constexpr int CENTER = (NB - 1) / 2;
-    const bool own = lane < K;
-    const int64_t e = c + C * lane;
-    bool act = own && index[e];
-    float u[D];
-#pragma unroll
-    for (int d = 0; d < D; ++d) u[d] = act ? off.p[d][e] : 0.0f;
-    for (int q = 0; q < NQ; ++q) {
-        float q0[D];
-#pragma unroll
-        for (int d = 0; d < D; ++d) q0[d] = 0.5f * (float)((q >> d) & 1);
-        bool inside = act;
-#pragma unroll
-        for (int d = 0; d < D; ++d) inside = inside & (q0[d] < u[d] && u[d] < q0[d] + 0.5f);
-        int num = __popcll(__ballot(inside));
-        if (num >= min_q) break;
-        uint64_t freeS = ~__ballot(act) & full;
-        while (freeS) {
-            const int ip = __builtin_ctzll(freeS);
-            freeS &= freeS - 1;
-            ++num;
-            float un[D];
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                const double r = uniform53(seed, (uint64_t)c, ip, d, 2, counter);
-                un[d] = (float)((double)q0[d] + 0.5 * fma(0.95, r, 0.05));
-            }
-            const int64_t enew = c + C * ip;
-            if (lane == ip) {
-                act = true;
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    u[d] = un[d];
-                    off.p[d][enew] = un[d];
-                }
-                index[enew] = 1;
-            }
-            double best = __builtin_inf();
-            int border = 0x7fffffff;
-            constexpr int NBB = 9;  // neighbour cells per batch, one round of loads each
-#pragma unroll
-            for (int nb0 = 0; nb0 < NB; nb0 += NBB) {
-                bool a[NBB];
-                int64_t e2[NBB];
-                int o[NBB][D];
-#pragma unroll
-                for (int v = 0; v < NBB; ++v) {
-                    int64_t J[D];
-                    bool ok = own;
-                    int r = nb0 + v;
-#pragma unroll
-                    for (int d = 0; d < D; ++d) {
-                        o[v][d] = (r % 3) - 1;
-                        J[d] = I[d] + o[v][d];
-                        r /= 3;
-                        ok = ok && J[d] >= 0 && J[d] < g.ni[d];
-                    }
-                    e2[v] = ok ? lin<D>(g.ni, J) + C * lane : 0;
-                    a[v] = ok;
-                }
-                uint8_t m[NBB];
-                float uq[NBB][D];
-#pragma unroll
-                for (int v = 0; v < NBB; ++v) {
-                    const bool other = a[v] && nb0 + v != CENTER;
-                    m[v] = other ? index[e2[v]] : (uint8_t)0;
-#pragma unroll
-                    for (int d = 0; d < D; ++d) uq[v][d] = other ? off.p[d][e2[v]] : u[d];
-                }
-#pragma unroll
-                for (int v = 0; v < NBB; ++v) {
-                    const bool av = (nb0 + v == CENTER) ? (act && lane != ip) : (m[v] != 0);
-                    if (!av) continue;
-                    double s2 = 0.0;
-#pragma unroll
-                    for (int d = 0; d < D; ++d) {
-                        const double r2 =
-                            ((double)o[v][d] + (double)uq[v][d] - (double)un[d]) * sg.h[d][0];
-                        s2 = s2 + r2 * r2;
-                    }
-                    const double dd = sqrt(s2);
-                    if (dd < best) {
-                        best = dd;
-                        border = (nb0 + v) * 64 + lane;
-                    }
-                }
-            }
-#pragma unroll
-            for (int m = 32; m >= 1; m >>= 1) {
-                const double ob = __shfl_xor(best, m, 64);
-                const int oo = __shfl_xor(border, m, 64);
-                if (ob < best || (ob == best && oo < border)) {
-                    best = ob;
-                    border = oo;
-                }
-            }
-            if (border == 0x7fffffff) {
-                ++n_orph;
-            } else if (lane == ip) {
-                int64_t J[D];
-                int r = border >> 6;
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    J[d] = I[d] + (r % 3) - 1;
-                    r /= 3;
-                }
-                const int64_t esrc = lin<D>(g.ni, J) + C * (border & 63);
-                for (int a = 0; a < nargs; ++a) args.p[a][enew] = args.p[a][esrc];
-            }
-            __threadfence_block();
-            ++n_inj;
-            if (num >= min_q) break;
-        }
-    }
-    }  // work list
-    if (lane == 0) {
-        stat_add(st, ST_INJECTED, n_inj);
-        stat_add(st, ST_ORPHAN, n_orph);
-    }
 }
 
 // ------------------------------------------------------------ host side
@@ -1010,7 +851,6 @@ int run_inject(jp_ctx* ctx, const jp_cellgrid* gc, float* const* off, uint8_t* i
                double* const* args, int min_xcell, uint64_t seed, uint64_t counter,
                jp_stats* stats) {
     Grid<D> G = to_grid<D>(gc);
-    SGrid<D> sg = sgrid<D>(G);
     int rc;
     if ((rc = stats_begin(ctx, stats))) return rc;
     constexpr int NQ = D == 2 ? 4 : 8;
@@ -1018,18 +858,15 @@ int run_inject(jp_ctx* ctx, const jp_cellgrid* gc, float* const* off, uint8_t* i
     int64_t cap = 1;
     for (int d = 0; d < D; ++d) cap *= (G.ni[d] + 1) / 2;
     InjectLists L;
-    if ((rc = inject_lists(ctx, G.C, NQ, cap, 0, L))) return rc;
     const bool two = D == 2 && nargs <= 1;  // the 2D kernel (k_inject2)
     const bool ordered = two && inject2_ordered(ctx);
-    if (!ordered) L.state = nullptr;
+    if ((rc = inject_lists(ctx, G.C, NQ, cap, ordered, L))) return rc;
     FPtr3 fp = fptr3<D>(off);
     if ((rc = split_geometry(ctx, gc, nullptr))) return rc;
     k_inj_scan_split<D><<<blocks_for(G.C), kBlock, 0, ctx->stream>>>(G, fp, index, min_q, L,
                                                                      geo_ptr(ctx));
     JP_LAUNCHED(ctx);
     if ((rc = join_segments(ctx, NQ, L))) return rc;
-    ArgPtrs ap;
-    for (int i = 0; i < JP_MAX_ARGS; ++i) ap.p[i] = i < nargs ? args[i] : nullptr;
     jp_stats* st = stats ? dstats(ctx) : nullptr;
     if constexpr (D == 2) {
         if (two) {
@@ -1037,8 +874,6 @@ int run_inject(jp_ctx* ctx, const jp_cellgrid* gc, float* const* off, uint8_t* i
             a.g = G;
             a.u[0] = off[0];
             a.u[1] = off[1];
-            a.h[0] = sg.h[0][0];
-            a.h[1] = sg.h[1][0];
             a.index = index;
             a.arg = nargs ? args[0] : nullptr;
             a.min_q = min_q;
@@ -1049,11 +884,18 @@ int run_inject(jp_ctx* ctx, const jp_cellgrid* gc, float* const* off, uint8_t* i
             if ((rc = launch_inject2<true>(ctx, a, L, cap))) return rc;
         }
     }
-    for (int ph = 0; ph < NQ && !two; ++ph) {
-        k_inj_wave_split<D><<<(unsigned)inject_blocks(ctx, cap), kBlock, 0, ctx->stream>>>(
-            G, sg, fp, index, nargs, ap, min_q, seed, counter, L.list + (int64_t)ph * cap,
-            L.total + ph, st);
-        JP_LAUNCHED(ctx);
+    if (!two) {
+        InjectCells<D> a{};
+        a.g = G;
+        for (int d = 0; d < D; ++d) a.u[d] = off[d];
+        a.index = index;
+        a.nargs = nargs;
+        for (int i = 0; i < JP_MAX_ARGS; ++i) a.args.p[i] = i < nargs ? args[i] : nullptr;
+        a.min_q = min_q;
+        a.seed = seed;
+        a.counter = counter;
+        a.st = st;
+        if ((rc = launch_inject_cells<D, true, false>(ctx, a, L, cap))) return rc;
     }
     if ((rc = stats_end(ctx, stats))) return rc;
     if (ordered && stats && (rc = inject_wait_report(ctx))) return rc;
