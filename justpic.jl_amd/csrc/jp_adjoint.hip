@@ -24,10 +24,10 @@
 //  - k_adj_bwd: blocks of steps in reverse order; a block is recomputed from
 //    its checkpoint into a tape (the position at the start of each step, in
 //    global scratch), then reversed step by step.  x0bar and Tpbar are per-thread
-//    values.  In 2D the velocity cotangent of a workgroup and block of steps
-//    is accumulated in an LDS tile covering exactly the nodes the recompute
-//    touched (LDS atomic adds), then added to Vbar once; when that footprint
-//    exceeds the tile, and in 3D, it goes to Vbar with FP64 atomic adds.
+//    values.
+// In 2D both trajectory kernels read the velocities and axes of a workgroup's
+// block of steps from a window in LDS, and the pullback sums its velocity
+// cotangents there (LDS atomic adds) before it adds them to Vbar once; see Window.
 // The adjoint is the exact derivative of the forward model on the branch the
 // forward pass takes (brackets, cells and survivors fixed): the n-linear
 // interpolation's weights and slopes, the integrator's stage weights, and for
@@ -42,8 +42,6 @@
 using namespace jp;
 
 namespace {
-
-constexpr int kAdjBlock = 512;  // backward workgroup: one 64-cell patch, 8 slot planes
 
 template <int D>
 struct AdjArgs {
@@ -79,48 +77,46 @@ __device__ inline bool in_limits(const Vel<D>& vg, int c, const double (&p)[D]) 
     return true;
 }
 
+// The velocity window of a workgroup and block of steps (2D): component c's nodes
+// lo[c] .. lo[c] + ext[c] - 1 per dimension.  In LDS lie the cotangent tile (the
+// components one after the other, c's at off[c]; `tiled`), and, where that fits as
+// well (`staged`), the velocities in the same order at `vo` and each axis's x and
+// idx at ax[c][d] and ax[c][d] + ext[c][d].  Points outside the window, and all
+// points of a footprint too large for it, take global loads and global FP64
+// atomic adds.
+// Particles of a patch disperse over a block (64 lanes from 4 to 28 cache lines of
+// velocities in 100 steps), and every one of those lines is a cycle of the CU's
+// address unit for each of the 16 loads of a velocity: 1 M particles, 100 RK2
+// steps, checkpoints every 10: pullback 7.18 ms and forward 1.64 ms with global
+// loads, 3.20 and 1.07 with windows (1200 and 200 cycles per CU, wavefront and
+// step, most of them the LDS's: its 48 loads and 16 adds of a reversed step).
+// (The array is named, not pointed to: a pointer that may be null makes the adds
+// flat ones, 7.61 ms for 7.18.)
+extern __shared__ double adj_lds[];
+
+template <int D>
+struct Window {
+    double* g[D];  // Vbar
+    bool staged, tiled;
+    int vo;
+    int lo[D][D], ext[D][D], off[D], ax[D][D];
+    double x0[D][D], i0[D][D];  // x[0] and idx[0] of every axis
+};
+
+// lower corner, values, local coordinates and inverse spacings of a point's
+// interval in component c
 template <int D>
 struct Corners {
-    int64_t at[1 << D];
+    int64_t at;  // lower corner: index in the tile (in) or in the component's array
     double v[1 << D];
     double t[D];
     double iv[D];
-    int64_t k[D];  // bracket (lower corner node) per dimension
+    bool in;     // the corners lie in the tile
 };
 
-// bracket observers of gather: NoTrack, or BoxTrack (per component and
-// dimension, the range of lower-corner nodes seen)
-struct NoTrack {
-    template <int D>
-    __device__ void operator()(int, const int64_t (&)[D]) const {}
-};
 template <int D>
-struct BoxTrack {
-    int lo[D][D], hi[D][D];
-    __device__ BoxTrack() {
-#pragma unroll
-        for (int c = 0; c < D; ++c)
-#pragma unroll
-            for (int d = 0; d < D; ++d) {
-                lo[c][d] = 0x7fffffff;
-                hi[c][d] = -1;
-            }
-    }
-    __device__ void operator()(int c, const int64_t (&k)[D]) {
-#pragma unroll
-        for (int cc = 0; cc < D; ++cc)
-            if (cc == c)
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    lo[cc][d] = min(lo[cc][d], (int)k[d]);
-                    hi[cc][d] = max(hi[cc][d], (int)k[d]);
-                }
-    }
-};
-
-template <int D, class Tr>
-__device__ inline void gather(const AdjArgs<D>& A, int c, const double (&p)[D], Corners<D>& K,
-                              Tr& tr) {
+__device__ inline void gather_global(const AdjArgs<D>& A, const Window<D>& Wn, int c,
+                                     const double (&p)[D], Corners<D>& K) {
     int64_t k[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) {
@@ -128,18 +124,89 @@ __device__ inline void gather(const AdjArgs<D>& A, int c, const double (&p)[D], 
         k[d] = adj_bracket(p[d], X);
         K.iv[d] = X.idx[k[d]];
         K.t[d] = (p[d] - X.x[k[d]]) * K.iv[d];
-        K.k[d] = k[d];
     }
-    tr(c, k);
     const int64_t n0 = A.vg.ax[c][0].n, n1 = A.vg.ax[c][1].n;
     const double* __restrict__ Vc = A.V[c];
+    K.at = k[0] + n0 * (k[1] + n1 * (D == 3 ? k[D - 1] : 0));
 #pragma unroll
-    for (int q = 0; q < (1 << D); ++q) {
-        const int64_t a = k[0] + (q & 1), b = k[1] + ((q >> 1) & 1);
-        const int64_t e = D == 3 ? k[D - 1] + ((q >> 2) & 1) : 0;
-        K.at[q] = a + n0 * (b + n1 * e);
-        K.v[q] = Vc[K.at[q]];
+    for (int q = 0; q < (1 << D); ++q)
+        K.v[q] = Vc[K.at + (q & 1) + n0 * (((q >> 1) & 1) + n1 * ((q >> 2) & 1))];
+    K.in = false;
+    if constexpr (D == 2) {
+        if (Wn.tiled) {
+            const unsigned a = (unsigned)((int)k[0] - Wn.lo[c][0]);
+            const unsigned b = (unsigned)((int)k[1] - Wn.lo[c][1]);
+            if (a < (unsigned)(Wn.ext[c][0] - 1) && b < (unsigned)(Wn.ext[c][1] - 1)) {
+                K.in = true;
+                K.at = Wn.off[c] + (int)a + Wn.ext[c][0] * (int)b;
+            }
+        }
     }
+}
+
+// corners of interval s of the window; true when p lies strictly inside it
+__device__ inline bool gather_window(const Window<2>& Wn, int c, const double (&p)[2],
+                                     const int (&s)[2], Corners<2>& K) {
+    bool ok = true;
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+        const double* __restrict__ x = adj_lds + Wn.ax[c][d] + s[d];
+        const double xa = x[0], xb = x[1];
+        K.iv[d] = x[Wn.ext[c][d]];
+        K.t[d] = (p[d] - xa) * K.iv[d];
+        ok = ok && xa < p[d] && p[d] < xb;
+    }
+    const int e0 = Wn.ext[c][0], at = Wn.off[c] + s[0] + e0 * s[1];
+    const double* __restrict__ v = adj_lds + Wn.vo + at;
+    K.v[0] = v[0];
+    K.v[1] = v[1];
+    K.v[2] = v[e0];
+    K.v[3] = v[e0 + 1];
+    K.at = at;
+    K.in = true;
+    return ok;
+}
+
+// interval of p among the n nodes x of a window axis (its last one or its first
+// where p lies outside)
+__device__ inline int window_search(const double* __restrict__ x, int n, double p) {
+    int a = 0, b = n - 1;
+    while (b - a > 1) {
+        const int m = (a + b) >> 1;
+        if (x[m] <= p)
+            a = m;
+        else
+            b = m;
+    }
+    return a;
+}
+
+// corners of p in component c.  In the window the interval is the one at the
+// uniform spacing's estimate when p lies strictly inside it, as in adj_bracket,
+// else the one a bisection finds.  True for a point strictly inside the window.
+template <int D>
+__device__ inline bool gather(const AdjArgs<D>& A, const Window<D>& Wn, int c,
+                              const double (&p)[D], Corners<D>& K) {
+    bool found = false;
+    if constexpr (D == 2) {
+        if (Wn.staged) {
+            int s[2];
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {
+                const int e = (int)((p[d] - Wn.x0[c][d]) * Wn.i0[c][d]) - Wn.lo[c][d];
+                s[d] = max(0, min(e, Wn.ext[c][d] - 2));
+            }
+            found = gather_window(Wn, c, p, s, K);
+            if (!found) {
+#pragma unroll
+                for (int d = 0; d < 2; ++d)
+                    s[d] = window_search(adj_lds + Wn.ax[c][d], Wn.ext[c][d], p[d]);
+                found = gather_window(Wn, c, p, s, K);
+            }
+        }
+    }
+    if (!found) gather_global(A, Wn, c, p, K);
+    return found;
 }
 
 // lerp(v, t) of src/Interpolations/ndlerp.jl:11-15
@@ -158,51 +225,30 @@ __device__ inline double lerp_n(const Corners<D>& K) {
 
 // velocity component c at p; +Inf outside its grid (check_local_limits,
 // src/Advection/advection.jl:83-91)
-template <int D, class Tr>
-__device__ inline double vel_c(const AdjArgs<D>& A, int c, const double (&p)[D], Tr& tr) {
-    if (!in_limits(A.vg, c, p)) return __builtin_inf();
-    Corners<D> K;
-    gather(A, c, p, K, tr);
-    return lerp_n(K);
+template <int D>
+__device__ inline double vel_c(const AdjArgs<D>& A, const Window<D>& Wn, int c,
+                               const double (&p)[D], Corners<D>& K) {
+    const bool inside = gather(A, Wn, c, p, K);
+    return inside || in_limits(A.vg, c, p) ? lerp_n(K) : __builtin_inf();
 }
 
-template <int D, class Tr>
-__device__ inline void vel(const AdjArgs<D>& A, const double (&p)[D], double (&v)[D], Tr& tr) {
+template <int D>
+__device__ inline void vel(const AdjArgs<D>& A, const Window<D>& Wn, const double (&p)[D],
+                           double (&v)[D]) {
 #pragma unroll
-    for (int c = 0; c < D; ++c) v[c] = vel_c(A, c, p, tr);
+    for (int c = 0; c < D; ++c) {
+        Corners<D> K;
+        v[c] = vel_c(A, Wn, c, p, K);
+    }
 }
 
+// adjoint of component c at the point of the corners K for the cotangent vb:
+// Vbar[c] += weights*vb, pb += slope*vb.  Only called on points the forward pass
+// found inside the component's grid.
 template <int D>
-__device__ inline void vel(const AdjArgs<D>& A, const double (&p)[D], double (&v)[D]) {
-    NoTrack tr;
-    vel(A, p, v, tr);
-}
-
-// destination of velocity cotangents: FP64 atomic adds to Vbar in global
-// memory, or into the workgroup's LDS tile (component c's nodes lo[c] ..
-// lo[c] + ext[c] - 1 per dimension, at tile offset off[c]) that is added to
-// Vbar once per block of steps
-// (named directly, not through a pointer in the sink: a pointer that may be null
-// makes the adds flat ones: 1 M particles, 100 RK2 steps 7.61 ms with them, 7.18
-// with LDS adds)
-extern __shared__ double adj_tile[];
-template <int D>
-struct VSink {
-    double* g[D];
-    bool tiled;  // false: global
-    int lo[D][D], ext[D][D], off[D];
-};
-
-// adjoint of component c at p for the cotangent vb: Vbar[c] += weights*vb,
-// pb += slope*vb.  Only called on points the forward pass found inside the
-// component's grid.
-template <int D>
-__device__ inline void vel_c_bw(const AdjArgs<D>& A, int c, const double (&p)[D], double vb,
-                                const VSink<D>& S, double (&pb)[D]) {
+__device__ inline void vel_c_bw(const AdjArgs<D>& A, const Window<D>& Wn, int c,
+                                const Corners<D>& K, double vb, double (&pb)[D]) {
     if (vb == 0.0) return;
-    Corners<D> K;
-    NoTrack nt;
-    gather(A, c, p, K, nt);
     const double* v = K.v;
     const double* t = K.t;
     double dd[D];
@@ -230,35 +276,35 @@ __device__ inline void vel_c_bw(const AdjArgs<D>& A, int c, const double (&p)[D]
     }
 #pragma unroll
     for (int d = 0; d < D; ++d) pb[d] += dd[d] * K.iv[d] * vb;
-    int base = 0;  // tile index of the lower corner
-    if (S.tiled) {
-        int stride = 1;
-#pragma unroll
-        for (int d = 0; d < D; ++d) {
-            base += ((int)K.k[d] - S.lo[c][d]) * stride;
-            stride *= S.ext[c][d];
-        }
-    }
+    const int64_t n0 = A.vg.ax[c][0].n, n1 = A.vg.ax[c][1].n;
 #pragma unroll
     for (int q = 0; q < (1 << D); ++q) {
         double w = 1.0;
 #pragma unroll
         for (int d = 0; d < D; ++d) w *= ((q >> d) & 1) ? t[d] : 1.0 - t[d];
-        if (S.tiled) {
-            int o = base + (q & 1) + ((q >> 1) & 1) * S.ext[c][0];
-            if constexpr (D == 3) o += ((q >> 2) & 1) * S.ext[c][0] * S.ext[c][1];
-            unsafeAtomicAdd(adj_tile + S.off[c] + o, w * vb);
-        } else {
-            unsafeAtomicAdd(S.g[c] + K.at[q], w * vb);
-        }
+        if (K.in)
+            unsafeAtomicAdd(adj_lds + (int)K.at + (q & 1) + ((q >> 1) & 1) * Wn.ext[c][0],
+                            w * vb);
+        else
+            unsafeAtomicAdd(
+                Wn.g[c] + K.at + (q & 1) + n0 * (((q >> 1) & 1) + n1 * ((q >> 2) & 1)), w * vb);
     }
+}
+template <int D>
+__device__ inline void vel_c_bw(const AdjArgs<D>& A, const Window<D>& Wn, int c,
+                                const double (&p)[D], double vb, double (&pb)[D]) {
+    if (vb == 0.0) return;
+    Corners<D> K;
+    gather(A, Wn, c, p, K);
+    vel_c_bw(A, Wn, c, K, vb, pb);
 }
 
 // one step (Euler.jl, RK2.jl with @muladd, RK4.jl unfused)
-template <int D, int M, class Tr>
-__device__ inline void step(const AdjArgs<D>& A, const double (&p0)[D], double (&out)[D], Tr& tr) {
+template <int D, int M>
+__device__ inline void step(const AdjArgs<D>& A, const Window<D>& Wn, const double (&p0)[D],
+                            double (&out)[D]) {
     double v0[D];
-    vel(A, p0, v0, tr);
+    vel(A, Wn, p0, v0);
     if constexpr (M == JP_EULER) {
 #pragma unroll
         for (int d = 0; d < D; ++d) out[d] = fma(A.dt, v0[d], p0[d]);
@@ -266,7 +312,7 @@ __device__ inline void step(const AdjArgs<D>& A, const double (&p0)[D], double (
         double p1[D], v1[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) p1[d] = fma(A.adt, v0[d], p0[d]);
-        vel(A, p1, v1, tr);
+        vel(A, Wn, p1, v1);
         if (A.half) {
 #pragma unroll
             for (int d = 0; d < D; ++d) out[d] = fma(A.dt, v1[d], p0[d]);
@@ -278,13 +324,13 @@ __device__ inline void step(const AdjArgs<D>& A, const double (&p0)[D], double (
         double q[D], k2[D], k3[D], k4[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) q[d] = p0[d] + (A.dt * v0[d]) / 2.0;
-        vel(A, q, k2, tr);
+        vel(A, Wn, q, k2);
 #pragma unroll
         for (int d = 0; d < D; ++d) q[d] = p0[d] + (A.dt * k2[d]) / 2.0;
-        vel(A, q, k3, tr);
+        vel(A, Wn, q, k3);
 #pragma unroll
         for (int d = 0; d < D; ++d) q[d] = p0[d] + A.dt * k3[d];
-        vel(A, q, k4, tr);
+        vel(A, Wn, q, k4);
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             const double sum = ((v0[d] + 2.0 * k2[d]) + 2.0 * k3[d]) + k4[d];
@@ -293,25 +339,23 @@ __device__ inline void step(const AdjArgs<D>& A, const double (&p0)[D], double (
     }
 }
 
-template <int D, int M>
-__device__ inline void step(const AdjArgs<D>& A, const double (&p0)[D], double (&out)[D]) {
-    NoTrack tr;
-    step<D, M>(A, p0, out, tr);
-}
-
 // reverse of step at p0: pb is the output's cotangent on entry, p0's on exit
 template <int D, int M>
-__device__ inline void step_bw(const AdjArgs<D>& A, const double (&p0)[D], double (&pb)[D],
-                               const VSink<D>& Vb) {
+__device__ inline void step_bw(const AdjArgs<D>& A, const Window<D>& Wn, const double (&p0)[D],
+                               double (&pb)[D]) {
     double ob[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) ob[d] = pb[d];
     if constexpr (M == JP_EULER) {
 #pragma unroll
-        for (int c = 0; c < D; ++c) vel_c_bw(A, c, p0, A.dt * ob[c], Vb, pb);
+        for (int c = 0; c < D; ++c) vel_c_bw(A, Wn, c, p0, A.dt * ob[c], pb);
     } else if constexpr (M == JP_RK2) {
         double v0[D], p1[D], v0b[D], v1b[D], p1b[D];
-        vel(A, p0, v0);
+        // kept for the reverse at p0, in 2D: four gathers for five (in 3D the
+        // registers would halve the wavefronts: 186 for 127)
+        Corners<D> K0[D];
+#pragma unroll
+        for (int c = 0; c < D; ++c) v0[c] = vel_c(A, Wn, c, p0, K0[c]);
 #pragma unroll
         for (int d = 0; d < D; ++d) p1[d] = fma(A.adt, v0[d], p0[d]);
         if (A.half) {
@@ -330,23 +374,28 @@ __device__ inline void step_bw(const AdjArgs<D>& A, const double (&p0)[D], doubl
 #pragma unroll
         for (int d = 0; d < D; ++d) p1b[d] = 0.0;
 #pragma unroll
-        for (int c = 0; c < D; ++c) vel_c_bw(A, c, p1, v1b[c], Vb, p1b);
+        for (int c = 0; c < D; ++c) vel_c_bw(A, Wn, c, p1, v1b[c], p1b);
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             pb[d] += p1b[d];
             v0b[d] += A.adt * p1b[d];
         }
 #pragma unroll
-        for (int c = 0; c < D; ++c) vel_c_bw(A, c, p0, v0b[c], Vb, pb);
+        for (int c = 0; c < D; ++c) {
+            if constexpr (D == 2)
+                vel_c_bw(A, Wn, c, K0[c], v0b[c], pb);
+            else
+                vel_c_bw(A, Wn, c, p0, v0b[c], pb);
+        }
     } else {
         double k1[D], k2[D], k3[D], q2[D], q3[D], q4[D], kb[4][D], qb[D];
-        vel(A, p0, k1);
+        vel(A, Wn, p0, k1);
 #pragma unroll
         for (int d = 0; d < D; ++d) q2[d] = p0[d] + (A.dt * k1[d]) / 2.0;
-        vel(A, q2, k2);
+        vel(A, Wn, q2, k2);
 #pragma unroll
         for (int d = 0; d < D; ++d) q3[d] = p0[d] + (A.dt * k2[d]) / 2.0;
-        vel(A, q3, k3);
+        vel(A, Wn, q3, k3);
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             q4[d] = p0[d] + A.dt * k3[d];
@@ -363,7 +412,7 @@ __device__ inline void step_bw(const AdjArgs<D>& A, const double (&p0)[D], doubl
 #pragma unroll
             for (int d = 0; d < D; ++d) qb[d] = 0.0;
 #pragma unroll
-            for (int c = 0; c < D; ++c) vel_c_bw(A, c, qs, kb[st][c], Vb, qb);
+            for (int c = 0; c < D; ++c) vel_c_bw(A, Wn, c, qs, kb[st][c], qb);
 #pragma unroll
             for (int d = 0; d < D; ++d) {
                 pb[d] += qb[d];
@@ -371,7 +420,7 @@ __device__ inline void step_bw(const AdjArgs<D>& A, const double (&p0)[D], doubl
             }
         }
 #pragma unroll
-        for (int c = 0; c < D; ++c) vel_c_bw(A, c, p0, kb[0][c], Vb, pb);
+        for (int c = 0; c < D; ++c) vel_c_bw(A, Wn, c, p0, kb[0][c], pb);
     }
 }
 
@@ -410,37 +459,205 @@ __device__ inline int64_t node_of(const AdjArgs<D>& A, const int64_t (&k)[D], in
     return D == 2 ? N[0] + A.nn[0] * N[1] : N[0] + A.nn[0] * (N[1] + A.nn[1] * N[D - 1]);
 }
 
-template <int D, int M>
-__global__ __launch_bounds__(kBlock) void k_adj_fwd(AdjArgs<D> A, CPtr3 x0,
-                                                    double* __restrict__ ckpt,
-                                                    uint8_t* __restrict__ alive, Ptr3 xN,
-                                                    int32_t* __restrict__ cell,
-                                                    int32_t* __restrict__ cnt) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= A.np) return;
-    double x[D];
+// threads of the largest workgroup with a window: 16 wavefronts
+constexpr int kWindowBlock = 1024;
+
+__device__ inline double uniform(double v) {
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)u);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(u >> 32));
+    return __longlong_as_double((int64_t)(((uint64_t)hi << 32) | lo));
+}
+
+// window index r -> component, column, row (r < 2^15: the product's rounding is
+// far below the 0.5/ext that r + 0.5 keeps from a row's edge)
+__device__ inline void window_node(const Window<2>& Wn, int r, int& c, int& x, int& y) {
+    c = r >= Wn.off[1] ? 1 : 0;
+    r -= c ? Wn.off[1] : 0;
+    const int e = c ? Wn.ext[1][0] : Wn.ext[0][0];
+    y = (int)(((float)r + 0.5f) * (1.0f / (float)e));
+    x = r - y * e;
+}
+
+template <int D>
+__device__ inline void init_window(const AdjArgs<D>& A, Window<D>& Wn) {
 #pragma unroll
-    for (int d = 0; d < D; ++d) x[d] = x0.p[d][i];
-    bool a = indomain(A.G, x);
+    for (int c = 0; c < D; ++c) {
+        Wn.g[c] = nullptr;
 #pragma unroll
-    for (int d = 0; d < D; ++d) ckpt[(int64_t)d * A.np + i] = x[d];
-    int64_t blk = 0;
-    int left = A.every;
-    for (int s = 0; s < A.nsteps; ++s) {
-        if (left == 0) {
-            ++blk;
-            left = A.every;
-#pragma unroll
-            for (int d = 0; d < D; ++d) ckpt[(blk * D + d) * A.np + i] = x[d];
+        for (int d = 0; d < D; ++d) {
+            Wn.x0[c][d] = uniform(A.vg.ax[c][d].x[0]);
+            Wn.i0[c][d] = uniform(A.vg.ax[c][d].idx[0]);
         }
-        --left;
-        if (!a) continue;
-        double y[D];
-        step<D, M>(A, x, y);
-#pragma unroll
-        for (int d = 0; d < D; ++d) x[d] = y[d];
-        a = indomain(A.G, x);
     }
+    Wn.staged = Wn.tiled = false;
+}
+
+// box of the brackets of the positions mn .. mx (the workgroup's, per dimension),
+// `margin` intervals wider; what fits of it (with TILE the tile, then the
+// velocities and axes) is cleared and loaded.  Called by the whole workgroup;
+// returns the tile's nodes (0: no tile).
+template <bool TILE>
+__device__ inline int open_window(const AdjArgs<2>& A, Window<2>& Wn, const double (&mn)[2],
+                                  const double (&mx)[2], int margin, int cap) {
+    __shared__ double sred[kWindowBlock / 64][4];
+    __shared__ int sbox[2][2][2];
+    const int lt = threadIdx.x, B = blockDim.x;
+    double m[4] = {mn[0], -mx[0], mn[1], -mx[1]};
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) m[j] = fmin(m[j], __shfl_xor(m[j], o));
+        if ((lt & 63) == 0) sred[lt >> 6][j] = m[j];
+    }
+    __syncthreads();
+    if (lt < 8) {
+        const int c = lt >> 2, d = (lt >> 1) & 1, hi = lt & 1;
+        double v = sred[0][2 * d + hi];
+        for (int w = 1; w < B / 64; ++w) v = fmin(v, sred[w][2 * d + hi]);
+        int k = -1;  // no live particle
+        if (v < __builtin_inf()) {
+            const Axis& X = A.vg.ax[c][d];
+            const double p = fmax(X.x[0], fmin(hi ? -v : v, X.x[X.n - 1]));
+            const int b = (int)adj_bracket(p, X);
+            k = hi ? min(b + 1 + margin, (int)X.n - 1) : max(b - margin, 0);
+        }
+        sbox[c][d][hi] = k;
+    }
+    __syncthreads();
+    int total = 0, axes = 0;
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            const int lo = __builtin_amdgcn_readfirstlane(sbox[c][d][0]);
+            const int hi = __builtin_amdgcn_readfirstlane(sbox[c][d][1]);
+            if (lo < 0) return 0;
+            Wn.lo[c][d] = lo;
+            Wn.ext[c][d] = hi - lo + 1;
+        }
+        const int64_t sz = (int64_t)Wn.ext[c][0] * Wn.ext[c][1];
+        Wn.off[c] = total;
+        if (sz > cap) return 0;
+        total += (int)sz;
+    }
+    if (total > cap) return 0;
+    Wn.tiled = TILE;
+    Wn.vo = TILE ? total : 0;
+#pragma unroll
+    for (int c = 0; c < 2; ++c)
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            Wn.ax[c][d] = Wn.vo + total + axes;
+            axes += 2 * Wn.ext[c][d];
+        }
+    Wn.staged = Wn.vo + total + axes <= cap;
+    if (TILE)
+        for (int t = lt; t < total; t += B) adj_lds[t] = 0.0;
+    if (Wn.staged) {
+        for (int t = lt; t < total; t += B) {
+            int c, x, y;
+            window_node(Wn, t, c, x, y);
+            const double* __restrict__ V = c ? A.V[1] : A.V[0];
+            const int64_t n = c ? A.vg.ax[1][0].n : A.vg.ax[0][0].n;
+            const int lx = c ? Wn.lo[1][0] : Wn.lo[0][0], ly = c ? Wn.lo[1][1] : Wn.lo[0][1];
+            adj_lds[Wn.vo + t] = V[lx + x + n * (ly + y)];
+        }
+#pragma unroll
+        for (int c = 0; c < 2; ++c)
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {
+                const Axis& X = A.vg.ax[c][d];
+                const int lo = Wn.lo[c][d], e = Wn.ext[c][d];
+                for (int t = lt; t < e; t += B) {
+                    adj_lds[Wn.ax[c][d] + t] = X.x[lo + t];
+                    // intervals: one fewer than nodes
+                    adj_lds[Wn.ax[c][d] + e + t] = t + 1 < e ? X.idx[lo + t] : 0.0;
+                }
+            }
+    }
+    __syncthreads();
+    return total;
+}
+
+// the tile's nonzero entries go to Vbar; called by the whole workgroup
+__device__ inline void close_window(const AdjArgs<2>& A, Window<2>& Wn, int total) {
+    __syncthreads();
+    for (int t = threadIdx.x; t < total; t += blockDim.x) {
+        const double v = adj_lds[t];
+        if (v == 0.0) continue;
+        int c, x, y;
+        window_node(Wn, t, c, x, y);
+        const int64_t n = c ? A.vg.ax[1][0].n : A.vg.ax[0][0].n;
+        const int lx = c ? Wn.lo[1][0] : Wn.lo[0][0], ly = c ? Wn.lo[1][1] : Wn.lo[0][1];
+        unsafeAtomicAdd((c ? Wn.g[1] : Wn.g[0]) + lx + x + n * (ly + y), v);
+    }
+    __syncthreads();  // the tile is reused by the next block
+    Wn.staged = Wn.tiled = false;
+}
+
+// 2D: the velocities of a block of steps from LDS windows (80 KB: two workgroups
+// of 16 wavefronts per CU), sized for a straight line on from the block before
+// (before the first: along the velocity at the start).
+constexpr int kFwd2 = 512;
+constexpr size_t kFwdLds = 80 * 1024 - 1024;  // less the static words
+template <int D, int M>
+__global__ __launch_bounds__(D == 2 ? kFwd2 : kBlock, D == 2 ? 4 : 1) void k_adj_fwd(
+    AdjArgs<D> A, CPtr3 x0, double* __restrict__ ckpt, uint8_t* __restrict__ alive, Ptr3 xN,
+    int32_t* __restrict__ cell, int32_t* __restrict__ cnt, int cap) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const bool own = i < A.np;  // every thread reaches the block-wide barriers
+    if (D == 3 && !own) return;
+    Window<D> Wn;
+    init_window(A, Wn);
+    double x[D], go[D];  // position, displacement expected of the block
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+        x[d] = own ? x0.p[d][i] : 0.0;
+        go[d] = 0.0;
+    }
+    bool a = own && indomain(A.G, x);
+    if (D == 2 && a) {
+        double v[D];
+        vel(A, Wn, x, v);
+#pragma unroll
+        for (int d = 0; d < D; ++d) go[d] = (A.every < A.nsteps ? A.every : A.nsteps) * (A.dt * v[d]);
+    }
+    for (int s0 = 0;; s0 += A.every) {
+        if (own) {
+#pragma unroll
+            for (int d = 0; d < D; ++d)
+                ckpt[((int64_t)(s0 / A.every) * D + d) * A.np + i] = x[d];
+        }
+        const int n = A.nsteps - s0 < A.every ? A.nsteps - s0 : A.every;
+        if (n <= 0) break;
+        if constexpr (D == 2) {
+            double mn[2], mx[2];
+#pragma unroll
+            for (int d = 0; d < 2; ++d) {
+                mn[d] = a ? fmin(x[d], x[d] + go[d]) : __builtin_inf();
+                mx[d] = a ? fmax(x[d], x[d] + go[d]) : -__builtin_inf();
+            }
+            open_window<false>(A, Wn, mn, mx, 1, cap);
+        }
+#pragma unroll
+        for (int d = 0; d < D; ++d) go[d] = -x[d];
+        for (int j = 0; j < n && a; ++j) {
+            double y[D];
+            step<D, M>(A, Wn, x, y);
+#pragma unroll
+            for (int d = 0; d < D; ++d) x[d] = y[d];
+            a = indomain(A.G, x);
+        }
+#pragma unroll
+        for (int d = 0; d < D; ++d) go[d] += x[d];
+        if (s0 + A.every >= A.nsteps) break;
+        if constexpr (D == 2) {
+            __syncthreads();  // the window is reused
+            Wn.staged = false;
+        }
+    }
+    if (!own) return;
     alive[i] = a ? 1 : 0;
 #pragma unroll
     for (int d = 0; d < D; ++d) xN.p[d][i] = x[d];
@@ -698,151 +915,111 @@ __global__ __launch_bounds__(kBlock) void k_adj_zero(double* __restrict__ p, int
     if (i < n) p[i] = 0.0;
 }
 
-// LDS tile for the velocity cotangents of one workgroup and block of steps
-// (2D only), the 64 KB workgroup budget less the static box words.  A
-// workgroup from a compact patch touches ~2-6 k nodes over ten steps; in 3D
-// the footprint rarely fits and global atomics are used.
-constexpr size_t kLdsBudget = 65536 - 256;
-template <int D>
-inline int tile_cap() {
-    return D == 2 ? (int)(kLdsBudget / sizeof(double)) : 0;
-}
+// Backward workgroups.  2D: the LDS of a CU holds the window of one workgroup, so
+// a workgroup has as many particles as spread the list over the CUs, up to 1024
+// (16 wavefronts, what 128 registers allow); a list from compact patches touches
+// 1.3-8 k nodes of both components in ten steps of CFL 1, patches of 1024 as many
+// as of 512 (the cells' rows and the flow set the extent).  3D: no window.
+constexpr int kBwd3 = 512;
+constexpr size_t kLdsBudget = 160 * 1024 - 1024;  // less the static words
 
 template <int D, int M>
-__global__ __launch_bounds__(kAdjBlock) void k_adj_bwd(
+__global__ __launch_bounds__(D == 2 ? kWindowBlock : kBwd3) void k_adj_bwd(
     AdjArgs<D> A, const double* __restrict__ ckpt, const uint8_t* __restrict__ alive,
     const double* __restrict__ Tp, const double* __restrict__ F, const double* __restrict__ W,
     const double* __restrict__ Fbar, Ptr3 Vb, Ptr3 x0b, double* __restrict__ Tpb,
     double* __restrict__ tape, int cap) {
-    // tape (global scratch, [every][D][np]): step-start positions of the block
-    // of steps being reversed; dynamic LDS: the cotangent tile of cap doubles
-    __shared__ int sbox[D][D][2];
+    // tape (global scratch, [every][D][threads of the grid]): step-start positions
+    // of the block of steps being reversed; dynamic LDS: the window (cap doubles)
     const int lt = threadIdx.x;
-    const int64_t i = (int64_t)blockIdx.x * kAdjBlock + lt;
-    // every thread reaches the block-wide barriers below
-    const bool live = i < A.np && alive[i];
-    VSink<D> S;
-#pragma unroll
-    for (int c = 0; c < D; ++c) S.g[c] = Vb.p[c];
-    S.tiled = false;
-    double pb[D];
-#pragma unroll
-    for (int d = 0; d < D; ++d) pb[d] = 0.0;
-    double tb = 0.0;
+    const int64_t nt = (int64_t)gridDim.x * blockDim.x;
+    const int64_t tid = (int64_t)blockIdx.x * blockDim.x + lt;
     const int nblk = A.nsteps == 0 ? 1 : (A.nsteps + A.every - 1) / A.every;
-    for (int b = nblk - 1; b >= 0; --b) {
-        const int s0 = b * A.every;
-        const int n = A.nsteps - s0 < A.every ? A.nsteps - s0 : A.every;
-        BoxTrack<D> box;
-        if (live) {
+    Window<D> Wn;
+    init_window(A, Wn);
+#pragma unroll
+    for (int c = 0; c < D; ++c) Wn.g[c] = Vb.p[c];
+    for (int64_t first = (int64_t)blockIdx.x * blockDim.x; first < A.np; first += nt) {
+        const int64_t i = first + lt;
+        // every thread reaches the block-wide barriers below
+        const bool live = i < A.np && alive[i];
+        double pb[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) pb[d] = 0.0;
+        double tb = 0.0;
+        for (int b = nblk - 1; b >= 0; --b) {
+            const int s0 = b * A.every;
+            const int n = A.nsteps - s0 < A.every ? A.nsteps - s0 : A.every;
             double x[D];
+            if (live) {
 #pragma unroll
-            for (int d = 0; d < D; ++d) x[d] = ckpt[((int64_t)b * D + d) * A.np + i];
-            for (int j = 0; j < n; ++j) {
-#pragma unroll
-                for (int d = 0; d < D; ++d) tape[((int64_t)j * D + d) * A.np + i] = x[d];
-                double y[D];
-                step<D, M>(A, x, y, box);
-#pragma unroll
-                for (int d = 0; d < D; ++d) x[d] = y[d];
+                for (int d = 0; d < D; ++d) x[d] = ckpt[((int64_t)b * D + d) * A.np + i];
             }
-            if (b == nblk - 1) {
-                // particle2grid! adjoint at the final position x
-                int64_t k[D];
+            int total = 0;
+            if constexpr (D == 2) {
+                // where the block begins and ends: the next block's start; for the
+                // last block a straight line on from the one before.  Points beyond
+                // it (a bend of the path) are few and take the global path.
+                double mn[2], mx[2];
 #pragma unroll
-                for (int d = 0; d < D; ++d) k[d] = adj_bracket(x[d], A.G.xv[d]);
-                const double t = Tp[i];
-#pragma unroll
-                for (int q = 0; q < (1 << D); ++q) {
-                    double xn[D], wi;
-                    const int64_t nd = node_of(A, k, q, x, xn, wi);
-                    const double iw = 1.0 / W[nd];
-                    const double fb = Fbar[nd];
-                    tb += fb * wi * iw;
-                    const double gw = fb * (t - F[nd]) * iw;
-#pragma unroll
-                    for (int d = 0; d < D; ++d) pb[d] += gw * (-2.0 * (x[d] - xn[d]) * wi * wi);
-                }
-            }
-        }
-        int total = 0;
-        if constexpr (D == 2) {
-            // the workgroup's node range per component and dimension
-            if (lt < D * D) {
-                (&sbox[0][0][0])[2 * lt] = 0x7fffffff;
-                (&sbox[0][0][0])[2 * lt + 1] = -1;
-            }
-            __syncthreads();
-            if (live && n > 0) {
-#pragma unroll
-                for (int c = 0; c < D; ++c)
-#pragma unroll
-                    for (int d = 0; d < D; ++d) {
-                        atomicMin(&sbox[c][d][0], box.lo[c][d]);
-                        atomicMax(&sbox[c][d][1], box.hi[c][d]);
+                for (int d = 0; d < 2; ++d) {
+                    mn[d] = __builtin_inf();
+                    mx[d] = -__builtin_inf();
+                    if (live && n > 0) {
+                        double e = x[d];
+                        if (b + 1 < nblk)
+                            e = ckpt[((int64_t)(b + 1) * 2 + d) * A.np + i];
+                        else if (b > 0)
+                            e += (x[d] - ckpt[((int64_t)(b - 1) * 2 + d) * A.np + i]) *
+                                 ((double)n / (double)A.every);
+                        mn[d] = fmin(x[d], e);
+                        mx[d] = fmax(x[d], e);
                     }
-            }
-            __syncthreads();
-            bool any = true;
-#pragma unroll
-            for (int c = 0; c < D; ++c) {
-                int sz = 1;
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    S.lo[c][d] = sbox[c][d][0];
-                    const int e = sbox[c][d][1] - sbox[c][d][0] + 2;  // corners k .. k+1
-                    any = any && sbox[c][d][1] >= sbox[c][d][0];
-                    S.ext[c][d] = e;
-                    sz *= e > 0 ? e : 0;
                 }
-                S.off[c] = total;
-                total += sz;
+                total = open_window<true>(A, Wn, mn, mx, nblk == 1 ? n : 1, cap);
             }
-            if (any && total <= cap) {
-                for (int t = lt; t < total; t += kAdjBlock) adj_tile[t] = 0.0;
-                S.tiled = true;
-            } else {
-                S.tiled = false;
-                total = 0;
-            }
-            __syncthreads();
-        }
-        if (live) {
-            for (int j = n - 1; j >= 0; --j) {
-                double p0[D];
+            if (live) {
+                for (int j = 0; j < n; ++j) {
 #pragma unroll
-                for (int d = 0; d < D; ++d) p0[d] = tape[((int64_t)j * D + d) * A.np + i];
-                step_bw<D, M>(A, p0, pb, S);
-            }
-        }
-        if constexpr (D == 2) {
-            __syncthreads();
-            // the tile's nonzero entries go to Vbar
-            for (int t = lt; t < total; t += kAdjBlock) {
-                const double v = adj_tile[t];
-                if (v == 0.0) continue;
-                int c = 0;
+                    for (int d = 0; d < D; ++d) tape[((int64_t)j * D + d) * nt + tid] = x[d];
+                    double y[D];
+                    step<D, M>(A, Wn, x, y);
 #pragma unroll
-                for (int cc = 1; cc < D; ++cc) c = t >= S.off[cc] ? cc : c;
-                int r = t - S.off[c];
-                int64_t gi = 0, stride = 1;
-#pragma unroll
-                for (int d = 0; d < D; ++d) {
-                    const int64_t node = S.lo[c][d] + r % S.ext[c][d];
-                    r /= S.ext[c][d];
-                    gi += node * stride;
-                    stride *= A.vg.ax[c][d].n;
+                    for (int d = 0; d < D; ++d) x[d] = y[d];
                 }
-                unsafeAtomicAdd(S.g[c] + gi, v);
-            }
-            __syncthreads();  // the tile and the box are reused by the next block
-            S.tiled = false;
-        }
-    }
-    if (i < A.np) {
+                if (b == nblk - 1) {
+                    // particle2grid! adjoint at the final position x
+                    int64_t k[D];
 #pragma unroll
-        for (int d = 0; d < D; ++d) x0b.p[d][i] = pb[d];
-        Tpb[i] = tb;
+                    for (int d = 0; d < D; ++d) k[d] = adj_bracket(x[d], A.G.xv[d]);
+                    const double t = Tp[i];
+#pragma unroll
+                    for (int q = 0; q < (1 << D); ++q) {
+                        double xn[D], wi;
+                        const int64_t nd = node_of(A, k, q, x, xn, wi);
+                        const double iw = 1.0 / W[nd];
+                        const double fb = Fbar[nd];
+                        tb += fb * wi * iw;
+                        const double gw = fb * (t - F[nd]) * iw;
+#pragma unroll
+                        for (int d = 0; d < D; ++d)
+                            pb[d] += gw * (-2.0 * (x[d] - xn[d]) * wi * wi);
+                    }
+                }
+                for (int j = n - 1; j >= 0; --j) {
+                    double p0[D];
+#pragma unroll
+                    for (int d = 0; d < D; ++d) p0[d] = tape[((int64_t)j * D + d) * nt + tid];
+                    step_bw<D, M>(A, Wn, p0, pb);
+                }
+            }
+            if constexpr (D == 2) close_window(A, Wn, total);
+        }
+        if (i < A.np) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) x0b.p[d][i] = pb[d];
+            Tpb[i] = tb;
+        }
     }
 }
 
@@ -914,6 +1091,14 @@ int zero(jp_ctx* ctx, double* p, int64_t n) {
     return JP_OK;
 }
 
+// threads of a workgroup with a window: as many as spread np particles over the
+// workgroups that the CUs hold at once, one wavefront at least
+int window_block(int64_t np, int held, int most) {
+    int B = 64;
+    while (B < most && (int64_t)B * held < np) B *= 2;
+    return B;
+}
+
 template <int D>
 int64_t node_count(const jp_cellgrid* g) {
     int64_t n = 1;
@@ -956,12 +1141,15 @@ int forward(jp_ctx* ctx, const AdjArgs<D>& A, const double* const* x0, const dou
         xq.p[d] = xN[d];
     }
     if (A.np > 0) {
-        if (sf.on)
+        if (sf.on) {
             k_adj_fwd_split<D, M><<<(unsigned)blocks_for(A.np), kBlock, 0, ctx->stream>>>(
                 A, sf.SV, sf.geo, sf.P, xp, ckpt, alive, xo, cell, cnt);
-        else
-            k_adj_fwd<D, M><<<(unsigned)blocks_for(A.np), kBlock, 0, ctx->stream>>>(
-                A, xp, ckpt, alive, xo, cell, cnt);
+        } else {
+            const int B = D == 2 ? window_block(A.np, 2 * ctx->num_cu, kFwd2) : kBlock;
+            const size_t lds = D == 2 ? kFwdLds : 0;
+            k_adj_fwd<D, M><<<(unsigned)blocks_for(A.np, B), B, lds, ctx->stream>>>(
+                A, xp, ckpt, alive, xo, cell, cnt, (int)(lds / sizeof(double)));
+        }
         JP_LAUNCHED(ctx);
     }
     k_adj_scan<<<1, kScan, 0, ctx->stream>>>(cnt, start, C);
@@ -993,13 +1181,20 @@ int backward(jp_ctx* ctx, const AdjArgs<D>& A, const jp_velgrid* vg, const doubl
         xb.p[c] = x0bar[c];
     }
     if (A.np > 0) {
-        const int cap = tile_cap<D>();
-        const size_t lds = (size_t)cap * sizeof(double);
-        int rc = ensure_scratch(ctx, (size_t)A.every * D * A.np * sizeof(double));
+        // 2D: one workgroup per CU at a time, each going on to further particles
+        int B = kBwd3;
+        int64_t grid = blocks_for(A.np, B);
+        size_t lds = 0;
+        if (D == 2) {
+            B = window_block(A.np, ctx->num_cu, kWindowBlock);
+            grid = std::min<int64_t>(blocks_for(A.np, B), ctx->num_cu);
+            lds = kLdsBudget;
+        }
+        int rc = ensure_scratch(ctx, (size_t)A.every * D * grid * B * sizeof(double));
         if (rc) return rc;
         double* tape = static_cast<double*>(ctx->scratch);
-        k_adj_bwd<D, M><<<(unsigned)blocks_for(A.np, kAdjBlock), kAdjBlock, lds, ctx->stream>>>(
-            A, ckpt, alive, Tp, F, W, Fbar, vb, xb, Tpbar, tape, cap);
+        k_adj_bwd<D, M><<<(unsigned)grid, B, lds, ctx->stream>>>(
+            A, ckpt, alive, Tp, F, W, Fbar, vb, xb, Tpbar, tape, (int)(lds / sizeof(double)));
         JP_LAUNCHED(ctx);
     }
     return finish(ctx);
