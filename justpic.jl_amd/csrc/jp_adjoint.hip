@@ -681,12 +681,6 @@ __global__ __launch_bounds__(D == 2 ? kFwd2 : kBlock, D == 2 ? 4 : 1) void k_adj
 // cell leaves the grid, or whose offset is not finite, is deleted.  The
 // checkpoints, xN and the gather use the FP64 position x_I + u*h, so the
 // FP64 backward recomputes each block from the split trajectory.
-struct NoWindow {  // every corner from global memory
-    __host__ __device__ static constexpr int n(int) { return 1; }
-    __host__ __device__ static constexpr int w(int) { return 0; }
-    __host__ __device__ static constexpr int size() { return 1; }
-};
-
 template <int D, int M>
 __global__ __launch_bounds__(kBlock) void k_adj_fwd_split(
     AdjArgs<D> A, split::SVelIn<D> SV, const SplitGeom* __restrict__ geo, split::RKf P, CPtr3 x0,
@@ -726,7 +720,6 @@ __global__ __launch_bounds__(kBlock) void k_adj_fwd_split(
     }
 #pragma unroll
     for (int d = 0; d < D; ++d) ckpt[(int64_t)d * A.np + i] = x[d];
-    const int w0[D][D] = {};
     int64_t blk = 0;
     int left = A.every;
     for (int s = 0; s < A.nsteps; ++s) {
@@ -741,7 +734,7 @@ __global__ __launch_bounds__(kBlock) void k_adj_fwd_split(
         split::CellMap<D> cm;
         split::cell_map<D, false>(m, I, cm);
         float out[D];
-        split::advect_split_one<D, M, NoWindow>(nullptr, SV, sc, w0, I, cm, P, u, out);
+        split::advect_split_one<D, M>(split::GlobalVelocity<D>{SV, sc, I, cm}, P, u, out);
         bool gone = false;
         int sd[D];
 #pragma unroll

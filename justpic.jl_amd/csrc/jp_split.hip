@@ -181,11 +181,12 @@ __device__ inline void adv_split_tile(const SGrid<D>& g, const SVelIn<D>& V, con
     double sc[D];
 #pragma unroll
     for (int c = 0; c < D; ++c) sc[c] = dt / g.h[c][0];
-    int w0[D][D];
+    SWindow<D> W;
 #pragma unroll
     for (int c = 0; c < D; ++c)
 #pragma unroll
-        for (int d = 0; d < D; ++d) w0[c][d] = window_origin<D, STD>(m, c, d, t0[d]);
+        for (int d = 0; d < D; ++d) W.w0[c][d] = window_origin<D, STD>(m, c, d, t0[d]);
+    window_limits<D, TS, STD>(V, W);
     const int tid = threadIdx.x;
     // window fill: every load issued before the LDS stores
     constexpr int NI = (TS::size() + kBlock - 1) / kBlock;
@@ -201,7 +202,7 @@ __device__ inline void adv_split_tile(const SGrid<D>& g, const SVelIn<D>& V, con
             bool ok = i < TS::size();
 #pragma unroll
             for (int d = 0; d < D; ++d) {
-                const int k = w0[c][d] + r % TS::w(d);
+                const int k = W.w0[c][d] + r % TS::w(d);
                 r /= TS::w(d);
                 ok = ok && k >= 0 && k < V.n[c][d];
                 node += k * stride;
@@ -216,82 +217,144 @@ __device__ inline void adv_split_tile(const SGrid<D>& g, const SVelIn<D>& V, con
         for (int it = 0; it < NI; ++it)
             if (tid + it * kBlock < TS::size()) sV[c][tid + it * kBlock] = wv[c][it];
     __syncthreads();
-    // the cell of thread t of the tile, its linear index, and whether it is
-    // in the grid
-    auto cell_of = [&](int t, int (&J)[D], int64_t& cj) {
-        bool in = true;
-        int r = t;
+    // A wavefront's cells: lane l is cell l % N0 of row l / N0 of its rows, from
+    // local cell w[] of the tile (uniform).
+    constexpr int N0 = TS::n(0) < 64 ? TS::n(0) : 64;
+    static_assert(TS::n(0) % N0 == 0 && TS::n(1) % (64 / N0) == 0, "rows of a wavefront");
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    int w[D];
+    {
+        int r = wave * 64;
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-            J[d] = t0[d] + r % TS::n(d);
+            w[d] = t0[d] + r % TS::n(d);
             r /= TS::n(d);
-            in = in && J[d] < g.ni[d];
         }
-        cj = J[D - 1];
+    }
+    int64_t first = w[D - 1];  // linear index of cell w
 #pragma unroll
-        for (int d = D - 2; d >= 0; --d) cj = cj * g.ni[d] + J[d];
-        return in;
-    };
-    int I[D];
-    int64_t c;
-    const bool in = cell_of(tid, I, c);
+    for (int d = D - 2; d >= 0; --d) first = first * g.ni[d] + w[d];
     const int64_t C = g.C;
+    const uint32_t n0 = (uint32_t)g.ni[0];
+    bool in = w[0] + lane % N0 < g.ni[0] && w[1] + lane / N0 < g.ni[1];
+    if constexpr (D == 3) in = in && w[2] < g.ni[2];
+    const int64_t c = first + lane % N0 + (int64_t)(lane / N0) * n0;
     // a thread outside the grid owns no particle but still takes work
     const uint64_t act = !in ? 0ull
                              : ((kb == 0 && ke == g.K) ? active_slots(index, c, C, g.K)
                                                        : active_slots_in(index, c, C, kb, ke));
-    // Chunks of CH slot planes.  The wavefront's active particles of a chunk
-    // are listed (plane-major, then lane) and dealt to its lanes in turn, so
-    // that every lane advects about the same number of particles (a lane per
-    // cell walking its own slots idles whenever its cell has fewer active
-    // slots in the chunk than the fullest cell); consecutive list entries are
-    // neighbouring cells of one plane, so the loads and stores stay
-    // coalesced.  The list is written and read by the same wavefront (its LDS
-    // operations complete in order).
-    constexpr int CH = D == 2 ? 8 : 4;  // 3D: fewer positions in registers
-    __shared__ uint16_t s_items[kBlock / 64][CH * 64];
-    uint16_t* items = s_items[tid >> 6];
-    const int lane = tid & 63, wbase = tid & ~63;
-    for (int k0 = kb; k0 < ke; k0 += CH) {
-        int n = 0;
+    // The wavefront's active particles are listed (plane-major, then lane) and
+    // dealt to its lanes in turn, G groups of 64 at a time, so that every lane
+    // advects about the same number of particles (a lane per cell walking its own
+    // slots idles whenever its cell has fewer active slots in the chunk than the
+    // fullest cell); consecutive list entries are neighbouring cells of one plane,
+    // so the loads and stores stay coalesced.  The next groups' positions are
+    // loaded before the current ones are advected.  The list is written, a chunk
+    // of CH planes ahead, and read by the same wavefront (its LDS operations
+    // complete in order).  (3D is bound by the slots' bytes: G = 1, 2 and 4 take
+    // 800, 810 and 822 us at 128^3; 2D: G = 4 46 us at 512^2, chunks without
+    // carried entries or loads ahead 49.)
+    constexpr int CH = 4, G = D == 2 ? 4 : 1;
+    __shared__ uint16_t s_items[kBlock / 64][(CH + G) * 64];
+    uint16_t* items = s_items[wave];
+    float* __restrict__ base[D];
 #pragma unroll
-        for (int j = 0; j < CH; ++j) {
-            const bool a = k0 + j < 64 && ((act >> (k0 + j)) & 1);
-            const uint64_t bal = __ballot(a);
-            const int below = (int)__builtin_amdgcn_mbcnt_hi(
-                (uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-            if (a) items[n + below] = (uint16_t)((j << 6) | lane);
-            n += __popcll(bal);
+    for (int d = 0; d < D; ++d) base[d] = off.p[d] + first;
+    // element of an entry (slot << 6 | lane) from there
+    auto at = [&](int item) __attribute__((always_inline)) {
+        const uint32_t l = (uint32_t)item & 63u;
+        return (uint64_t)((uint32_t)item >> 6) * (uint64_t)C +
+               (l % N0 + (N0 == 32 ? ((l & 32u) ? n0 : 0u) : (l / N0) * n0));
+    };
+    // slots that a stage takes out of the windows (steps of more than a cell)
+    __shared__ uint32_t s_miss[kBlock][2];
+    s_miss[tid][0] = s_miss[tid][1] = 0;
+    int n = 0;  // entries waiting
+    int k0 = kb;
+    // the next groups: their entries and positions (past the end the last entry,
+    // whose result is not stored)
+    auto next = [&](int (&dq)[G], float (&uq)[G][D]) __attribute__((always_inline)) {
+        while (n < 64 * G && k0 < ke) {
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                const bool a = k0 + j < 64 && ((act >> (k0 + j)) & 1);
+                const uint64_t bal = __ballot(a);
+                const int below = (int)__builtin_amdgcn_mbcnt_hi(
+                    (uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+                if (a) items[n + below] = (uint16_t)(((k0 + j) << 6) | lane);
+                n += __popcll(bal);
+            }
+            k0 += CH;
         }
-        if (!n) continue;
-        // this lane's entries lane, lane + 64, ...: positions loaded first
-        float uq[CH][D];
-        int dq[CH];
+        const int take = n < 64 * G ? n : 64 * G;
 #pragma unroll
-        for (int q = 0; q < CH; ++q) {
-            const int item = lane + 64 * q;
-            dq[q] = item < n ? items[item] : -1;
-            int J[D];
-            int64_t cj;
-            cell_of(wbase + (dq[q] & 63), J, cj);
-            const int64_t e = cj + C * (k0 + (dq[q] >> 6));
+        for (int q = 0; q < G; ++q) dq[q] = items[max(0, min(lane + 64 * q, take - 1))];
+        n -= take;
+        if (lane < n) items[lane] = items[take + lane];
+        for (int i = lane + 64; i < n; i += 64) items[i] = items[take + i];
 #pragma unroll
-            for (int d = 0; d < D; ++d) uq[q][d] = dq[q] >= 0 ? off.p[d][e] : 0.0f;
+        for (int q = 0; q < G; ++q) {
+            const uint64_t e = at(dq[q]);
+#pragma unroll
+            for (int d = 0; d < D; ++d) uq[q][d] = base[d][e];
         }
+        return take;
+    };
+    float uq[G][D], un[G][D];
+    int dq[G], dn[G];
+    int take = __any(act != 0) ? next(dq, uq) : 0;
+    while (take) {
+        const int then = next(dn, un);
 #pragma unroll
-        for (int q = 0; q < CH; ++q) {
-            if (dq[q] < 0) break;
+        for (int q = 0; q < G; ++q) {
+            if (64 * q >= take) break;
+            const int l = dq[q] & 63;
             int J[D];
-            int64_t cj;
-            cell_of(wbase + (dq[q] & 63), J, cj);
+            J[0] = w[0] + l % N0;
+            J[1] = w[1] + l / N0;
+            if constexpr (D == 3) J[2] = w[2];
             CellMap<D> cm;
             cell_map<D, STD>(m, J, cm);
             float out[D];
-            advect_split_one<D, M, TS>(sV, V, sc, w0, J, cm, P, uq[q], out);
-            const int64_t e = cj + C * (k0 + (dq[q] >> 6));
+            const bool ok = advect_split_one<D, M>(WindowVelocity<D, TS>{sV, W, J, cm}, P, uq[q],
+                                                   out);
+            if (lane + 64 * q < take) {
+                if (ok) {
+                    const uint64_t e = at(dq[q]);
 #pragma unroll
-            for (int d = 0; d < D; ++d) off.p[d][e] = out[d];
+                    for (int d = 0; d < D; ++d) base[d][e] = out[d];
+                } else {
+                    atomicOr(&s_miss[tid - lane + l][dq[q] >> 11], 1u << ((dq[q] >> 6) & 31));
+                }
+            }
         }
+        take = then;
+#pragma unroll
+        for (int q = 0; q < G; ++q) {
+            dq[q] = dn[q];
+#pragma unroll
+            for (int d = 0; d < D; ++d) uq[q][d] = un[q][d];
+        }
+    }
+    // those, each by its cell's lane (inside the loop above, the global path took
+    // half its code and a quarter of its registers: 104 for 78)
+    uint64_t miss = ((uint64_t)s_miss[tid][1] << 32) | s_miss[tid][0];
+    while (miss) {
+        const int k = __builtin_ctzll(miss);
+        miss &= miss - 1;
+        int J[D];
+        J[0] = w[0] + lane % N0;
+        J[1] = w[1] + lane / N0;
+        if constexpr (D == 3) J[2] = w[2];
+        CellMap<D> cm;
+        cell_map<D, STD>(m, J, cm);
+        const uint64_t e = at((k << 6) | lane);
+        float u[D], out[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) u[d] = base[d][e];
+        advect_split_one<D, M>(GlobalVelocity<D>{V, sc, J, cm}, P, u, out);
+#pragma unroll
+        for (int d = 0; d < D; ++d) base[d][e] = out[d];
     }
 }
 
