@@ -240,6 +240,52 @@ __device__ inline uint64_t active_slots_in(const uint8_t* __restrict__ index, in
     return bits;
 }
 
+// ---- grid to particles: a thread takes kSlots8 slots of its cell (grid2particle_flip!,
+// with more values per slot, half of them)
+constexpr int kSlots8 = 8;
+
+// The positions (or any D arrays) of slots kb.. of cell c, those of a slot plane
+// in which the wavefront has an active slot: unguarded but for that (uniform), so
+// that they are all in flight together; other planes cost no bandwidth.  `on`: the
+// cell's active slots, bit j slot kb + j.
+template <int D, int N, class P, typename T>
+__device__ inline void load_slots(const P& a, int64_t c, int64_t C, int kb, uint32_t on,
+                                  T (&p)[N][D]) {
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) p[j][d] = T(0);
+        if (__ballot((on >> j) & 1)) {
+            const int64_t e = c + C * (kb + j);
+#pragma unroll
+            for (int d = 0; d < D; ++d) p[j][d] = a.p[d][e];
+        }
+    }
+}
+
+// The nodal values at the corners of cell I.
+template <int D>
+__device__ inline void cell_corners(const Grid<D>& g, const double* __restrict__ F,
+                                    const int64_t (&I)[D], double (&v)[1 << D]) {
+    const int64_t n0 = g.ni[0] + 1, n1 = g.ni[1] + 1;
+    const int64_t b = I[0] + n0 * (I[1] + (D == 3 ? n1 * I[D - 1] : 0));
+#pragma unroll
+    for (int q = 0; q < (1 << D); ++q)
+        v[q] = F[b + (q & 1) + n0 * (((q >> 1) & 1) + n1 * ((q >> 2) & 1))];
+}
+
+// lerp(v, t) of src/Interpolations/ndlerp.jl:11-15
+template <int D>
+__device__ inline double lerp_cell(const double (&v)[1 << D], const double (&t)[D]) {
+    const double lo = lerp1(t[1], lerp1(t[0], v[0], v[1]), lerp1(t[0], v[2], v[3]));
+    if constexpr (D == 2) {
+        return lo;
+    } else {
+        const double hi = lerp1(t[1], lerp1(t[0], v[4], v[5]), lerp1(t[0], v[6], v[7]));
+        return lerp1(t[2], lo, hi);
+    }
+}
+
 // Minimum over the wavefront by data-parallel-primitive shifts (no LDS round
 // trips): within rows of 16 lanes, then across the rows; lane 63 holds it.
 __device__ inline uint32_t wave_min(uint32_t v) {

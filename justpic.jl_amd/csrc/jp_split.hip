@@ -557,23 +557,19 @@ __global__ void __launch_bounds__(kBlock) k_g2p_split(Grid<D> g, double* __restr
                                                       const uint8_t* __restrict__ index) {
     int64_t c, I[D];
     if (!row_cell<D>(g, c, I)) return;
-    const int64_t e = c + g.C * (int64_t)blockIdx.y;
-    if (!index[e]) return;
-    double t[D];
+    const int kb = (int)blockIdx.y * kSlots8, ke = kb + kSlots8 < g.K ? kb + kSlots8 : g.K;
+    double v[1 << D];
+    cell_corners<D>(g, F, I, v);
+    const uint32_t on = (uint32_t)(active_slots_in(index, c, g.C, kb, ke) >> kb);
+    float u[kSlots8][D];
+    load_slots<D, kSlots8>(off, c, g.C, kb, on, u);
 #pragma unroll
-    for (int d = 0; d < D; ++d) t[d] = (double)off.p[d][e];
-    const int64_t n0 = g.ni[0] + 1;
-    if constexpr (D == 2) {
-        const int64_t b = I[0] + n0 * I[1];
-        Fp[e] = lerp1(t[1], lerp1(t[0], F[b], F[b + 1]), lerp1(t[0], F[b + n0], F[b + n0 + 1]));
-    } else {
-        const int64_t n1 = g.ni[1] + 1, s = n0 * n1;
-        const int64_t b = I[0] + n0 * (I[1] + n1 * I[2]);
-        const double lo =
-            lerp1(t[1], lerp1(t[0], F[b], F[b + 1]), lerp1(t[0], F[b + n0], F[b + n0 + 1]));
-        const double hi = lerp1(t[1], lerp1(t[0], F[b + s], F[b + s + 1]),
-                                lerp1(t[0], F[b + s + n0], F[b + s + n0 + 1]));
-        Fp[e] = lerp1(t[2], lo, hi);
+    for (int j = 0; j < kSlots8; ++j) {
+        if (!((on >> j) & 1)) continue;
+        double t[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) t[d] = (double)u[j][d];
+        Fp[c + g.C * (kb + j)] = lerp_cell<D>(v, t);
     }
 }
 
@@ -897,7 +893,7 @@ template <int D>
 int run_g2p(jp_ctx* ctx, const jp_cellgrid* gc, double* Fp, const double* F, float* const* off,
             const uint8_t* index) {
     Grid<D> G = to_grid<D>(gc);
-    dim3 grid((unsigned)row_blocks<D>(G), (unsigned)G.K);
+    const dim3 grid((unsigned)row_blocks<D>(G), (unsigned)((G.K + kSlots8 - 1) / kSlots8));
     k_g2p_split<D><<<grid, kBlock, 0, ctx->stream>>>(G, Fp, F, fptr3<D>(off), index);
     JP_LAUNCHED(ctx);
     return finish(ctx);

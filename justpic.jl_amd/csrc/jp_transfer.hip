@@ -58,9 +58,12 @@ __global__ void __launch_bounds__(kBlock) k_min_spacing(Grid<D> g, double* __res
     }
 }
 
-// grid2particle_flip! (src/Interpolations/grid_to_particle.jl:125-207): one
-// thread per slot (row mapping); F_pic and F0_pic at the same t, F_flip =
-// Fp + (F_pic - F0_pic), Fp = muladd(F_pic, α, F_flip * (1 - α))
+// grid2particle_flip! (src/Interpolations/grid_to_particle.jl:125-207): a thread
+// takes 4 slots of its cell (row mapping); F_pic and F0_pic at the same t, F_flip =
+// Fp + (F_pic - F0_pic), Fp = muladd(F_pic, α, F_flip * (1 - α)).  512 x 384 cells of
+// 48 slots: a thread per slot 104 us (the corners of two fields and a division for
+// each), 8 slots 126 (176 registers), 4 slots 87.
+constexpr int kSlotsFlip = 4;
 template <int D>
 __global__ void __launch_bounds__(kBlock) k_g2p_flip(Grid<D> g, int nf, ArgPtrs Fp, FieldPtrs F,
                                                      FieldPtrs F0, CPtr3 coords,
@@ -69,23 +72,37 @@ __global__ void __launch_bounds__(kBlock) k_g2p_flip(Grid<D> g, int nf, ArgPtrs 
                                                      const double* __restrict__ h) {
     int64_t c, I[D];
     if (!row_cell<D>(g, c, I)) return;
-    const int64_t e = c + g.C * (int64_t)blockIdx.y;
-    if (!index[e]) return;
-    int64_t nn[D], k[D];
-    double t[D];
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-        nn[d] = g.ni[d] + 1;
-        k[d] = I[d];
-        t[d] = (coords.p[d][e] - g.xv[d].x[I[d]]) * (1.0 / h[d]);
-    }
+    const int kb = (int)blockIdx.y * kSlotsFlip, ke = kb + kSlotsFlip < g.K ? kb + kSlotsFlip : g.K;
+    const uint32_t on = (uint32_t)(active_slots_in(index, c, g.C, kb, ke) >> kb);
+    if (!__ballot(on != 0)) return;
+    double t[kSlotsFlip][D];
+    load_slots<D, kSlotsFlip>(coords, c, g.C, kb, on, t);
     const double om = 1.0 - alpha;
     for (int f = 0; f < nf; ++f) {
-        const double Fpic = lerp_corners<D>(F.p[f], nn, k, t);
-        const double F0pic = lerp_corners<D>(F0.p[f], nn, k, t);
-        const double dF = Fpic - F0pic;
-        const double Fflip = Fp.p[f][e] + dF;
-        Fp.p[f][e] = fma(Fpic, alpha, Fflip * om);
+        struct {
+            double* p[1];
+        } a{{Fp.p[f]}};
+        double v[1 << D], v0[1 << D], q[kSlotsFlip][1];
+        cell_corners<D>(g, F.p[f], I, v);
+        cell_corners<D>(g, F0.p[f], I, v0);
+        load_slots<1, kSlotsFlip>(a, c, g.C, kb, on, q);
+        if (f == 0) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                const double x = g.xv[d].x[I[d]], ih = 1.0 / h[d];
+#pragma unroll
+                for (int j = 0; j < kSlotsFlip; ++j) t[j][d] = (t[j][d] - x) * ih;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < kSlotsFlip; ++j) {
+            if (!((on >> j) & 1)) continue;
+            const double Fpic = lerp_cell<D>(v, t[j]);
+            const double F0pic = lerp_cell<D>(v0, t[j]);
+            const double dF = Fpic - F0pic;
+            const double Fflip = q[j][0] + dF;
+            a.p[0][c + g.C * (kb + j)] = fma(Fpic, alpha, Fflip * om);
+        }
     }
 }
 
@@ -111,34 +128,54 @@ __global__ void __launch_bounds__(kBlock) k_p2c(Grid<D> g, CAxes<D> xc, int nf, 
         inv[d] = g.xv[d].idx[I[d]];
     }
     for (int f = 0; f < nf; ++f) wF[f] = 0.0;
-    for (int ip = 0; ip < g.K; ++ip) {
-        const int64_t e = c + g.C * ip;
-        double p[D];
+    // 8 slots at a time, their loads in flight together (unguarded: an empty slot's
+    // values are not used; slot by slot, 512 x 384 cells of 48 took 58 us for 35)
+    constexpr int B = 8;
+    for (int k0 = 0; k0 < g.K; k0 += B) {
+        int64_t e[B];
+        double p[B][D], f0[B], wi[B];
 #pragma unroll
-        for (int d = 0; d < D; ++d) p[d] = coords.p[d][e];
-        bool skip = p[0] != p[0];
-        if (!first_only)
+        for (int j = 0; j < B; ++j) {
+            e[j] = c + g.C * (k0 + j < g.K ? k0 + j : g.K - 1);
 #pragma unroll
-            for (int d = 1; d < D; ++d) skip = skip || (p[d] != p[d]);
-        if (skip) continue;
-        double wi;
-        if (dist) {
-            double a = m[0] - p[0];
-            double s = a * a;
-#pragma unroll
-            for (int d = 1; d < D; ++d) {
-                const double b = m[d] - p[d];
-                s = s + b * b;
-            }
-            const double dd = sqrt(s);
-            wi = 1.0 / (dd * dd);
-        } else {
-            wi = 1.0;
-#pragma unroll
-            for (int d = 0; d < D; ++d) wi = wi * fma(-fabs(m[d] - p[d]), inv[d], 1.0);
+            for (int d = 0; d < D; ++d) p[j][d] = coords.p[d][e[j]];
+            f0[j] = Fp.p[0][e[j]];
         }
-        w += wi;
-        for (int f = 0; f < nf; ++f) wF[f] = fma(wi, Fp.p[f][e], wF[f]);
+        uint32_t on = 0;
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            bool skip = k0 + j >= g.K || p[j][0] != p[j][0];
+            if (!first_only)
+#pragma unroll
+                for (int d = 1; d < D; ++d) skip = skip || (p[j][d] != p[j][d]);
+            if (dist) {
+                double a = m[0] - p[j][0];
+                double s = a * a;
+#pragma unroll
+                for (int d = 1; d < D; ++d) {
+                    const double b = m[d] - p[j][d];
+                    s = s + b * b;
+                }
+                const double dd = sqrt(s);
+                wi[j] = 1.0 / (dd * dd);
+            } else {
+                wi[j] = 1.0;
+#pragma unroll
+                for (int d = 0; d < D; ++d)
+                    wi[j] = wi[j] * fma(-fabs(m[d] - p[j][d]), inv[d], 1.0);
+            }
+            on |= (skip ? 0u : 1u) << j;
+            w = skip ? w : w + wi[j];
+            wF[0] = skip ? wF[0] : fma(wi[j], f0[j], wF[0]);
+        }
+        for (int f = 1; f < nf; ++f) {
+            double v[B];
+#pragma unroll
+            for (int j = 0; j < B; ++j) v[j] = Fp.p[f][e[j]];
+#pragma unroll
+            for (int j = 0; j < B; ++j)
+                if ((on >> j) & 1) wF[f] = fma(wi[j], v[j], wF[f]);
+        }
     }
     if (D == 2 && !tuple) {
         F.p[0][c] = wF[0] / w;
@@ -148,34 +185,56 @@ __global__ void __launch_bounds__(kBlock) k_p2c(Grid<D> g, CAxes<D> xc, int nf, 
     }
 }
 
-// centroid2particle! (src/Interpolations/centroid_to_particle.jl:15-76): one
-// thread per slot; shifted_index against xci[I], clamped to 1..ni-1
-// (1-based), lerp of the centred field's corners
+// centroid2particle! (src/Interpolations/centroid_to_particle.jl:15-76): a thread
+// takes 8 slots of its cell; shifted_index against xci[I], clamped to 1..ni-1
+// (1-based), lerp of the centred field's corners (512 x 384 cells of 48 slots: a
+// thread per slot 67 us, 51)
 template <int D>
 __global__ void __launch_bounds__(kBlock) k_c2p(Grid<D> g, CAxes<D> xc, int nf, ArgPtrs Fp,
                                                 FieldPtrs F, CPtr3 coords) {
     int64_t c, I[D];
     if (!row_cell<D>(g, c, I)) return;
-    const int64_t e = c + g.C * (int64_t)blockIdx.y;
-    double p[D];
-    bool nan = false;
+    const int kb = (int)blockIdx.y * kSlots8;
+    double p[kSlots8][D];
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
-        p[d] = coords.p[d][e];
-        nan = nan || (p[d] != p[d]);
+    for (int j = 0; j < kSlots8; ++j) {
+        const int64_t e = c + g.C * (kb + j < g.K ? kb + j : g.K - 1);
+#pragma unroll
+        for (int d = 0; d < D; ++d) p[j][d] = coords.p[d][e];
     }
-    if (nan) return;
-    int64_t nn[D], k[D];
-    double t[D];
+    // the two intervals a particle can lie in: below (k[d][0]) and above its
+    // cell's centre
+    int64_t nn[D], k[D][2];
+    double m[D], x[D][2], ix[D][2];
 #pragma unroll
     for (int d = 0; d < D; ++d) {
         nn[d] = g.ni[d];
-        int64_t kk = p[d] < xc.a[d].x[I[d]] ? I[d] - 1 : I[d];
-        kk = kk > g.ni[d] - 2 ? g.ni[d] - 2 : (kk < 0 ? 0 : kk);
-        k[d] = kk;
-        t[d] = (p[d] - xc.a[d].x[kk]) * xc.a[d].idx[kk];
+        m[d] = xc.a[d].x[I[d]];
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+            const int64_t kk = I[d] - 1 + s;
+            k[d][s] = kk > g.ni[d] - 2 ? g.ni[d] - 2 : (kk < 0 ? 0 : kk);
+            x[d][s] = xc.a[d].x[k[d][s]];
+            ix[d][s] = xc.a[d].idx[k[d][s]];
+        }
     }
-    for (int f = 0; f < nf; ++f) Fp.p[f][e] = lerp_corners<D>(F.p[f], nn, k, t);
+#pragma unroll
+    for (int j = 0; j < kSlots8; ++j) {
+        bool nan = kb + j >= g.K;
+#pragma unroll
+        for (int d = 0; d < D; ++d) nan = nan || p[j][d] != p[j][d];
+        if (nan) continue;
+        int64_t kk[D];
+        double t[D];
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            const bool lo = p[j][d] < m[d];
+            kk[d] = lo ? k[d][0] : k[d][1];
+            t[d] = (p[j][d] - (lo ? x[d][0] : x[d][1])) * (lo ? ix[d][0] : ix[d][1]);
+        }
+        for (int f = 0; f < nf; ++f)
+            Fp.p[f][c + g.C * (kb + j)] = lerp_corners<D>(F.p[f], nn, kk, t);
+    }
 }
 
 template <int D>
@@ -226,7 +285,7 @@ int run_flip(jp_ctx* ctx, const jp_cellgrid* gc, int nf, double* const* Fp, cons
     double* h = reinterpret_cast<double*>(static_cast<char*>(ctx->dsmall) + 2048);
     k_min_spacing<D><<<1, kBlock, 0, ctx->stream>>>(G, h);
     JP_LAUNCHED(ctx);
-    const dim3 grid((unsigned)row_blocks<D>(G), (unsigned)G.K);
+    const dim3 grid((unsigned)row_blocks<D>(G), (unsigned)((G.K + kSlotsFlip - 1) / kSlotsFlip));
     k_g2p_flip<D><<<grid, kBlock, 0, ctx->stream>>>(G, nf, argptrs(Fp, nf), fieldptrs(F, nf),
                                                     fieldptrs(F0, nf), cptr3(coords, D), index,
                                                     alpha, h);
@@ -292,11 +351,11 @@ int jp_centroid2particle(jp_ctx* ctx, const jp_cellgrid* g, const jp_axis* xc, i
     if ((rc = check_arrays(ctx, nfields, (const void* const*)Fp, "Fp"))) return rc;
     if (g->ndim == 2) {
         Grid<2> G = to_grid<2>(g);
-        k_c2p<2><<<dim3((unsigned)row_blocks<2>(G), (unsigned)G.K), kBlock, 0, ctx->stream>>>(
+        k_c2p<2><<<dim3((unsigned)row_blocks<2>(G), (unsigned)((G.K + kSlots8 - 1) / kSlots8)), kBlock, 0, ctx->stream>>>(
             G, caxes<2>(xc), nfields, argptrs(Fp, nfields), fieldptrs(F, nfields), cptr3(coords, 2));
     } else {
         Grid<3> G = to_grid<3>(g);
-        k_c2p<3><<<dim3((unsigned)row_blocks<3>(G), (unsigned)G.K), kBlock, 0, ctx->stream>>>(
+        k_c2p<3><<<dim3((unsigned)row_blocks<3>(G), (unsigned)((G.K + kSlots8 - 1) / kSlots8)), kBlock, 0, ctx->stream>>>(
             G, caxes<3>(xc), nfields, argptrs(Fp, nfields), fieldptrs(F, nfields), cptr3(coords, 3));
     }
     JP_LAUNCHED(ctx);
