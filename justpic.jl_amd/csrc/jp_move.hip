@@ -700,279 +700,6 @@ __global__ void __launch_bounds__(BS) k_mv_phase(Grid<D> g, MoveScratch ms, Off3
     }
 }
 
-// ------------------------------------------------------------ 2'. 2D phases in tiles
-// All nine colour phases of the 2D move in one launch.  A workgroup owns a
-// tile of cells and replays the phases on the occupancy, pending, arrival and
-// touched words of the tile plus a halo, all in LDS, with a barrier between
-// phases; it keeps the results of its own cells.
-//
-// The halo is the dependency cone of the phases.  The processing of cell A in
-// phase p reads and writes the words of A's 3x3 neighbourhood, so it depends
-// on the processings, in earlier phases, of the cells B within 2 of A (their
-// neighbourhoods overlap A's), and on theirs in turn.  A step from A to B
-// moves, per dimension, by a multiple of 3 plus the difference of their
-// colours, within [-2, 2]; taking the phases down from p, the offsets that can
-// be reached lie in lo_p..hi_p with, for phase p = 3 c0 + c1 (c0 = I0 mod 3,
-// the outer digit of the phase, c1 = I1 mod 3):
-//   dimension 0: -c0 .. 2 c0,  dimension 1: -p .. 2 p.
-// A processing is exact here when A + [lo_p - 1, hi_p + 1] lies inside the
-// region (or leaves the grid there), and a processing that changes an exact
-// one is itself exact, so only those run.  The final words of an owned cell
-// come from the processings of its 3x3 neighbourhood, so the region is the
-// tile widened by the largest cone plus 2: 4 cells below and 6 above in
-// dimension 0, 10 below and 18 above in dimension 1.
-//
-// Tiles overlap, so a halo processing also runs in the tile that owns it;
-// both compute the same slots from the same exact inputs.  Origins, counts and
-// final words come from owned cells only.  (An arrival that is re-slotted has
-// its origin read again, but stays in its cell: in a cell of another tile
-// neither the read nor the store matters.)
-//
-// A pending slot that holds an arrival of this call is always re-slotted in
-// its own cell (an arrival that fails the strict test of its new cell, or a
-// particle re-slotted higher in its own cell), so the destination code of
-// such a slot is the centre and the code words are read-only here.
-constexpr int kTileHalo0Lo = 4, kTileHalo0Hi = 6, kTileHalo1Lo = 10, kTileHalo1Hi = 18;
-
-__device__ inline int cone_lo(int p, int d) { return d == 0 ? -(p / 3) : -p; }
-__device__ inline int cone_hi(int p, int d) { return d == 0 ? 2 * (p / 3) : 2 * p; }
-
-template <int TX, int TY, int BS, bool STATS>
-__global__ void __launch_bounds__(BS) k_mv_tiles2(Grid<2> g, MoveScratch ms,
-                                                  const int* __restrict__ flag, jp_stats* st) {
-    constexpr int RX = TX + kTileHalo0Lo + kTileHalo0Hi;
-    constexpr int RY = TY + kTileHalo1Lo + kTileHalo1Hi;
-    constexpr int R = RX * RY;
-    static_assert(((RX + 2) / 3) * ((RY + 2) / 3) <= BS, "one cell per thread and phase");
-    static_assert(RX == kPitch2, "the codes' row pitch");
-    __shared__ NbEntry s_nb[R];
-    __shared__ uint64_t s_gap[R];
-    __shared__ uint32_t s_code[BS * kRow / 4];
-    if (*flag) return;  // far jump or rejected grid: nothing moves here
-    const int n0 = (int)g.ni[0], n1 = (int)g.ni[1];
-    const int ntx = (n0 + TX - 1) / TX;
-    // neighbouring tiles read each other's halo words: consecutive tiles of
-    // a row on one XCD
-    const int tile = (int)xcd_block(blockIdx.x, gridDim.x);
-    const int tx0 = (tile % ntx) * TX, ty0 = (tile / ntx) * TY;
-    const int tx1 = (tx0 + TX < n0 ? tx0 + TX : n0) - 1;
-    const int ty1 = (ty0 + TY < n1 ? ty0 + TY : n1) - 1;
-    const int gx0 = tx0 - kTileHalo0Lo > 0 ? tx0 - kTileHalo0Lo : 0;
-    const int gx1 = tx1 + kTileHalo0Hi < n0 - 1 ? tx1 + kTileHalo0Hi : n0 - 1;
-    const int gy0 = ty0 - kTileHalo1Lo > 0 ? ty0 - kTileHalo1Lo : 0;
-    const int gy1 = ty1 + kTileHalo1Hi < n1 - 1 ? ty1 + kTileHalo1Hi : n1 - 1;
-    const int rw = gx1 - gx0 + 1, rh = gy1 - gy0 + 1;
-    const uint32_t K = (uint32_t)g.K;
-    const uint32_t C32 = (uint32_t)g.C;
-    const uint64_t full = K == 64 ? ~0ull : ((1ull << K) - 1);
-    for (int i = threadIdx.x; i < rw * rh; i += BS) {
-        const int x = i % rw, y = i / rw;
-        const uint32_t c = (uint32_t)(gx0 + x) + (uint32_t)n0 * (uint32_t)(gy0 + y);
-        const int r = x + RX * y;
-        const bool own = tx0 <= gx0 + x && gx0 + x <= tx1 && ty0 <= gy0 + y && gy0 + y <= ty1;
-        s_nb[r] = NbEntry{~ms.occ0[c] & full, own ? c : kNoCell, 0u};
-        s_gap[r] = ms.rar[c];  // (ms.gap: other tiles may have written theirs)
-    }
-    __syncthreads();
-    const int nw = ((int)K + 7) >> 3;
-    uint32_t* const row = s_code + threadIdx.x * (kRow / 4);
-    int n_moved = 0, n_del = 0, n_drop = 0;
-    // the colour-p cells whose processing is exact in the region: x = vx +
-    // 3i (i < cx), y = vy + 3j (j < cy); this thread's one of them
-    auto my_cell = [&](int p, int& x, int& y) {
-        const int ax = gx0 == 0 ? 0 : gx0 - cone_lo(p, 0) + 1;
-        const int bx = gx1 == n0 - 1 ? n0 - 1 : gx1 - cone_hi(p, 0) - 1;
-        const int ay = gy0 == 0 ? 0 : gy0 - cone_lo(p, 1) + 1;
-        const int by = gy1 == n1 - 1 ? n1 - 1 : gy1 - cone_hi(p, 1) - 1;
-        const int vx = ax + (p / 3 - ax % 3 + 3) % 3;
-        const int vy = ay + (p % 3 - ay % 3 + 3) % 3;
-        const int cx = vx <= bx ? (bx - vx) / 3 + 1 : 0;
-        const int cy = vy <= by ? (by - vy) / 3 + 1 : 0;
-        const int t = threadIdx.x;
-        if (t >= cx * cy) return false;
-        x = vx + 3 * (t % cx);
-        y = vy + 3 * (t / cx);
-        return true;
-    };
-    // the words and code words of a phase's cell are loaded one phase ahead,
-    // so that they are in flight during the phase before
-    uint64_t nxt[8], mov = 0, stm = 0;
-    int x = 0, y = 0;
-    auto fetch = [&](int p) {
-        const bool ok = my_cell(p, x, y);
-        if (ok) {
-            const uint32_t S32 = (uint32_t)x + (uint32_t)n0 * (uint32_t)y;
-            load_codes(ms, S32, C32, nw, nxt);
-            mov = ms.mov[S32];
-            stm = ms.stm[S32];
-        }
-        return ok;
-    };
-    bool mine = fetch(0);
-    for (int p = 0; p < kNB<2>; ++p) {
-        const int px = x, py = y;
-        const bool live = mine;
-        const uint64_t mov_p = mov, stm_p = stm;
-        if (live) put_codes(row, nxt, nw);
-        if (p + 1 < kNB<2>) mine = fetch(p + 1);
-        const int r = (px - gx0) + RX * (py - gy0);
-        uint64_t gap = live ? s_gap[r] : 0ull;
-        if (live && (mov_p | gap)) {
-            const uint32_t S32 = (uint32_t)px + (uint32_t)n0 * (uint32_t)py;
-            const int col0 = p / 3, col1 = p % 3;
-            const uint64_t gap0 = gap;
-            NbEntry* const nb0 = s_nb + (r - 1 - RX);
-            auto at = [&](uint32_t cd) -> NbEntry& { return nb0[cd]; };
-            auto later = [&](uint32_t cd, NbEntry& to, uint64_t fb) {
-                const int n = neighbour_of<2>(cd), dx = n % 3 - 1, dy = n / 3 - 1;
-                if (((col0 + dx + 3) % 3) * 3 + (col1 + dy + 3) % 3 > p)
-                    atomicOr(reinterpret_cast<unsigned long long*>(&s_gap[&to - s_nb]),
-                             (unsigned long long)fb);
-            };
-            int mv = 0, dl = 0, dr = 0;
-            run_cell<2, STATS>(mov_p, stm_p, gap, s_nb[r].free, row, at, later, ms.org, S32, C32,
-                               K, mv, dl, dr);
-            if (gap != gap0) s_gap[r] = gap;
-            if (STATS && tx0 <= px && px <= tx1 && ty0 <= py && py <= ty1) {
-                n_moved += mv;
-                n_del += dl;
-                n_drop += dr;
-            }
-        }
-        __syncthreads();
-    }
-    const int ow = tx1 - tx0 + 1, oh = ty1 - ty0 + 1;
-    for (int i = threadIdx.x; i < ow * oh; i += BS) {
-        const int cx = i % ow, cy = i / ow;
-        const uint32_t c = (uint32_t)(tx0 + cx) + (uint32_t)n0 * (uint32_t)(ty0 + cy);
-        const int r = (tx0 - gx0) + cx + RX * ((ty0 - gy0) + cy);
-        ms.occ[c] = ~s_nb[r].free & full;
-        if (s_gap[r]) ms.gap[c] = s_gap[r];
-    }
-    if (STATS) {
-        stat_add(st, ST_MOVED, n_moved);
-        stat_add(st, ST_DELETED, n_del);
-        stat_add(st, ST_DROPPED, n_drop);
-    }
-}
-
-// ------------------------------------------------------------ 3. scatter
-// T: coordinate type (double: FP64 drop-in, float: split offsets)
-template <int D, typename T>
-struct TPtr3 {
-    T* p[3];
-};
-
-// REC16: 2D split with one field (16-byte records, one load per arrival)
-template <int D, typename T, bool REC16 = false>
-__global__ void __launch_bounds__(kBlock) k_mv_scatter(Grid<D> g, TPtr3<D, T> coords,
-                                                       uint8_t* __restrict__ index, int nargs,
-                                                       ArgPtrs args, MoveScratch ms,
-                                                       const SplitGeom* __restrict__ geo,
-                                                       int span) {
-    // one thread per cell and slot group (blockIdx.y, `span` slots), chunks of
-    // 8 slot planes in lockstep across the wavefront (coalesced origin loads
-    // and final stores); only the reads of the staged data are scattered.
-    // Arrivals copy their staged data, vacated slots are emptied
-    // (empty_particle!, src/Particles/move_safe.jl:243-251).  Nothing moves
-    // when the split grid was rejected (geo: null in the FP64 form).
-    if (geo && geo->bad) return;
-    // 2D: XCD-contiguous cell ranges (a destination's sources are its
-    // neighbour cells, whose staged lines other threads of the same L2 also
-    // read; a row of cells above or below is only a few workgroups away, which
-    // round-robin dealing puts on other XCDs); slot groups of one cell block
-    // stay together.  3D keeps the dealt order: there the plane above or below
-    // is a multiple of 8 workgroups away, already on the same XCD, and the
-    // renumbering measured slower.
-    const unsigned lb = D == 2 ? xcd_block(blockIdx.x + gridDim.x * blockIdx.y,
-                                           gridDim.x * gridDim.y)
-                               : blockIdx.x * gridDim.y + blockIdx.y;
-    const int64_t c = (lb / gridDim.y) * (int64_t)blockDim.x + threadIdx.x;
-    if (c >= g.C) return;
-    const int kb = (int)(lb % gridDim.y) * span;
-    const int ke = kb + span < g.K ? kb + span : g.K;
-    const int64_t C = g.C;
-    // the first chunk's origins go out with the cell's words: unguarded loads
-    // (slot clamped to K - 1, values used for arrivals only), one round trip
-    // fewer than loading them after the arrival bits are known
-    uint16_t o0[8];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int k = kb + j < g.K ? kb + j : g.K - 1;
-        o0[j] = ms.org[org_at<D>((uint32_t)c, (uint32_t)k, (uint32_t)C, (uint32_t)g.K)];
-    }
-    const uint64_t occ = ms.occ[c], occ0 = ms.occ0[c], gap = ms.gap[c];
-    const uint64_t arr = arrivals(occ, occ0, ms.mov[c]);
-    const uint64_t work = arr | (~occ & (occ0 | gap));  // arrivals, emptied slots
-    if (!(work >> kb)) return;
-    const int str1 = (int)g.ni[0], str2 = (int)(g.ni[0] * g.ni[1]);
-    for (int k0 = kb; k0 < ke; k0 += 8) {
-        const uint32_t wb = (uint32_t)(work >> k0) & 0xFFu;
-        if (!wb) continue;
-        const uint32_t ab = (uint32_t)(arr >> k0) & 0xFFu;
-        uint32_t o[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const uint32_t at = org_at<D>((uint32_t)c, (uint32_t)(k0 + j), (uint32_t)C,
-                                          (uint32_t)g.K);
-            o[j] = k0 == kb ? (uint32_t)o0[j] : ((ab >> j) & 1) ? (uint32_t)ms.org[at] : 0u;
-        }
-        // the record numbers: of the source cell, its rank-th
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const uint32_t src = (uint32_t)c - (uint32_t)move_offset<D>((o[j] >> 6) & 0x7Fu, str1,
-                                                                        str2);
-            if (((ab >> j) & 1) && o[j] == kOrgFar)
-                o[j] = ms.orgf[org_at<D>((uint32_t)c, (uint32_t)(k0 + j), (uint32_t)C,
-                                         (uint32_t)g.K)];
-            else
-                o[j] = src * (uint32_t)g.K + (o[j] & 63u);
-        }
-        if constexpr (REC16) {
-            float u0[8], u1[8];
-            double fv[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                u0[j] = u1[j] = __builtin_nanf("");
-                fv[j] = dnan();
-                if ((ab >> j) & 1) stg_get16(ms, o[j], u0[j], u1[j], fv[j]);
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                if (!((wb >> j) & 1)) continue;
-                const int64_t e = c + C * (k0 + j);
-                coords.p[0][e] = (T)u0[j];
-                coords.p[D - 1][e] = (T)u1[j];
-                index[e] = (uint8_t)((ab >> j) & 1);
-                args.p[0][e] = fv[j];
-            }
-            continue;
-        }
-        T v[8][D];
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-#pragma unroll
-            for (int d = 0; d < D; ++d)
-                v[j][d] = ((ab >> j) & 1) ? stg_coord<D, T>(ms, o[j], d) : (T)dnan();
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            if (!((wb >> j) & 1)) continue;
-            const int64_t e = c + C * (k0 + j);
-#pragma unroll
-            for (int d = 0; d < D; ++d) coords.p[d][e] = v[j][d];
-            index[e] = (uint8_t)((ab >> j) & 1);
-        }
-        for (int a = 0; a < nargs; ++a) {
-            double av[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) av[j] = ((ab >> j) & 1) ? stg_field<D>(ms, o[j], a) : dnan();
-#pragma unroll
-            for (int j = 0; j < 8; ++j)
-                if ((wb >> j) & 1) args.p[a][c + C * (k0 + j)] = av[j];
-        }
-    }
-}
-
 // ------------------------------------------------------------ far jumps
 // The colour phases when some particle jumps more than one cell (flag[0] has
 // kFlagFar, flag[1] holds the largest jump R in cells), in one workgroup on
@@ -1166,19 +893,11 @@ __device__ inline void far_cell(const Grid<D>& g, const MoveScratch& ms, const i
     if (again & ~pend0) ms.gap[S] = gapS | again;
 }
 
+// (R: the largest jump; called by the whole workgroup of kFarBlock threads)
 template <int D, typename T>
-__global__ void __launch_bounds__(kFarBlock) k_mv_far(Grid<D> g, MoveScratch ms,
-                                                      int* __restrict__ flag, jp_stats* st) {
-    __shared__ NbEntry s_nb[kNB<D>][kFarBlock];
-    __shared__ uint32_t s_code[kFarBlock * kRow / 4];
-    const int fl = flag[0];
-    if (!fl) return;
-    const int R = flag[1];
-    __syncthreads();  // every thread has read the words before they are cleared
-    if (!(fl & kFlagFar) || (fl & kFlagRejected)) {
-        if (threadIdx.x == 0) flag[0] = flag[1] = 0;
-        return;
-    }
+__device__ inline void far_phases(const Grid<D>& g, const MoveScratch& ms, int R,
+                                  NbEntry (&s_nb)[kNB<D>][kFarBlock],
+                                  uint32_t (&s_code)[kFarBlock * kRow / 4], jp_stats* st) {
     int64_t ncol[D], m[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) ncol[d] = (g.ni[d] + 2) / 3;
@@ -1232,7 +951,308 @@ __global__ void __launch_bounds__(kFarBlock) k_mv_far(Grid<D> g, MoveScratch ms,
     stat_add(st, ST_DELETED, n_del);
     stat_add(st, ST_DROPPED, n_drop);
     stat_add(st, ST_FAR, n_far);
-    if (threadIdx.x == 0) flag[0] = flag[1] = 0;  // ready for the next move
+}
+
+template <int D, typename T>
+__global__ void __launch_bounds__(kFarBlock) k_mv_far(Grid<D> g, MoveScratch ms,
+                                                      const int* __restrict__ flag,
+                                                      jp_stats* st) {
+    __shared__ NbEntry s_nb[kNB<D>][kFarBlock];
+    __shared__ uint32_t s_code[kFarBlock * kRow / 4];
+    const int fl = flag[0];
+    if (!(fl & kFlagFar) || (fl & kFlagRejected)) return;
+    far_phases<D, T>(g, ms, flag[1], s_nb, s_code, st);
+}
+
+// ------------------------------------------------------------ 2'. 2D phases in tiles
+// All nine colour phases of the 2D move in one launch.  A workgroup owns a
+// tile of cells and replays the phases on the occupancy, pending, arrival and
+// touched words of the tile plus a halo, all in LDS, with a barrier between
+// phases; it keeps the results of its own cells.
+//
+// The halo is the dependency cone of the phases.  The processing of cell A in
+// phase p reads and writes the words of A's 3x3 neighbourhood, so it depends
+// on the processings, in earlier phases, of the cells B within 2 of A (their
+// neighbourhoods overlap A's), and on theirs in turn.  A step from A to B
+// moves, per dimension, by a multiple of 3 plus the difference of their
+// colours, within [-2, 2]; taking the phases down from p, the offsets that can
+// be reached lie in lo_p..hi_p with, for phase p = 3 c0 + c1 (c0 = I0 mod 3,
+// the outer digit of the phase, c1 = I1 mod 3):
+//   dimension 0: -c0 .. 2 c0,  dimension 1: -p .. 2 p.
+// A processing is exact here when A + [lo_p - 1, hi_p + 1] lies inside the
+// region (or leaves the grid there), and a processing that changes an exact
+// one is itself exact, so only those run.  The final words of an owned cell
+// come from the processings of its 3x3 neighbourhood, so the region is the
+// tile widened by the largest cone plus 2: 4 cells below and 6 above in
+// dimension 0, 10 below and 18 above in dimension 1.
+//
+// Tiles overlap, so a halo processing also runs in the tile that owns it;
+// both compute the same slots from the same exact inputs.  Origins, counts and
+// final words come from owned cells only.  (An arrival that is re-slotted has
+// its origin read again, but stays in its cell: in a cell of another tile
+// neither the read nor the store matters.)
+//
+// A pending slot that holds an arrival of this call is always re-slotted in
+// its own cell (an arrival that fails the strict test of its new cell, or a
+// particle re-slotted higher in its own cell), so the destination code of
+// such a slot is the centre and the code words are read-only here.
+constexpr int kTileHalo0Lo = 4, kTileHalo0Hi = 6, kTileHalo1Lo = 10, kTileHalo1Hi = 18;
+
+__device__ inline int cone_lo(int p, int d) { return d == 0 ? -(p / 3) : -p; }
+__device__ inline int cone_hi(int p, int d) { return d == 0 ? 2 * (p / 3) : 2 * p; }
+
+// With a far jump one workgroup takes the far-jump path instead (a launch of its own
+// for it, which nearly always returned at once, took 4.5 us of every move).
+template <int TX, int TY, int BS, bool STATS, typename T>
+__global__ void __launch_bounds__(BS) k_mv_tiles2(Grid<2> g, MoveScratch ms,
+                                                  const int* __restrict__ flag, jp_stats* st) {
+    constexpr int RX = TX + kTileHalo0Lo + kTileHalo0Hi;
+    constexpr int RY = TY + kTileHalo1Lo + kTileHalo1Hi;
+    constexpr int R = RX * RY;
+    static_assert(((RX + 2) / 3) * ((RY + 2) / 3) <= BS, "one cell per thread and phase");
+    static_assert(RX == kPitch2, "the codes' row pitch");
+    static_assert(BS == kFarBlock, "the far-jump path's workgroup");
+    union Entries {  // of the region, or of the far-jump path's cells
+        struct {
+            NbEntry nb[R];
+            uint64_t gap[R];
+        } tile;
+        NbEntry far[kNB<2>][kFarBlock];
+    };
+    __shared__ __attribute__((aligned(16))) char s_raw[sizeof(Entries)];
+    __shared__ uint32_t s_code[BS * kRow / 4];
+    Entries& s_e = *reinterpret_cast<Entries*>(s_raw);
+    if (*flag) {  // far jump or rejected grid
+        if (blockIdx.x == 0 && (flag[0] & kFlagFar) && !(flag[0] & kFlagRejected))
+            far_phases<2, T>(g, ms, flag[1], s_e.far, s_code, st);
+        return;
+    }
+    NbEntry(&s_nb)[R] = s_e.tile.nb;
+    uint64_t(&s_gap)[R] = s_e.tile.gap;
+    const int n0 = (int)g.ni[0], n1 = (int)g.ni[1];
+    const int ntx = (n0 + TX - 1) / TX;
+    // neighbouring tiles read each other's halo words: consecutive tiles of
+    // a row on one XCD
+    const int tile = (int)xcd_block(blockIdx.x, gridDim.x);
+    const int tx0 = (tile % ntx) * TX, ty0 = (tile / ntx) * TY;
+    const int tx1 = (tx0 + TX < n0 ? tx0 + TX : n0) - 1;
+    const int ty1 = (ty0 + TY < n1 ? ty0 + TY : n1) - 1;
+    const int gx0 = tx0 - kTileHalo0Lo > 0 ? tx0 - kTileHalo0Lo : 0;
+    const int gx1 = tx1 + kTileHalo0Hi < n0 - 1 ? tx1 + kTileHalo0Hi : n0 - 1;
+    const int gy0 = ty0 - kTileHalo1Lo > 0 ? ty0 - kTileHalo1Lo : 0;
+    const int gy1 = ty1 + kTileHalo1Hi < n1 - 1 ? ty1 + kTileHalo1Hi : n1 - 1;
+    const int rw = gx1 - gx0 + 1, rh = gy1 - gy0 + 1;
+    const uint32_t K = (uint32_t)g.K;
+    const uint32_t C32 = (uint32_t)g.C;
+    const uint64_t full = K == 64 ? ~0ull : ((1ull << K) - 1);
+    for (int i = threadIdx.x; i < rw * rh; i += BS) {
+        const int x = i % rw, y = i / rw;
+        const uint32_t c = (uint32_t)(gx0 + x) + (uint32_t)n0 * (uint32_t)(gy0 + y);
+        const int r = x + RX * y;
+        const bool own = tx0 <= gx0 + x && gx0 + x <= tx1 && ty0 <= gy0 + y && gy0 + y <= ty1;
+        s_nb[r] = NbEntry{~ms.occ0[c] & full, own ? c : kNoCell, 0u};
+        s_gap[r] = ms.rar[c];  // (ms.gap: other tiles may have written theirs)
+    }
+    __syncthreads();
+    const int nw = ((int)K + 7) >> 3;
+    uint32_t* const row = s_code + threadIdx.x * (kRow / 4);
+    int n_moved = 0, n_del = 0, n_drop = 0;
+    // the colour-p cells whose processing is exact in the region: x = vx +
+    // 3i (i < cx), y = vy + 3j (j < cy); this thread's one of them
+    auto my_cell = [&](int p, int& x, int& y) {
+        const int ax = gx0 == 0 ? 0 : gx0 - cone_lo(p, 0) + 1;
+        const int bx = gx1 == n0 - 1 ? n0 - 1 : gx1 - cone_hi(p, 0) - 1;
+        const int ay = gy0 == 0 ? 0 : gy0 - cone_lo(p, 1) + 1;
+        const int by = gy1 == n1 - 1 ? n1 - 1 : gy1 - cone_hi(p, 1) - 1;
+        const int vx = ax + (p / 3 - ax % 3 + 3) % 3;
+        const int vy = ay + (p % 3 - ay % 3 + 3) % 3;
+        const int cx = vx <= bx ? (bx - vx) / 3 + 1 : 0;
+        const int cy = vy <= by ? (by - vy) / 3 + 1 : 0;
+        const int t = threadIdx.x;
+        if (t >= cx * cy) return false;
+        x = vx + 3 * (t % cx);
+        y = vy + 3 * (t / cx);
+        return true;
+    };
+    // the words and code words of a phase's cell are loaded one phase ahead,
+    // so that they are in flight during the phase before
+    uint64_t nxt[8], mov = 0, stm = 0;
+    int x = 0, y = 0;
+    auto fetch = [&](int p) {
+        const bool ok = my_cell(p, x, y);
+        if (ok) {
+            const uint32_t S32 = (uint32_t)x + (uint32_t)n0 * (uint32_t)y;
+            load_codes(ms, S32, C32, nw, nxt);
+            mov = ms.mov[S32];
+            stm = ms.stm[S32];
+        }
+        return ok;
+    };
+    bool mine = fetch(0);
+    for (int p = 0; p < kNB<2>; ++p) {
+        const int px = x, py = y;
+        const bool live = mine;
+        const uint64_t mov_p = mov, stm_p = stm;
+        if (live) put_codes(row, nxt, nw);
+        if (p + 1 < kNB<2>) mine = fetch(p + 1);
+        const int r = (px - gx0) + RX * (py - gy0);
+        uint64_t gap = live ? s_gap[r] : 0ull;
+        if (live && (mov_p | gap)) {
+            const uint32_t S32 = (uint32_t)px + (uint32_t)n0 * (uint32_t)py;
+            const int col0 = p / 3, col1 = p % 3;
+            const uint64_t gap0 = gap;
+            NbEntry* const nb0 = s_nb + (r - 1 - RX);
+            auto at = [&](uint32_t cd) -> NbEntry& { return nb0[cd]; };
+            auto later = [&](uint32_t cd, NbEntry& to, uint64_t fb) {
+                const int n = neighbour_of<2>(cd), dx = n % 3 - 1, dy = n / 3 - 1;
+                if (((col0 + dx + 3) % 3) * 3 + (col1 + dy + 3) % 3 > p)
+                    atomicOr(reinterpret_cast<unsigned long long*>(&s_gap[&to - s_nb]),
+                             (unsigned long long)fb);
+            };
+            int mv = 0, dl = 0, dr = 0;
+            run_cell<2, STATS>(mov_p, stm_p, gap, s_nb[r].free, row, at, later, ms.org, S32, C32,
+                               K, mv, dl, dr);
+            if (gap != gap0) s_gap[r] = gap;
+            if (STATS && tx0 <= px && px <= tx1 && ty0 <= py && py <= ty1) {
+                n_moved += mv;
+                n_del += dl;
+                n_drop += dr;
+            }
+        }
+        __syncthreads();
+    }
+    const int ow = tx1 - tx0 + 1, oh = ty1 - ty0 + 1;
+    for (int i = threadIdx.x; i < ow * oh; i += BS) {
+        const int cx = i % ow, cy = i / ow;
+        const uint32_t c = (uint32_t)(tx0 + cx) + (uint32_t)n0 * (uint32_t)(ty0 + cy);
+        const int r = (tx0 - gx0) + cx + RX * ((ty0 - gy0) + cy);
+        ms.occ[c] = ~s_nb[r].free & full;
+        if (s_gap[r]) ms.gap[c] = s_gap[r];
+    }
+    if (STATS) {
+        stat_add(st, ST_MOVED, n_moved);
+        stat_add(st, ST_DELETED, n_del);
+        stat_add(st, ST_DROPPED, n_drop);
+    }
+}
+
+// ------------------------------------------------------------ 3. scatter
+// T: coordinate type (double: FP64 drop-in, float: split offsets)
+template <int D, typename T>
+struct TPtr3 {
+    T* p[3];
+};
+
+// REC16: 2D split with one field (16-byte records, one load per arrival)
+template <int D, typename T, bool REC16 = false>
+__global__ void __launch_bounds__(kBlock) k_mv_scatter(Grid<D> g, TPtr3<D, T> coords,
+                                                       uint8_t* __restrict__ index, int nargs,
+                                                       ArgPtrs args, MoveScratch ms,
+                                                       const SplitGeom* __restrict__ geo,
+                                                       int span, int* __restrict__ flag) {
+    // the phases are over: the flag words are ready for the next move
+    if (blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0) flag[0] = flag[1] = 0;
+    // one thread per cell and slot group (blockIdx.y, `span` slots), chunks of
+    // 8 slot planes in lockstep across the wavefront (coalesced origin loads
+    // and final stores); only the reads of the staged data are scattered.
+    // Arrivals copy their staged data, vacated slots are emptied
+    // (empty_particle!, src/Particles/move_safe.jl:243-251).  Nothing moves
+    // when the split grid was rejected (geo: null in the FP64 form).
+    if (geo && geo->bad) return;
+    // 2D: XCD-contiguous cell ranges (a destination's sources are its
+    // neighbour cells, whose staged lines other threads of the same L2 also
+    // read; a row of cells above or below is only a few workgroups away, which
+    // round-robin dealing puts on other XCDs); slot groups of one cell block
+    // stay together.  3D keeps the dealt order: there the plane above or below
+    // is a multiple of 8 workgroups away, already on the same XCD, and the
+    // renumbering measured slower.
+    const unsigned lb = D == 2 ? xcd_block(blockIdx.x + gridDim.x * blockIdx.y,
+                                           gridDim.x * gridDim.y)
+                               : blockIdx.x * gridDim.y + blockIdx.y;
+    const int64_t c = (lb / gridDim.y) * (int64_t)blockDim.x + threadIdx.x;
+    if (c >= g.C) return;
+    const int kb = (int)(lb % gridDim.y) * span;
+    const int ke = kb + span < g.K ? kb + span : g.K;
+    const int64_t C = g.C;
+    // the first chunk's origins go out with the cell's words: unguarded loads
+    // (slot clamped to K - 1, values used for arrivals only), one round trip
+    // fewer than loading them after the arrival bits are known
+    uint16_t o0[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const int k = kb + j < g.K ? kb + j : g.K - 1;
+        o0[j] = ms.org[org_at<D>((uint32_t)c, (uint32_t)k, (uint32_t)C, (uint32_t)g.K)];
+    }
+    const uint64_t occ = ms.occ[c], occ0 = ms.occ0[c], gap = ms.gap[c];
+    const uint64_t arr = arrivals(occ, occ0, ms.mov[c]);
+    const uint64_t work = arr | (~occ & (occ0 | gap));  // arrivals, emptied slots
+    if (!(work >> kb)) return;
+    const int str1 = (int)g.ni[0], str2 = (int)(g.ni[0] * g.ni[1]);
+    for (int k0 = kb; k0 < ke; k0 += 8) {
+        const uint32_t wb = (uint32_t)(work >> k0) & 0xFFu;
+        if (!wb) continue;
+        const uint32_t ab = (uint32_t)(arr >> k0) & 0xFFu;
+        uint32_t o[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t at = org_at<D>((uint32_t)c, (uint32_t)(k0 + j), (uint32_t)C,
+                                          (uint32_t)g.K);
+            o[j] = k0 == kb ? (uint32_t)o0[j] : ((ab >> j) & 1) ? (uint32_t)ms.org[at] : 0u;
+        }
+        // the record numbers: of the source cell, its rank-th
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const uint32_t src = (uint32_t)c - (uint32_t)move_offset<D>((o[j] >> 6) & 0x7Fu, str1,
+                                                                        str2);
+            if (((ab >> j) & 1) && o[j] == kOrgFar)
+                o[j] = ms.orgf[org_at<D>((uint32_t)c, (uint32_t)(k0 + j), (uint32_t)C,
+                                         (uint32_t)g.K)];
+            else
+                o[j] = src * (uint32_t)g.K + (o[j] & 63u);
+        }
+        if constexpr (REC16) {
+            float u0[8], u1[8];
+            double fv[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                u0[j] = u1[j] = __builtin_nanf("");
+                fv[j] = dnan();
+                if ((ab >> j) & 1) stg_get16(ms, o[j], u0[j], u1[j], fv[j]);
+            }
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                if (!((wb >> j) & 1)) continue;
+                const int64_t e = c + C * (k0 + j);
+                coords.p[0][e] = (T)u0[j];
+                coords.p[D - 1][e] = (T)u1[j];
+                index[e] = (uint8_t)((ab >> j) & 1);
+                args.p[0][e] = fv[j];
+            }
+            continue;
+        }
+        T v[8][D];
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+#pragma unroll
+            for (int d = 0; d < D; ++d)
+                v[j][d] = ((ab >> j) & 1) ? stg_coord<D, T>(ms, o[j], d) : (T)dnan();
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (!((wb >> j) & 1)) continue;
+            const int64_t e = c + C * (k0 + j);
+#pragma unroll
+            for (int d = 0; d < D; ++d) coords.p[d][e] = v[j][d];
+            index[e] = (uint8_t)((ab >> j) & 1);
+        }
+        for (int a = 0; a < nargs; ++a) {
+            double av[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) av[j] = ((ab >> j) & 1) ? stg_field<D>(ms, o[j], a) : dnan();
+#pragma unroll
+            for (int j = 0; j < 8; ++j)
+                if ((wb >> j) & 1) args.p[a][c + C * (k0 + j)] = av[j];
+        }
+    }
 }
 
 // ------------------------------------------------------------ split classify
@@ -1372,9 +1392,9 @@ TPtr3<D, T> tptr3(T* const* c) {
 size_t align_up(size_t x, size_t a) { return (x + a - 1) / a * a; }
 
 // classify -> colour phases (2D: one tiled launch; 3D: 3^D launches) -> far-
-// jump phases (one workgroup; returns at once unless a particle jumped more
-// than one cell, in which case the regular phases returned at once) ->
-// scatter
+// jump phases (one workgroup, of the tiled launch or of one that returns at once
+// unless a particle jumped more than one cell; then the regular phases returned
+// at once) -> scatter
 template <int D, typename T>
 int run_move(jp_ctx* ctx, const jp_cellgrid* gc, T* const* coords, uint8_t* index, int nargs,
              double* const* args, jp_stats* stats) {
@@ -1413,10 +1433,9 @@ int run_move(jp_ctx* ctx, const jp_cellgrid* gc, T* const* coords, uint8_t* inde
     ms.stg = base + o_stg;
 
     int* flag = dflags(ctx);
-    // the flag words are zero here: a new context starts with them cleared,
-    // the far-jump kernel, which runs on every move after the regular phases,
-    // clears them after use, and a launch that fails after classify clears
-    // them here
+    // the flag words are zero here: a new context starts with them cleared, the
+    // scatter, which runs on every move after the phases, clears them after use,
+    // and a launch that fails after classify clears them here
     auto launched = [&]() -> int {
         const hipError_t e = hipGetLastError();
         if (e == hipSuccess) return JP_OK;
@@ -1463,10 +1482,10 @@ int run_move(jp_ctx* ctx, const jp_cellgrid* gc, T* const* coords, uint8_t* inde
             return fail(ctx, JP_ERR_ARG, "grid too large%s");
         Grid<2> g2 = to_grid<2>(gc);
         if (st)
-            k_mv_tiles2<TX, TY, 256, true><<<(unsigned)tiles, 256, 0, ctx->stream>>>(g2, ms, flag,
+            k_mv_tiles2<TX, TY, 256, true, T><<<(unsigned)tiles, 256, 0, ctx->stream>>>(g2, ms, flag,
                                                                                    st);
         else
-            k_mv_tiles2<TX, TY, 256, false><<<(unsigned)tiles, 256, 0, ctx->stream>>>(g2, ms,
+            k_mv_tiles2<TX, TY, 256, false, T><<<(unsigned)tiles, 256, 0, ctx->stream>>>(g2, ms,
                                                                                     flag, st);
         if ((rc = launched())) return rc;
     }
@@ -1484,19 +1503,21 @@ int run_move(jp_ctx* ctx, const jp_cellgrid* gc, T* const* coords, uint8_t* inde
             k_mv_phase<D, BS, false><<<nb, BS, 0, ctx->stream>>>(g, ms, o, ph, flag, st);
         if ((rc = launched())) return rc;
     }
-    k_mv_far<D, T><<<1, kFarBlock, 0, ctx->stream>>>(g, ms, flag, st);
-    if ((rc = launched())) return rc;
+    if (nphase) {
+        k_mv_far<D, T><<<1, kFarBlock, 0, ctx->stream>>>(g, ms, flag, st);
+        if ((rc = launched())) return rc;
+    }
     const SplitGeom* geo = std::is_same<T, double>::value ? nullptr : geo_ptr(ctx);
     bool rec16 = false;  // 2D split, one field: 16-byte records
     if constexpr (D == 2 && std::is_same<T, float>::value) {
         rec16 = nargs == 1;
         if (rec16)
             k_mv_scatter<D, T, true><<<cgrid, kBlock, 0, ctx->stream>>>(g, cp, index, nargs, ap,
-                                                                        ms, geo, span);
+                                                                        ms, geo, span, flag);
     }
     if (!rec16)
         k_mv_scatter<D, T><<<cgrid, kBlock, 0, ctx->stream>>>(g, cp, index, nargs, ap, ms, geo,
-                                                             span);
+                                                             span, flag);
     if ((rc = launched())) return rc;
 
     if ((rc = stats_end(ctx, stats))) return rc;
