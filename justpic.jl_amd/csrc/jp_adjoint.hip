@@ -17,10 +17,10 @@
 //    record their final cell and count themselves into it.
 //  - particle2grid! of the survivors without float atomics: the per-cell
 //    counts are scanned, particle ids are bucketed by cell and each bucket is
-//    sorted by id; every node then merges the id-sorted buckets of its 2^D
-//    cells and accumulates w and fma(w, T, .) in increasing particle id, the
-//    order of the oracle's restatement, so F and W are reproducible and equal
-//    to it bit for bit.
+//    put in order of id, with its positions and tracers; every node then merges
+//    the buckets of its 2^D cells and accumulates w and fma(w, T, .) in
+//    increasing particle id, the order of the oracle's restatement, so F and W
+//    are reproducible and equal to it bit for bit.
 //  - k_adj_bwd: blocks of steps in reverse order; a block is recomputed from
 //    its checkpoint into a tape (the position at the start of each step, in
 //    global scratch), then reversed step by step.  x0bar and Tpbar are per-thread
@@ -772,34 +772,69 @@ __global__ __launch_bounds__(kBlock) void k_adj_fwd_split(
     cell[i] = c;
 }
 
-// exclusive scan of the C cell counts into start[0..C] (one workgroup)
-constexpr int kScan = 1024;
-__global__ __launch_bounds__(kScan) void k_adj_scan(const int32_t* __restrict__ cnt,
-                                                    int32_t* __restrict__ start, int64_t C) {
-    __shared__ int32_t part[kScan];
-    const int t = threadIdx.x;
-    const int64_t per = (C + kScan - 1) / kScan;
-    const int64_t lo = t * per < C ? t * per : C;
-    const int64_t hi = lo + per < C ? lo + per : C;
+// exclusive scan of the C cell counts into start[0..C], kScan counts per workgroup:
+// the workgroups' sums, then each one's scan from the sum of those before it (one
+// workgroup for all, a chunk per thread, took 110 us for 65536 cells; the two 10)
+constexpr int kScan = 2048;
+__device__ inline int32_t scan_chunk(const int32_t* __restrict__ cnt, int64_t C, int64_t c,
+                                     int32_t (&v)[kScan / kBlock]) {
     int32_t s = 0;
-    for (int64_t c = lo; c < hi; ++c) s += cnt[c];
-    part[t] = s;
+#pragma unroll
+    for (int j = 0; j < kScan / kBlock; ++j) {
+        v[j] = c + j < C ? cnt[c + j] : 0;
+        s += v[j];
+    }
+    return s;
+}
+__device__ inline int32_t block_sum(int32_t s, int32_t* part) {  // all threads; part: a word per wave
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
     __syncthreads();
-    for (int off = 1; off < kScan; off <<= 1) {
-        const int32_t v = t >= off ? part[t - off] : 0;
-        __syncthreads();
-        part[t] += v;
-        __syncthreads();
+    int32_t r = 0;
+#pragma unroll
+    for (int w = 0; w < kBlock / 64; ++w) r += part[w];
+    __syncthreads();
+    return r;
+}
+__global__ __launch_bounds__(kBlock) void k_adj_sums(const int32_t* __restrict__ cnt,
+                                                     int32_t* __restrict__ sums, int64_t C) {
+    __shared__ int32_t part[kBlock / 64];
+    int32_t v[kScan / kBlock];
+    const int64_t c = blockIdx.x * (int64_t)kScan + threadIdx.x * (kScan / kBlock);
+    const int32_t s = block_sum(scan_chunk(cnt, C, c, v), part);
+    if (threadIdx.x == 0) sums[blockIdx.x] = s;
+}
+__global__ __launch_bounds__(kBlock) void k_adj_starts(const int32_t* __restrict__ cnt,
+                                                       const int32_t* __restrict__ sums,
+                                                       int32_t* __restrict__ start, int64_t C) {
+    __shared__ int32_t part[kBlock / 64];
+    int32_t before = 0;
+    for (unsigned b = threadIdx.x; b < blockIdx.x; b += kBlock) before += sums[b];
+    before = block_sum(before, part);
+    int32_t v[kScan / kBlock];
+    const int64_t c = blockIdx.x * (int64_t)kScan + threadIdx.x * (kScan / kBlock);
+    const int32_t s = scan_chunk(cnt, C, c, v);
+    int32_t incl = s;
+    const int lane = threadIdx.x & 63;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int32_t u = __shfl_up(incl, o);
+        if (lane >= o) incl += u;
     }
-    int32_t run = part[t] - s;  // exclusive prefix of this thread's chunk
-    for (int64_t c = lo; c < hi; ++c) {
-        start[c] = run;
-        run += cnt[c];
+    if (lane == 63) part[threadIdx.x >> 6] = incl;
+    __syncthreads();
+    int32_t run = before + incl - s;
+    for (int w = 0; w < (int)(threadIdx.x >> 6); ++w) run += part[w];
+#pragma unroll
+    for (int j = 0; j < kScan / kBlock; ++j) {
+        if (c + j < C) start[c + j] = run;
+        run += v[j];
+        if (c + j == C - 1) start[C] = run;
     }
-    if (t == kScan - 1) start[C] = part[t];
 }
 
-// bucket the survivors by cell (order inside a bucket fixed by k_adj_sort);
+// bucket the survivors by cell (order inside a bucket fixed by k_adj_order);
 // consumes the counts
 __global__ __launch_bounds__(kBlock) void k_adj_bucket(const int32_t* __restrict__ cell,
                                                       int32_t* __restrict__ cnt,
@@ -813,35 +848,51 @@ __global__ __launch_bounds__(kBlock) void k_adj_bucket(const int32_t* __restrict
     list[start[c] + slot] = (int32_t)i;
 }
 
-// sort every bucket by particle id (insertion sort; buckets hold tens of ids)
-__global__ __launch_bounds__(kBlock) void k_adj_sort(const int32_t* __restrict__ start,
-                                                    int32_t* __restrict__ list, int64_t C) {
-    const int64_t c = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= C) return;
+// every bucket in order of particle id, with the positions and tracers (a thread
+// per survivor counts the smaller ids of its bucket, which holds tens): what the
+// gather reads then lies together
+template <int D>
+__global__ __launch_bounds__(kBlock) void k_adj_order(const int32_t* __restrict__ cell,
+                                                     const int32_t* __restrict__ start,
+                                                     const int32_t* __restrict__ list,
+                                                     CPtr3 xN, const double* __restrict__ Tp,
+                                                     int64_t C, int32_t* __restrict__ ids,
+                                                     Ptr3 xs, double* __restrict__ Ts) {
+    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= start[C]) return;
+    const int32_t id = list[i];
+    const int32_t c = cell[id];
     const int32_t lo = start[c], hi = start[c + 1];
-    for (int32_t j = lo + 1; j < hi; ++j) {
-        const int32_t v = list[j];
-        int32_t k = j - 1;
-        while (k >= lo && list[k] > v) {
-            list[k + 1] = list[k];
-            --k;
-        }
-        list[k + 1] = v;
-    }
+    double x[D];
+#pragma unroll
+    for (int d = 0; d < D; ++d) x[d] = xN.p[d][id];
+    const double T = Tp[id];
+    int32_t at = lo;
+    for (int32_t j = lo; j < hi; ++j) at += list[j] < id ? 1 : 0;
+    ids[at] = id;
+#pragma unroll
+    for (int d = 0; d < D; ++d) xs.p[d][at] = x[d];
+    Ts[at] = T;
 }
 
 // per node: merge the id-sorted buckets of its 2^D cells; w = inv(distance^2),
 // W += w, S = fma(w, T, S) in increasing particle id; F = S / W (2D),
-// S * inv(W) (3D); a node without particles gets 0/0 = NaN
+// S * inv(W) (3D); a node without particles gets 0/0 = NaN.  The heads of the
+// buckets are in registers, and the one taken is replaced by its successor, one
+// load from where its bucket lies (the ids' list and then the particle's own
+// arrays: two dependent loads far apart, 165 us for 257 x 257 nodes of 1 M
+// particles, with the sort 231; now with the order 144).
 template <int D>
 __global__ __launch_bounds__(kBlock) void k_adj_gather(AdjArgs<D> A,
                                                       const int32_t* __restrict__ start,
-                                                      const int32_t* __restrict__ list, CPtr3 xN,
-                                                      const double* __restrict__ Tp,
+                                                      const int32_t* __restrict__ ids, CPtr3 xs,
+                                                      const double* __restrict__ Ts,
                                                       double* __restrict__ F,
                                                       double* __restrict__ W, int64_t nodes) {
     const int64_t n = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (n >= nodes) return;
+    constexpr int NQ = 1 << D;
+    constexpr int32_t kNone = 0x7fffffff;
     int64_t N[D];
     int64_t r = n;
 #pragma unroll
@@ -852,9 +903,10 @@ __global__ __launch_bounds__(kBlock) void k_adj_gather(AdjArgs<D> A,
     double xn[D];
 #pragma unroll
     for (int d = 0; d < D; ++d) xn[d] = A.G.xv[d].x[N[d]];
-    int32_t h[1 << D], e[1 << D];
+    int32_t h[NQ], e[NQ], id[NQ];
+    double x[NQ][D], T[NQ];
 #pragma unroll
-    for (int q = 0; q < (1 << D); ++q) {
+    for (int q = 0; q < NQ; ++q) {
         int64_t I[D];
         bool ok = true;
 #pragma unroll
@@ -869,35 +921,68 @@ __global__ __launch_bounds__(kBlock) void k_adj_gather(AdjArgs<D> A,
             e[q] = start[c + 1];
         }
     }
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        id[q] = kNone;
+        T[q] = 0.0;
+#pragma unroll
+        for (int d = 0; d < D; ++d) x[q][d] = 0.0;
+        if (h[q] < e[q]) {
+            id[q] = ids[h[q]];
+#pragma unroll
+            for (int d = 0; d < D; ++d) x[q][d] = xs.p[d][h[q]];
+            T[q] = Ts[h[q]];
+        }
+    }
     double w = 0.0, s = 0.0;
     for (;;) {
-        int best = -1;
-        int32_t id = 0;
+        int32_t first = id[0];
 #pragma unroll
-        for (int q = 0; q < (1 << D); ++q) {
-            if (h[q] < e[q]) {
-                const int32_t v = list[h[q]];
-                if (best < 0 || v < id) {
-                    best = q;
-                    id = v;
-                }
-            }
+        for (int q = 1; q < NQ; ++q) first = id[q] < first ? id[q] : first;
+        if (first == kNone) break;
+        double p[D], t = T[0];
+        int32_t nx = h[0], end = e[0];
+#pragma unroll
+        for (int d = 0; d < D; ++d) p[d] = x[0][d];
+#pragma unroll
+        for (int q = 1; q < NQ; ++q) {
+            const bool m = id[q] == first;
+            t = m ? T[q] : t;
+            nx = m ? h[q] : nx;
+            end = m ? e[q] : end;
+#pragma unroll
+            for (int d = 0; d < D; ++d) p[d] = m ? x[q][d] : p[d];
         }
-        if (best < 0) break;
+        // its successor (the last one again at the bucket's end: not used)
+        nx += 1;
+        const bool more = nx < end;
+        const int32_t at = more ? nx : nx - 1;
+        const int32_t idn = ids[at];
+        double pn[D];
 #pragma unroll
-        for (int q = 0; q < (1 << D); ++q) h[q] += q == best ? 1 : 0;
+        for (int d = 0; d < D; ++d) pn[d] = xs.p[d][at];
+        const double tn = Ts[at];
         // distance (src/Interpolations/utils.jl:9-19), node minus particle
-        double dl = xn[0] - xN.p[0][id];
+        double dl = xn[0] - p[0];
         double ss = dl * dl;
 #pragma unroll
         for (int d = 1; d < D; ++d) {
-            dl = xn[d] - xN.p[d][id];
+            dl = xn[d] - p[d];
             ss = ss + dl * dl;
         }
         const double dist = sqrt(ss);
         const double wi = 1.0 / (dist * dist);
         w += wi;
-        s = fma(wi, Tp[id], s);
+        s = fma(wi, t, s);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) {
+            const bool m = id[q] == first;
+            h[q] = m ? nx : h[q];
+            T[q] = m ? tn : T[q];
+#pragma unroll
+            for (int d = 0; d < D; ++d) x[q][d] = m ? pn[d] : x[q][d];
+            id[q] = m ? (more ? idn : kNone) : id[q];
+        }
     }
     W[n] = w;
     F[n] = D == 2 ? s / w : s * (1.0 / w);
@@ -1113,18 +1198,36 @@ template <int D, int M>
 int forward(jp_ctx* ctx, const AdjArgs<D>& A, const double* const* x0, const double* Tp,
             double* ckpt, uint8_t* alive, double* const* xN, double* F, double* W,
             int64_t nodes, const SplitFwd<D>& sf = SplitFwd<D>()) {
-    // scratch: counts (C) | bucket starts (C+1) | cell of each particle | buckets
+    // scratch: counts (C) | bucket starts (C+1) | the scan's sums | cell of each
+    // particle | buckets | their ids, positions and tracers in order
     const int64_t C = A.G.C;
-    const size_t a = ((size_t)C * 4 + 255) & ~(size_t)255;
-    const size_t b = a + (((size_t)(C + 1) * 4 + 255) & ~(size_t)255);
-    const size_t c = b + (((size_t)A.np * 4 + 255) & ~(size_t)255);
-    int rc = ensure_scratch(ctx, c + (size_t)A.np * 4 + 4);
+    const int64_t scans = (C + kScan - 1) / kScan;
+    size_t end = 0;
+    auto part = [&](size_t bytes) {
+        const size_t at = end;
+        end = (end + bytes + 255) & ~(size_t)255;
+        return at;
+    };
+    const size_t o_cnt = part((size_t)C * 4), o_start = part((size_t)(C + 1) * 4);
+    const size_t o_sums = part((size_t)scans * 4), o_cell = part((size_t)A.np * 4);
+    const size_t o_list = part((size_t)A.np * 4), o_ids = part((size_t)A.np * 4);
+    const size_t o_xs = part((size_t)A.np * 8 * D), o_Ts = part((size_t)A.np * 8);
+    int rc = ensure_scratch(ctx, end);
     if (rc) return rc;
     char* base = static_cast<char*>(ctx->scratch);
-    int32_t* cnt = reinterpret_cast<int32_t*>(base);
-    int32_t* start = reinterpret_cast<int32_t*>(base + a);
-    int32_t* cell = reinterpret_cast<int32_t*>(base + b);
-    int32_t* list = reinterpret_cast<int32_t*>(base + c);
+    int32_t* cnt = reinterpret_cast<int32_t*>(base + o_cnt);
+    int32_t* start = reinterpret_cast<int32_t*>(base + o_start);
+    int32_t* sums = reinterpret_cast<int32_t*>(base + o_sums);
+    int32_t* cell = reinterpret_cast<int32_t*>(base + o_cell);
+    int32_t* list = reinterpret_cast<int32_t*>(base + o_list);
+    int32_t* ids = reinterpret_cast<int32_t*>(base + o_ids);
+    double* Ts = reinterpret_cast<double*>(base + o_Ts);
+    CPtr3 cxs{{nullptr, nullptr, nullptr}};
+    Ptr3 xs{{nullptr, nullptr, nullptr}};
+    for (int d = 0; d < D; ++d) {
+        xs.p[d] = reinterpret_cast<double*>(base + o_xs) + (int64_t)d * A.np;
+        cxs.p[d] = xs.p[d];
+    }
     if ((rc = zero_bytes(ctx, cnt, (size_t)C * 4))) return rc;
     CPtr3 xp{{nullptr, nullptr, nullptr}}, xq{{nullptr, nullptr, nullptr}};
     Ptr3 xo{{nullptr, nullptr, nullptr}};
@@ -1145,17 +1248,20 @@ int forward(jp_ctx* ctx, const AdjArgs<D>& A, const double* const* x0, const dou
         }
         JP_LAUNCHED(ctx);
     }
-    k_adj_scan<<<1, kScan, 0, ctx->stream>>>(cnt, start, C);
+    k_adj_sums<<<(unsigned)scans, kBlock, 0, ctx->stream>>>(cnt, sums, C);
+    JP_LAUNCHED(ctx);
+    k_adj_starts<<<(unsigned)scans, kBlock, 0, ctx->stream>>>(cnt, sums, start, C);
     JP_LAUNCHED(ctx);
     if (A.np > 0) {
         k_adj_bucket<<<(unsigned)blocks_for(A.np), kBlock, 0, ctx->stream>>>(cell, cnt, start,
                                                                              list, A.np);
         JP_LAUNCHED(ctx);
+        k_adj_order<D><<<(unsigned)blocks_for(A.np), kBlock, 0, ctx->stream>>>(
+            cell, start, list, xq, Tp, C, ids, xs, Ts);
+        JP_LAUNCHED(ctx);
     }
-    k_adj_sort<<<(unsigned)blocks_for(C), kBlock, 0, ctx->stream>>>(start, list, C);
-    JP_LAUNCHED(ctx);
-    k_adj_gather<D><<<(unsigned)blocks_for(nodes), kBlock, 0, ctx->stream>>>(A, start, list, xq,
-                                                                            Tp, F, W, nodes);
+    k_adj_gather<D><<<(unsigned)blocks_for(nodes), kBlock, 0, ctx->stream>>>(A, start, ids, cxs,
+                                                                            Ts, F, W, nodes);
     JP_LAUNCHED(ctx);
     return sf.on ? split_finish(ctx) : finish(ctx);
 }
