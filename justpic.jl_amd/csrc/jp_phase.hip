@@ -114,9 +114,9 @@ __device__ inline void gather_half(const Grid<D>& g, const CPtr3& coords,
 // phase_ratios_center_kernel! (src/PhaseRatios/centers.jl:14-30): the
 // particles of cell I whose first coordinate is not NaN, about xci[I]
 template <int D, int NP>
-__global__ void __launch_bounds__(kBlock) k_ratio_center(Grid<D> g, CAxes<D> xc, CPtr3 coords,
-                                                         const double* __restrict__ phases,
-                                                         int nph, double* __restrict__ out) {
+__device__ inline void ratio_center(const Grid<D>& g, const CAxes<D>& xc, const CPtr3& coords,
+                                    const double* __restrict__ phases, int nph,
+                                    double* __restrict__ out) {
     const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (c >= g.C) return;
     int64_t I[D];
@@ -140,9 +140,9 @@ __global__ void __launch_bounds__(kBlock) k_ratio_center(Grid<D> g, CAxes<D> xc,
 // particles strictly within half a cell of vertex N, from the up to 2^D
 // cells around it with the first dimension's offset outermost
 template <int D, int NP>
-__global__ void __launch_bounds__(kBlock) k_ratio_vertex(Grid<D> g, CPtr3 coords,
-                                                         const double* __restrict__ phases,
-                                                         int nph, double* __restrict__ out) {
+__device__ inline void ratio_vertex(const Grid<D>& g, const CPtr3& coords,
+                                    const double* __restrict__ phases, int nph,
+                                    double* __restrict__ out) {
     int64_t nn[D], NN = 1;
 #pragma unroll
     for (int d = 0; d < D; ++d) {
@@ -208,9 +208,9 @@ __device__ inline int64_t lin_dims(const int64_t (&I)[D], const int64_t (&dims)[
 // also writes face I from its own particles about xci - di e_dim / 2, with
 // the spacing of the last cell gathered
 template <int D, int NP>
-__global__ void __launch_bounds__(kBlock) k_ratio_face(Grid<D> g, CAxes<D> xc, CPtr3 coords,
-                                                       const double* __restrict__ phases, int nph,
-                                                       int dim, double* __restrict__ out) {
+__device__ inline void ratio_face(const Grid<D>& g, const CAxes<D>& xc, const CPtr3& coords,
+                                  const double* __restrict__ phases, int nph, int dim,
+                                  double* __restrict__ out) {
     const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (c >= g.C) return;
     int64_t I[D], dims[D];
@@ -335,28 +335,50 @@ __global__ void __launch_bounds__(kBlock) k_ratio_midpoint(Grid<3> g, CAxes<3> x
     }
 }
 
+// Vertices, faces and centres in one launch, the workgroups of a kind one after the
+// other, the longest first (out[y]: kind's output; kind -1 centres, 0 vertices, d + 1
+// the faces normal to d).  A kind alone has one wavefront or two per SIMD at 256 x 256
+// to 384 x 257 cells and lasts as long as the SIMDs with two: 384 x 257 cells of 48
+// slots 81 us (vertices), 2 x 43 and 20, together 147 (136 registers; bound by 4
+// wavefronts to 128, 151).
+struct RatioKinds {
+    int kind[5];
+    double* out[5];
+};
+template <int D, int NP>
+__global__ void __launch_bounds__(kBlock) k_ratios(Grid<D> g, CAxes<D> xc, CPtr3 coords,
+                                                   const double* __restrict__ phases, int nph,
+                                                   RatioKinds r) {
+    const int kind = r.kind[blockIdx.y];
+    double* const out = r.out[blockIdx.y];
+    if (kind == 0)
+        ratio_vertex<D, NP>(g, coords, phases, nph, out);
+    else if (kind < 0)
+        ratio_center<D, NP>(g, xc, coords, phases, nph, out);
+    else
+        ratio_face<D, NP>(g, xc, coords, phases, nph, kind - 1, out);
+}
+
 template <int D, int NP>
 int launch_ratios(jp_ctx* ctx, const Grid<D>& G, const CAxes<D>& xa, const CPtr3& cp,
                   const double* phases, int nph, double* center, double* vertex,
                   double* const* faces) {
-    if (center) {
-        k_ratio_center<D, NP><<<(unsigned)blocks_for(G.C), kBlock, 0, ctx->stream>>>(
-            G, xa, cp, phases, nph, center);
-        JP_LAUNCHED(ctx);
-    }
-    if (vertex) {
-        int64_t NN = 1;
-        for (int d = 0; d < D; ++d) NN *= G.ni[d] + 1;
-        k_ratio_vertex<D, NP><<<(unsigned)blocks_for(NN), kBlock, 0, ctx->stream>>>(
-            G, cp, phases, nph, vertex);
-        JP_LAUNCHED(ctx);
-    }
-    for (int d = 0; d < D; ++d) {
-        if (!faces || !faces[d]) continue;
-        k_ratio_face<D, NP><<<(unsigned)blocks_for(G.C), kBlock, 0, ctx->stream>>>(
-            G, xa, cp, phases, nph, d, faces[d]);
-        JP_LAUNCHED(ctx);
-    }
+    RatioKinds r{};
+    unsigned n = 0;
+    auto add = [&](int kind, double* out) {
+        if (!out) return;
+        r.kind[n] = kind;
+        r.out[n++] = out;
+    };
+    add(0, vertex);
+    for (int d = 0; d < D; ++d) add(d + 1, faces ? faces[d] : nullptr);
+    add(-1, center);
+    if (!n) return JP_OK;
+    int64_t locations = 1;  // of the vertices, the most
+    for (int d = 0; d < D; ++d) locations *= G.ni[d] + 1;
+    k_ratios<D, NP><<<dim3((unsigned)blocks_for(locations), n), kBlock, 0, ctx->stream>>>(
+        G, xa, cp, phases, nph, r);
+    JP_LAUNCHED(ctx);
     return JP_OK;
 }
 
