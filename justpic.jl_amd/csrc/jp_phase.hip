@@ -268,82 +268,75 @@ __device__ inline void ratio_face(const Grid<D>& g, const CAxes<D>& xc, const CP
 // for the masks (1,0,0), (0,1,0), (0,0,1), (1,1,1) about xci + di .* o / 2; a
 // cell on a first boundary (I_d = 1 where o_d = 1, 1-based) also writes the
 // edges I and I + b, b_d = (ni_d == o_d I_d), about xci - (di .* o .* (-b)) / 2
+template <int NP>
 __device__ inline void midpoint_pass(const Grid<3>& g, const CPtr3& coords,
                                      const double* __restrict__ phases, int nph,
                                      const int64_t (&I)[3], const int (&o)[3],
-                                     const double (&m)[3], double (&w)[16], int np) {
-    constexpr int MASK[4][3] = {{1, 0, 0}, {0, 1, 0}, {0, 0, 1}, {1, 1, 1}};
-    (void)np;
-#pragma unroll
+                                     const double (&m)[3], double (&w)[NP]) {
+    // masks (1,0,0), (0,1,0), (0,0,1), (1,1,1)
+#pragma unroll 1
     for (int mk = 0; mk < 4; ++mk) {
         int64_t J[3];
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            const int64_t k = I[d] + o[d] * MASK[mk][d];
+            const int64_t k = I[d] + (mk == d || mk == 3 ? o[d] : 0);
             J[d] = k > g.ni[d] - 1 ? g.ni[d] - 1 : k;
         }
         double di[3], inv[3];
-        gather_half<3, 16>(g, coords, phases, nph, J, m, w, di, inv);
+        gather_half<3, NP>(g, coords, phases, nph, J, m, w, di, inv);
     }
 }
 
-__global__ void __launch_bounds__(kBlock) k_ratio_midpoint(Grid<3> g, CAxes<3> xc, CPtr3 coords,
-                                                           const double* __restrict__ phases,
-                                                           int nph, int o0, int o1, int o2,
-                                                           double* __restrict__ out) {
+template <int NP>
+__device__ inline void ratio_midpoint(const Grid<3>& g, const CAxes<3>& xc, const CPtr3& coords,
+                                      const double* __restrict__ phases, int nph,
+                                      const int (&o)[3], double* __restrict__ out) {
     const int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
     if (c >= g.C) return;
-    const int o[3] = {o0, o1, o2};
     int64_t I[3], dims[3];
     unlin<3>(g.ni, c, I);
-    double xcen[3], m[3], dm[3], w[16];
+    double xcen[3], m[3], dm[3];
     int64_t L = 1;
+    bool first = false;
+    int b[3];
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
         dims[d] = g.ni[d] + o[d];
         L *= dims[d];
         xcen[d] = xc.a[d].x[I[d]];
         dm[d] = g.xv[d].dx[I[d]];
-        m[d] = xcen[d] + (dm[d] * (double)o[d]) / 2.0;
-    }
-#pragma unroll
-    for (int j = 0; j < 16; ++j) w[j] = 0.0;
-    midpoint_pass(g, coords, phases, nph, I, o, m, w, 16);
-    int64_t Io[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) Io[d] = I[d] + o[d];
-    normalise_write<16>(w, nph, out, L, lin_dims<3>(Io, dims), true);
-    bool first = false;
-    int b[3];
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
         first = first || (o[d] * (I[d] + 1) == 1);
         b[d] = g.ni[d] == (int64_t)o[d] * (I[d] + 1) ? 1 : 0;
     }
-    if (!first) return;
-    for (int it = 0; it < 2; ++it) {
-        double w2[16];
+    // pass 0: edge I + o; on a first boundary also the edges I and I + b
+#pragma unroll 1
+    for (int it = 0; it < (first ? 3 : 1); ++it) {
+        double w[NP];
 #pragma unroll
-        for (int j = 0; j < 16; ++j) w2[j] = 0.0;
+        for (int j = 0; j < NP; ++j) w[j] = 0.0;
+        int64_t E[3];
 #pragma unroll
-        for (int d = 0; d < 3; ++d) m[d] = xcen[d] - ((dm[d] * (double)o[d]) * (double)(0 - b[d])) / 2.0;
-        midpoint_pass(g, coords, phases, nph, I, o, m, w2, 16);
-        int64_t Ib[3];
-#pragma unroll
-        for (int d = 0; d < 3; ++d) Ib[d] = I[d] + (it ? b[d] : 0);
-        normalise_write<16>(w2, nph, out, L, lin_dims<3>(Ib, dims), true);
+        for (int d = 0; d < 3; ++d) {
+            E[d] = I[d] + (it == 0 ? o[d] : (it == 1 ? 0 : b[d]));
+            m[d] = it == 0 ? xcen[d] + (dm[d] * (double)o[d]) / 2.0
+                           : xcen[d] - ((dm[d] * (double)o[d]) * (double)(0 - b[d])) / 2.0;
+        }
+        midpoint_pass<NP>(g, coords, phases, nph, I, o, m, w);
+        normalise_write<NP>(w, nph, out, L, lin_dims<3>(E, dims), true);
     }
 }
 
-// Vertices, faces and centres in one launch, the workgroups of a kind one after the
-// other, the longest first (out[y]: kind's output; kind -1 centres, 0 vertices, d + 1
-// the faces normal to d).  A kind alone has one wavefront or two per SIMD at 256 x 256
-// to 384 x 257 cells and lasts as long as the SIMDs with two: 384 x 257 cells of 48
-// slots 81 us (vertices), 2 x 43 and 20, together 147 (136 registers; bound by 4
-// wavefronts to 128, 151).
+// All kinds of locations in one launch, the workgroups of a kind one after the other,
+// the longest first (out[y]: kind's output).  A kind alone has one wavefront or two
+// per SIMD at 256 x 256 to 384 x 257 cells and lasts as long as the SIMDs with two:
+// 384 x 257 cells of 48 slots 81 us (vertices), 2 x 43 and 20, together 147 (136
+// registers; bound by 4 wavefronts to 128, 151).  20 x 23 x 17 cells of 54 slots, 3
+// phases: three launches of 297 us (midpoints, 400 registers for 16 phases and four
+// unrolled cells) and 121, together 172.
+enum { kCentres = -1, kVertices = 0, kFaces = 1, kEdges = 4 };  // + dimension; + xy, yz, xz
 struct RatioKinds {
-    int kind[5];
-    double* out[5];
+    int kind[8];
+    double* out[8];
 };
 template <int D, int NP>
 __global__ void __launch_bounds__(kBlock) k_ratios(Grid<D> g, CAxes<D> xc, CPtr3 coords,
@@ -351,18 +344,26 @@ __global__ void __launch_bounds__(kBlock) k_ratios(Grid<D> g, CAxes<D> xc, CPtr3
                                                    RatioKinds r) {
     const int kind = r.kind[blockIdx.y];
     double* const out = r.out[blockIdx.y];
-    if (kind == 0)
+    if constexpr (D == 3) {
+        if (kind >= kEdges) {  // offsets (src/PhaseRatios/midpoints.jl:214-225)
+            const int k = kind - kEdges;
+            const int o[3] = {k != 1 ? 1 : 0, k != 2 ? 1 : 0, k != 0 ? 1 : 0};
+            ratio_midpoint<NP>(g, xc, coords, phases, nph, o, out);
+            return;
+        }
+    }
+    if (kind == kVertices)
         ratio_vertex<D, NP>(g, coords, phases, nph, out);
-    else if (kind < 0)
+    else if (kind == kCentres)
         ratio_center<D, NP>(g, xc, coords, phases, nph, out);
     else
-        ratio_face<D, NP>(g, xc, coords, phases, nph, kind - 1, out);
+        ratio_face<D, NP>(g, xc, coords, phases, nph, kind - kFaces, out);
 }
 
 template <int D, int NP>
 int launch_ratios(jp_ctx* ctx, const Grid<D>& G, const CAxes<D>& xa, const CPtr3& cp,
                   const double* phases, int nph, double* center, double* vertex,
-                  double* const* faces) {
+                  double* const* faces, double* const* midpoints) {
     RatioKinds r{};
     unsigned n = 0;
     auto add = [&](int kind, double* out) {
@@ -370,9 +371,11 @@ int launch_ratios(jp_ctx* ctx, const Grid<D>& G, const CAxes<D>& xa, const CPtr3
         r.kind[n] = kind;
         r.out[n++] = out;
     };
-    add(0, vertex);
-    for (int d = 0; d < D; ++d) add(d + 1, faces ? faces[d] : nullptr);
-    add(-1, center);
+    if (D == 3)
+        for (int k = 0; k < 3; ++k) add(kEdges + k, midpoints ? midpoints[k] : nullptr);
+    add(kVertices, vertex);
+    for (int d = 0; d < D; ++d) add(kFaces + d, faces ? faces[d] : nullptr);
+    add(kCentres, center);
     if (!n) return JP_OK;
     int64_t locations = 1;  // of the vertices, the most
     for (int d = 0; d < D; ++d) locations *= G.ni[d] + 1;
@@ -391,19 +394,11 @@ int run_ratios(jp_ctx* ctx, const jp_cellgrid* gc, const jp_axis* xc, const doub
     for (int d = 0; d < D; ++d) xa.a[d] = Axis{xc[d].x, xc[d].dx, xc[d].inv_dx, xc[d].n};
     CPtr3 cp{{nullptr, nullptr, nullptr}};
     for (int d = 0; d < D; ++d) cp.p[d] = coords[d];
-    int rc = nph <= 4 ? launch_ratios<D, 4>(ctx, G, xa, cp, phases, nph, center, vertex, faces)
-                      : launch_ratios<D, 16>(ctx, G, xa, cp, phases, nph, center, vertex, faces);
+    const int rc = nph <= 4 ? launch_ratios<D, 4>(ctx, G, xa, cp, phases, nph, center, vertex,
+                                                  faces, midpoints)
+                            : launch_ratios<D, 16>(ctx, G, xa, cp, phases, nph, center, vertex,
+                                                   faces, midpoints);
     if (rc) return rc;
-    if constexpr (D == 3) {
-        // xy, yz, xz (src/PhaseRatios/midpoints.jl:214-225)
-        constexpr int OFF[3][3] = {{1, 1, 0}, {0, 1, 1}, {1, 0, 1}};
-        for (int k = 0; k < 3; ++k) {
-            if (!midpoints || !midpoints[k]) continue;
-            k_ratio_midpoint<<<(unsigned)blocks_for(G.C), kBlock, 0, ctx->stream>>>(
-                G, xa, cp, phases, nph, OFF[k][0], OFF[k][1], OFF[k][2], midpoints[k]);
-            JP_LAUNCHED(ctx);
-        }
-    }
     return finish(ctx);
 }
 
