@@ -394,10 +394,15 @@ int run_ratios(jp_ctx* ctx, const jp_cellgrid* gc, const jp_axis* xc, const doub
     for (int d = 0; d < D; ++d) xa.a[d] = Axis{xc[d].x, xc[d].dx, xc[d].inv_dx, xc[d].n};
     CPtr3 cp{{nullptr, nullptr, nullptr}};
     for (int d = 0; d < D; ++d) cp.p[d] = coords[d];
-    const int rc = nph <= 4 ? launch_ratios<D, 4>(ctx, G, xa, cp, phases, nph, center, vertex,
-                                                  faces, midpoints)
-                            : launch_ratios<D, 16>(ctx, G, xa, cp, phases, nph, center, vertex,
-                                                   faces, midpoints);
+    // a slot adds to every phase's sum under its condition, so the sums held are few:
+    // 4, 8 or 16 (38 x 41 x 33 cells, 6 phases: 16 sums 520 us, 8 479)
+    const int rc =
+        nph <= 4   ? launch_ratios<D, 4>(ctx, G, xa, cp, phases, nph, center, vertex, faces,
+                                         midpoints)
+        : nph <= 8 ? launch_ratios<D, 8>(ctx, G, xa, cp, phases, nph, center, vertex, faces,
+                                         midpoints)
+                   : launch_ratios<D, 16>(ctx, G, xa, cp, phases, nph, center, vertex, faces,
+                                          midpoints);
     if (rc) return rc;
     return finish(ctx);
 }
