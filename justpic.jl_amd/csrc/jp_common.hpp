@@ -287,7 +287,8 @@ __device__ inline double lerp_cell(const double (&v)[1 << D], const double (&t)[
 }
 
 // Minimum over the wavefront by data-parallel-primitive shifts (no LDS round
-// trips): within rows of 16 lanes, then across the rows; lane 63 holds it.
+// trips): within rows of 16 lanes, then across the rows; lane 63 holds it, so every
+// lane must be there (in rows of less than 64 cells the last ones may have left).
 __device__ inline uint32_t wave_min(uint32_t v) {
     constexpr int kId = -1;
     auto step = [&](uint32_t o) { v = o < v ? o : v; };
