@@ -13,7 +13,9 @@
 // search's bound reaches it (in the slot-plane layout every particle read is a
 // cache line, and reading all 26 neighbours bound the launch by those
 // requests): the distance to the neighbour's box, which holds all of its
-// particles unless the scan found one outside.  The neighbours that are needed
+// particles unless the scan found one outside, or an earlier colour put one there
+// (a cell's spacing may exceed the distance of its vertices: a range axis has its
+// first spacing for every cell).  The neighbours that are needed
 // are read once for all searches, four at a time, each search's per-lane
 // minimum kept in LDS.  The wavefront minima, the copies of the sources'
 // values (an earlier injection's copy when the source is one) and the stores
@@ -48,7 +50,7 @@ struct InjectCells {
     float* u[3];   // split form: offsets in cell units
     uint8_t* index;
     uint64_t* occw;       // occupancy word of every cell (updated here)
-    const uint32_t* out;  // per cell: a particle lies outside the cell's box (the scan)
+    uint32_t* out;        // per cell: a particle lies outside the cell's box (the scan, updated here)
     int nargs;
     ArgPtrs args;
     int min_q;  // particles wanted per quadrant
@@ -351,6 +353,12 @@ __global__ void __launch_bounds__(kBlock) k_inject_cells(InjectCells<D> a) {
             a.index[e] = 1;
         }
         if (lane == 0) a.occw[c] = occ | injm;  // for the later colours
+        if constexpr (!SPLIT) {  // (a split offset drawn lies in [0, 1])
+            bool out = false;
+#pragma unroll
+            for (int d = 0; d < D; ++d) out = out || !(xv[d] <= q[d] && q[d] <= xw[d]);
+            if (__any(inj && out) && lane == 0) a.out[c] = 1;
+        }
         // values copied from the sources: one load per injection, all in
         // flight together; then the copies in injection order, a source in
         // this cell read from the current values

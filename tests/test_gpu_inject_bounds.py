@@ -1,0 +1,77 @@
+"""Injection where its neighbour search meets particles outside their cells'
+boxes: new particles of a cell whose spacing exceeds the distance of its vertices
+(a range axis carries its first spacing for every cell), of an earlier colour
+than the cell that searches.  FP64 bit for bit against the oracle (runs on an
+MI355X)."""
+import numpy as np
+import pytest
+
+import justpic_hip as jp
+from justpic_hip.grids import Axis, staggered_grid
+from oracle import oracle as O
+
+from test_gpu_inject_cells import cells_of
+from test_gpu_parity import assert_field, assert_state_equal, to_dev
+
+pytestmark = pytest.mark.gpu
+
+
+def narrowing(n):
+    """A range axis of n cells whose first cell is the widest by 2 to 1, or less."""
+    w = np.where(np.arange(n) % 3 == 0, 2.0, np.where(np.arange(n) % 3 == 1, 1.0, 1.4))
+    return Axis(np.concatenate([[0.0], np.cumsum(w)]) / w.sum(), "range")
+
+
+def sparse(n, K, seed):
+    """A particle or none per cell, inside the cell."""
+    xv = tuple(narrowing(m) for m in n)
+    hp = O.HostParticles(xv, K, staggered_grid(xv))
+    rng = np.random.default_rng(seed)
+    e = np.arange(hp.S)
+    occ = (e < hp.C) & (rng.random(hp.S) < 0.6)
+    I = np.unravel_index(e % hp.C, hp.ni, order="F")
+    for d in range(hp.D):
+        a, b = hp.xv[d].x[I[d]], hp.xv[d].x[I[d] + 1]
+        hp.coords[d][:] = np.where(occ, a + rng.uniform(0.05, 0.95, hp.S) * (b - a), np.nan)
+    hp.index[:] = occ
+    fields = [np.where(occ, rng.random(hp.S), np.nan) for _ in range(3)]
+    return hp, fields, rng
+
+
+# (cells, slots, min_xcell, fields)
+CASES = [((7, 8, 5), 16, 8, 1), ((7, 8, 5), 24, 16, 2), ((9, 14), 12, 4, 2), ((9, 14), 24, 16, 3),
+         ((9, 14), 12, 4, 1)]
+
+
+@pytest.mark.parametrize("n,K,mn,nf", CASES)
+def test_new_particles_outside_their_cell(ctx, n, K, mn, nf):
+    print("[gpu-inject-bounds]", n, K, mn, nf, flush=True)
+    hp, fields, _ = sparse(n, K, seed=K + nf)
+    p = to_dev(ctx, hp, min_xcell=mn, seed=5)
+    fd = [cells_of(ctx, hp, a) for a in fields[:nf]]
+    st = jp.inject_particles_(p, tuple(fd), stats=True)
+    so = O.inject_particles(hp, fields[:nf], mn, 5, 0)
+    assert st == so and so["injected"] > 0
+    assert_state_equal(p, hp, exact=True)
+    for a, b in zip(fd, fields):
+        assert_field(a.data.flat(), b, exact=True)
+
+
+@pytest.mark.parametrize("n,K,mn,nf", CASES)
+def test_new_particles_outside_their_cell_phase(ctx, n, K, mn, nf):
+    print("[gpu-inject-bounds] phase", n, K, mn, nf, flush=True)
+    hp, fields, rng = sparse(n, K, seed=K + nf)
+    phases = np.where(hp.index == 1, rng.integers(1, 9, hp.S), np.nan).astype(float)
+    grids = [rng.random(tuple(m + 1 for m in n)) for _ in range(nf)]
+    p = to_dev(ctx, hp, min_xcell=mn, seed=9)
+    ph = cells_of(ctx, hp, phases)
+    fd = [cells_of(ctx, hp, a) for a in fields[:nf]]
+    st = jp.inject_particles_phase_(p, ph, tuple(fd),
+                                    tuple(jp.DeviceArray.from_host(ctx, g) for g in grids),
+                                    stats=True)
+    so = O.inject_particles_phase(hp, phases, fields[:nf], grids, mn, 9, 0)
+    assert st == so and so["injected"] > 0
+    assert_state_equal(p, hp, exact=True)
+    assert_field(ph.data.flat(), phases, exact=True)
+    for a, b in zip(fd, fields):
+        assert_field(a.data.flat(), b, exact=True)
