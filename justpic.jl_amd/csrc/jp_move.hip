@@ -48,6 +48,8 @@ constexpr uint8_t kRare = 0x80;  // re-slotted in its own cell (the centre's cod
 constexpr uint8_t kFar = 0xFF;
 constexpr int kFlagFar = 1;       // a mover jumps more than one cell
 constexpr int kFlagRejected = 2;  // split geometry rejected
+// s_waitcnt immediate of gfx9 for vmcnt(0) with expcnt and lgkmcnt left free
+constexpr int kVmcnt0 = 0x0F70;
 
 __device__ inline double dnan() { return __builtin_nan(""); }
 
@@ -782,9 +784,13 @@ __device__ inline void far_cell(const Grid<D>& g, const MoveScratch& ms, const i
         const int rank = __popcll(stmS & (bit - 1));
         uint32_t origin = S32 * (uint32_t)K + (uint32_t)rank;
         uint32_t cd = kFar;
-        if (arrival)
+        if (arrival) {
             origin = ms.orgf[org_at<D>(S32, (uint32_t)ip, C32, (uint32_t)K)];
-        else if (stmS & bit)
+            // waited for here, on the rare path: otherwise every round of the loop
+            // waits for it, and with it (one counter for loads and stores) for the
+            // stores of the round before (split, 64^3 cells, CFL 2.5: 195 ms a move, now 187)
+            __builtin_amdgcn_s_waitcnt(kVmcnt0);
+        } else if (stmS & bit)
             cd = reinterpret_cast<const uint8_t*>(row)[rank];
         if (selfm & bit) cd = kHere<D>;
         occC &= ~bit;  // empty_particle! on the source slot
