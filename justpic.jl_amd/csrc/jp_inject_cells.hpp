@@ -404,7 +404,8 @@ __global__ void __launch_bounds__(kBlock) k_inject_cells(InjectCells<D> a) {
             copy(ph, 1);
             if (inj) {
                 // args from fields: nodal at this cell's corners, cell-centred
-                // at the shifted index clamped to 1..ni-1 (1-based)
+                // at the shifted index clamped to 1..ni-1 (1-based; a grid of one
+                // cell in a dimension has none, and no cell-centred field)
                 int64_t nnv[D], nnc[D], ic[D], Iv[D];
                 double xc0[D], ivc[D], xv0[D], ivv[D], pn[D];
 #pragma unroll
@@ -415,11 +416,12 @@ __global__ void __launch_bounds__(kBlock) k_inject_cells(InjectCells<D> a) {
                     Iv[d] = I[d];
                     xv0[d] = xv[d];
                     ivv[d] = g.xv[d].idx[I[d]];
-                    int64_t k = pn[d] < xv[d] + dq[d] ? I[d] - 1 : I[d];
-                    k = k > g.ni[d] - 2 ? g.ni[d] - 2 : (k < 0 ? 0 : k);
-                    ic[d] = k;
-                    xc0[d] = a.pi.xc[d].x[k];
-                    ivc[d] = a.pi.xc[d].idx[k];
+                    if (a.pi.centred) {
+                        const int64_t k = pn[d] < xv[d] + dq[d] ? I[d] - 1 : I[d];
+                        ic[d] = k > g.ni[d] - 2 ? g.ni[d] - 2 : (k < 0 ? 0 : k);
+                        xc0[d] = a.pi.xc[d].x[ic[d]];
+                        ivc[d] = a.pi.xc[d].idx[ic[d]];
+                    }
                 }
                 for (int f = 0; f < a.nargs; ++f)
                     a.args.p[f][e] = ((a.pi.centred >> f) & 1)

@@ -1,12 +1,16 @@
 """Injection where its neighbour search meets particles outside their cells'
 boxes: new particles of a cell whose spacing exceeds the distance of its vertices
 (a range axis carries its first spacing for every cell), of an earlier colour
-than the cell that searches.  FP64 bit for bit against the oracle (runs on an
-MI355X)."""
+than the cell that searches; and on grids of one cell in a dimension.  FP64 bit
+for bit against the oracle (runs on an MI355X)."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 import justpic_hip as jp
+from justpic_hip import _abi
+from justpic_hip.particles import DeviceAxis
 from justpic_hip.grids import Axis, staggered_grid
 from oracle import oracle as O
 
@@ -74,4 +78,61 @@ def test_new_particles_outside_their_cell_phase(ctx, n, K, mn, nf):
     assert_state_equal(p, hp, exact=True)
     assert_field(ph.data.flat(), phases, exact=True)
     for a, b in zip(fd, fields):
+        assert_field(a.data.flat(), b, exact=True)
+
+
+@pytest.mark.parametrize("n,K,nf", [((1, 6), 12, 1), ((5, 1), 12, 2), ((1, 1), 8, 0), ((3, 1, 4), 16, 2),
+                                    ((1, 4, 1), 16, 1)])
+def test_phase_one_cell_thick(ctx, n, K, nf):
+    """One cell in a dimension: no cell-centred field is possible and the centre axis
+    has one point and no spacing; phases and nodal fields through the C interface."""
+    print("[gpu-inject-bounds] thin", n, K, nf, flush=True)
+    D, mn = len(n), 8
+    xv = tuple(Axis.lin(0.0, 1.0 + d, m + 1) for d, m in enumerate(n))
+    hp = O.HostParticles(xv, K)
+    rng = np.random.default_rng(K + nf)
+    e = np.arange(hp.S)
+    occ = (e < 2 * hp.C) & (rng.random(hp.S) < 0.5)
+    occ[0] = True
+    I = np.unravel_index(e % hp.C, hp.ni, order="F")
+    for d in range(D):
+        u = rng.uniform(0.05, 0.95, hp.S)
+        hp.coords[d][:] = np.where(occ, xv[d].x[I[d]] + u * xv[d].dx[I[d]], np.nan)
+    hp.index[:] = occ
+    phases = np.where(occ, rng.integers(1, 9, hp.S), np.nan).astype(float)
+    fields = [np.where(occ, rng.random(hp.S), np.nan) for _ in range(nf)]
+    grids = [rng.random(int(np.prod([m + 1 for m in n]))) for _ in range(nf)]
+    cen = (C.c_int * max(1, nf))()
+
+    def centres(arrays):  # x of every centre; spacings that no call has a use for
+        return (_abi.jp_axis * D)(*[_abi.jp_axis(a, b, b, m) for (a, b), m in zip(arrays, n)])
+
+    xc = [(a.x[:-1] + a.x[1:]) / 2 for a in xv]
+    dc = [1.0 / a.dx for a in xv]
+
+    axes = [DeviceAxis(ctx, a) for a in xv]
+    grid = _abi.jp_cellgrid()
+    grid.ndim, grid.max_xcell = D, K
+    for d in range(D):
+        grid.ni[d], grid.xv[d] = n[d], axes[d].abi()
+    dx = [(jp.DeviceArray.from_host(ctx, a), jp.DeviceArray.from_host(ctx, b)) for a, b in zip(xc, dc)]
+    dev = [cells_of(ctx, hp, a) for a in hp.coords + [phases] + fields]
+    index = jp.CellArray(ctx, hp.ni, K, dtype=np.uint8)
+    index.copy_from(hp.index)
+    dg = [jp.DeviceArray.from_host(ctx, a) for a in grids]
+    st = _abi.jp_stats()
+    ctx.check(ctx.lib.jp_inject_particles_phase(
+        ctx.h, C.byref(grid), centres([(a.ptr, b.ptr) for a, b in dx]),
+        _abi.ptr_array([a.ptr for a in dev[:D]]), index.ptr, dev[D].ptr, nf,
+        _abi.ptr_array([a.ptr for a in dev[D + 1:]]), _abi.ptr_array([a.ptr for a in dg]), cen, mn,
+        3, 0, C.byref(st)), "inject_particles_phase!")
+    so = _abi.jp_stats()
+    p = O._p
+    assert O.lib().jpo_inject_particles_phase(
+        C.byref(hp._grid), centres([(p(a), p(b)) for a, b in zip(xc, dc)]), hp.coord_ptrs(),
+        p(hp.index), p(phases), nf, _abi.ptr_array([p(a) for a in fields]),
+        _abi.ptr_array([p(a) for a in grids]), cen, mn, 3, 0, C.byref(so)) == 0
+    assert st.as_dict() == so.as_dict() and so.injected > 0
+    assert np.array_equal(index.data.flat(), hp.index)
+    for a, b in zip(dev, hp.coords + [phases] + fields):
         assert_field(a.data.flat(), b, exact=True)
