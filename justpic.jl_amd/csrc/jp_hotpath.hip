@@ -369,7 +369,9 @@ __global__ void __launch_bounds__(kBlock) k_g2p(Grid<D> g, double* __restrict__ 
 // phases then run the reference loop on those cells only.  ANYQ (the phase
 // variant, which moves on to the next quadrant instead of breaking,
 // src/Particles/injection.jl:278): a cell is listed when any quadrant is short.
-template <int D, bool ANYQ = false>
+// BOX: also whether a particle lies outside the cell's box, for k_inject_cells (in
+// the scan of k_inject2 it took 16.1 us for 12.8 at 32^2).
+template <int D, bool ANYQ, bool BOX>
 __global__ void __launch_bounds__(kBlock) k_inject_scan(Grid<D> g, CPtr3 coords,
                                                         const uint8_t* __restrict__ index,
                                                         int min_q, InjectLists L) {
@@ -385,7 +387,7 @@ __global__ void __launch_bounds__(kBlock) k_inject_scan(Grid<D> g, CPtr3 coords,
 #pragma unroll
         for (int d = 0; d < D; ++d) {
             lo[d] = g.xv[d].x[I[d]];
-            hi[d] = g.xv[d].x[I[d] + 1];
+            hi[d] = BOX ? g.xv[d].x[I[d] + 1] : 0.0;
             hq[d] = g.xv[d].dx[I[d]] / 2.0;
         }
         // quadrant c11: vertex + dq*0 (src/Particles/injection.jl:442-448)
@@ -412,7 +414,7 @@ __global__ void __launch_bounds__(kBlock) k_inject_scan(Grid<D> g, CPtr3 coords,
 #pragma unroll
                 for (int d = 0; d < D; ++d) {
                     inside = inside & (q0[d] < pb[j][d] && pb[j][d] < q1[d]);
-                    out = out || (on && !(lo[d] <= pb[j][d] && pb[j][d] <= hi[d]));
+                    if constexpr (BOX) out = out | (on & !(lo[d] <= pb[j][d] & pb[j][d] <= hi[d]));
                 }
                 num += inside ? 1 : 0;
                 if constexpr (ANYQ) {
@@ -431,7 +433,7 @@ __global__ void __launch_bounds__(kBlock) k_inject_scan(Grid<D> g, CPtr3 coords,
             }
         }
         L.occ[c] = act;
-        if (L.out) L.out[c] = out ? 1u : 0u;
+        if (BOX) L.out[c] = out ? 1u : 0u;
     }
     bool want = valid && num < min_q;
     if constexpr (ANYQ) {
@@ -584,8 +586,12 @@ int run_inject(jp_ctx* ctx, const jp_cellgrid* gc, double* const* coords, uint8_
     const bool two = D == 2 && nargs <= 1;  // the 2D kernel (k_inject2)
     const bool ordered = two && inject2_ordered(ctx);
     if ((rc = inject_lists(ctx, G.C, NQ, cap, ordered, L))) return rc;
-    k_inject_scan<D><<<blocks_for(G.C), kBlock, 0, ctx->stream>>>(G, cptr3(coords, D), index,
-                                                                  min_q, L);
+    if (two)
+        k_inject_scan<D, false, D == 3><<<blocks_for(G.C), kBlock, 0, ctx->stream>>>(
+            G, cptr3(coords, D), index, min_q, L);
+    else
+        k_inject_scan<D, false, true><<<blocks_for(G.C), kBlock, 0, ctx->stream>>>(
+            G, cptr3(coords, D), index, min_q, L);
     JP_LAUNCHED(ctx);
     if ((rc = join_segments(ctx, NQ, L))) return rc;
     jp_stats* st = stats ? dstats(ctx) : nullptr;
@@ -630,8 +636,8 @@ int run_inject_phase(jp_ctx* ctx, const jp_cellgrid* gc, const jp_axis* xc,
     for (int d = 0; d < D; ++d) cap *= (G.ni[d] + 1) / 2;
     InjectLists L;
     if ((rc = inject_lists(ctx, G.C, NQ, cap, false, L))) return rc;
-    k_inject_scan<D, true><<<blocks_for(G.C), kBlock, 0, ctx->stream>>>(G, cptr3(coords, D),
-                                                                        index, min_q, L);
+    k_inject_scan<D, true, true><<<blocks_for(G.C), kBlock, 0, ctx->stream>>>(
+        G, cptr3(coords, D), index, min_q, L);
     JP_LAUNCHED(ctx);
     if ((rc = join_segments(ctx, NQ, L))) return rc;
     InjectCells<D> a = inject_cells<D>(G, coords, index, nargs, args, min_q, seed, counter,

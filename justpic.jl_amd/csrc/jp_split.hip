@@ -579,7 +579,8 @@ __global__ void __launch_bounds__(kBlock) k_g2p_split(Grid<D> g, double* __restr
 // listed cell fills free slots with vertex + dq*muladd(0.95, rand, 0.05)
 // (in cell units: q/2 + muladd(0.95, rand, 0.05)/2) and copies the fields of
 // the nearest particle (distances in physical units, FP64).
-template <int D>
+// BOX: also whether an offset lies outside the cell, for k_inject_cells.
+template <int D, bool BOX>
 __global__ void __launch_bounds__(kBlock) k_inj_scan_split(Grid<D> g, FPtr3 off,
                                                            const uint8_t* __restrict__ index,
                                                            int min_q, InjectLists L,
@@ -609,13 +610,13 @@ __global__ void __launch_bounds__(kBlock) k_inj_scan_split(Grid<D> g, FPtr3 off,
 #pragma unroll
                 for (int d = 0; d < D; ++d) {
                     inside = inside & (0.0f < ub[j][d] && ub[j][d] < 0.5f);
-                    out = out || (on && !(0.0f <= ub[j][d] && ub[j][d] <= 1.0f));
+                    if constexpr (BOX) out = out | (on & !(0.0f <= ub[j][d] & ub[j][d] <= 1.0f));
                 }
                 num += inside ? 1 : 0;
             }
         }
         L.occ[c] = act;
-        if (L.out) L.out[c] = out ? 1u : 0u;
+        if (BOX) L.out[c] = out ? 1u : 0u;
     }
     if (valid && L.state) L.state[c] = num < min_q ? 1u : 0u;
     int col = 0;
@@ -916,8 +917,12 @@ int run_inject(jp_ctx* ctx, const jp_cellgrid* gc, float* const* off, uint8_t* i
     if ((rc = inject_lists(ctx, G.C, NQ, cap, ordered, L))) return rc;
     FPtr3 fp = fptr3<D>(off);
     if ((rc = split_geometry(ctx, gc, nullptr))) return rc;
-    k_inj_scan_split<D><<<blocks_for(G.C), kBlock, 0, ctx->stream>>>(G, fp, index, min_q, L,
-                                                                     geo_ptr(ctx));
+    if (two)
+        k_inj_scan_split<D, D == 3><<<blocks_for(G.C), kBlock, 0, ctx->stream>>>(
+            G, fp, index, min_q, L, geo_ptr(ctx));
+    else
+        k_inj_scan_split<D, true><<<blocks_for(G.C), kBlock, 0, ctx->stream>>>(
+            G, fp, index, min_q, L, geo_ptr(ctx));
     JP_LAUNCHED(ctx);
     if ((rc = join_segments(ctx, NQ, L))) return rc;
     jp_stats* st = stats ? dstats(ctx) : nullptr;

@@ -136,3 +136,70 @@ def test_phase_one_cell_thick(ctx, n, K, nf):
     assert np.array_equal(index.data.flat(), hp.index)
     for a, b in zip(dev, hp.coords + [phases] + fields):
         assert_field(a.data.flat(), b, exact=True)
+
+
+def nearest_copies(before, after, u, fields, n, K, h):
+    """Values of the new particles' fields: colours in order, slots of a cell in order,
+    each copied from its nearest particle (offsets u; neighbour cell, then slot, on
+    equal distances).  Also how many of the sources lie outside their cell."""
+    D, C_ = len(n), int(np.prod(n))
+    act, u = before.copy(), [a.astype(np.float64) for a in u]
+    out, outside = [f.copy() for f in fields], 0
+    cells = np.stack(np.unravel_index(np.arange(C_), n, order="F"), 1)
+    for col in range(2 ** D):
+        odd = [(col >> (D - 1 - d)) & 1 for d in range(D)]
+        for c in np.nonzero((cells % 2 == odd).all(1))[0]:
+            for k in np.nonzero(after[c::C_] & ~before[c::C_])[0]:
+                e = c + C_ * k
+                src, best = -1, np.inf
+                for nb in range(3 ** D):
+                    o = [(nb // 3 ** d) % 3 - 1 for d in range(D)]
+                    J = cells[c] + o
+                    if (J < 0).any() or (J >= n).any():
+                        continue
+                    j = int(np.ravel_multi_index(J, n, order="F")) + C_ * np.arange(K)
+                    s = 0.0
+                    for d in range(D):
+                        r = (o[d] + u[d][j] - u[d][e]) * h[d]
+                        s = s + r * r
+                    s = np.where(act[j] & ~np.isnan(s), np.sqrt(s), np.inf)
+                    q = int(np.argmin(s))
+                    if s[q] < best:
+                        src, best = int(j[q]), s[q]
+                if src >= 0:
+                    outside += any(not 0 <= u[d][src] <= 1 for d in range(D))
+                    for f in out:
+                        f[e] = f[src]
+                act[e] = True
+    return out, outside
+
+
+@pytest.mark.parametrize("n,K,mn,nf", [((7, 6, 5), 24, 14, 1), ((5, 4, 6), 40, 32, 2),
+                                       ((13, 11), 20, 12, 2), ((9, 14), 64, 48, 3)])
+def test_split_particles_outside_their_cell(ctx, n, K, mn, nf):
+    """Split offsets up to two cells out (advected and not moved) and NaN."""
+    print("[gpu-inject-bounds] split", n, K, mn, nf, flush=True)
+    xv = tuple(Axis.lin(0.0, 1.0, m + 1) for m in n)
+    hp = O.HostParticles(xv, K, staggered_grid(xv))
+    rng = np.random.default_rng(K + nf)
+    fill = rng.choice([0.0, 0.05, 0.3, 0.9], hp.C, p=[0.25, 0.3, 0.35, 0.1])
+    occ = rng.random(hp.S) < fill[np.arange(hp.S) % hp.C]
+    I = np.unravel_index(np.arange(hp.S) % hp.C, hp.ni, order="F")
+    for d in range(hp.D):  # (any place inside the cell: the offsets are replaced below)
+        hp.coords[d][:] = np.where(occ, xv[d].x[I[d]] + 0.5 * xv[d].dx[I[d]], np.nan)
+    hp.index[:] = occ
+    s = jp.to_split(to_dev(ctx, hp, min_xcell=mn, seed=5))
+    for a in s.coords:
+        u = rng.uniform(0.0, 1.0, hp.S) + rng.choice([0, 0, 0, -2, -1, 1, 2], hp.S)
+        u = np.where(rng.random(hp.S) < 0.01, np.nan, u)
+        a.copy_from(np.where(occ, u, np.nan).astype(np.float32))
+    fields = [np.where(occ, rng.random(hp.S), np.nan) for _ in range(nf)]
+    fd = [cells_of(ctx, hp, a) for a in fields]
+    st = jp.inject_particles_(s, tuple(fd), stats=True)
+    after = s.index.data.flat().astype(bool)
+    assert st["injected"] == (after & ~occ).sum() > 0
+    want, outside = nearest_copies(occ, after, [a.data.flat() for a in s.coords], fields, hp.ni, K,
+                                   [a.dx[0] for a in xv])
+    assert outside > 0
+    for a, b in zip(fd, want):
+        assert_field(a.data.flat(), b, exact=True)
