@@ -8,11 +8,11 @@
 // nodes, and its axis windows, staged in LDS; the wavefronts walk the cells'
 // slots in lockstep chunks of planes (k_advect_tile, all three schemes).  A
 // particle with a stage point outside a window is advected on the slot path
-// after the tile's others.  The slot path (also k_advect_slot): the velocity
-// gathered from global memory.  A bracket lookup costs one guess (uniform
-// spacing estimate; in the windows of refined axes a short search from the
-// particle's cell) and one strict test against the stored axis, with the
-// reference search for everything else (ties).
+// after the others.  The slot path: the velocity gathered from global memory
+// (also k_advect_slot, one thread per slot, for MQS and LinP on small grids).
+// A bracket lookup costs one guess (uniform spacing estimate; in the windows
+// of refined axes a short search from the particle's cell) and one strict test
+// against the stored axis, with the reference search for everything else (ties).
 #include "jp_ctx.hpp"
 
 #include <type_traits>
@@ -505,10 +505,14 @@ __device__ inline bool interp_tile_f64(const TileLds<D, S>& L, const TileWin<D>&
 
 // B: slot planes per chunk.  A particle whose step leaves the windows (or
 // sits on a node) is marked in its cell's word and advected as k_advect_slot
-// does after the tile's other particles: inside the chunk loop that path costs
-// the loop's occupancy (2D RK2 169 registers, two wavefronts per SIMD instead
-// of four: 165 us against 98 at 512^2), and a flag per slot with a pass of its
-// own costs a launch.
+// does after the wavefront's other particles, dealt to the lanes in the same
+// way: inside the chunk loop that path costs the loop's occupancy (2D RK2 169
+// registers, two wavefronts per SIMD instead of four: 165 us against 98 at
+// 512^2), and a flag per slot with a pass of its own costs a launch.  When most
+// of a chunk's first 64 particles miss, the steps are longer than the windows'
+// margin and the wavefront's other slots are marked untried.  Steps of 6 cells at
+// 256^2: MQS RK4 149 us, linear RK4 on refined axes 313 (each cell's particles one
+// after the other by its own lane, the windows tried for all: 261 and 641).
 template <int D, int M, int S, int B>
 __global__ void __launch_bounds__(kBlock, D == 2 ? 4 : 2) k_advect_tile(Grid<D> g, Vel<D> vg, VPtrs<D> V,
                                                         Ptr3 coords,
@@ -650,6 +654,20 @@ __global__ void __launch_bounds__(kBlock, D == 2 ? 4 : 2) k_advect_tile(Grid<D> 
     __shared__ uint16_t s_items[kBlock / 64][B * 64];
     uint16_t* items = s_items[tid >> 6];
     const int lane = tid & 63, wbase = tid & ~63;
+    // the entries (slot in the chunk << 6 | lane) of the set bits of slots k0 ..
+    auto list = [&](uint64_t bits, int k0) {
+        int n = 0;
+#pragma unroll
+        for (int j = 0; j < B; ++j) {
+            const bool a = k0 + j < 64 && ((bits >> (k0 + j)) & 1);
+            const uint64_t bal = __ballot(a);
+            const int below = (int)__builtin_amdgcn_mbcnt_hi(
+                (uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+            if (a) items[n + below] = (uint16_t)((j << 6) | lane);
+            n += __popcll(bal);
+        }
+        return n;
+    };
     auto chunks = [&](auto ref) {
         auto interp = [&](const double (&p)[D], double (&v)[D]) {
 #pragma unroll
@@ -658,16 +676,7 @@ __global__ void __launch_bounds__(kBlock, D == 2 ? 4 : 2) k_advect_tile(Grid<D> 
                       win;
         };
         for (int k0 = kb; k0 < ke; k0 += B) {
-            int n = 0;
-#pragma unroll
-            for (int j = 0; j < B; ++j) {
-                const bool a = k0 + j < 64 && ((act >> (k0 + j)) & 1);
-                const uint64_t bal = __ballot(a);
-                const int below = (int)__builtin_amdgcn_mbcnt_hi(
-                    (uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-                if (a) items[n + below] = (uint16_t)((j << 6) | lane);
-                n += __popcll(bal);
-            }
+            const int n = list(act, k0);
             if (!n) continue;
             // this lane's entries lane, lane + 64, ...: positions loaded first
             double pq[B][D];
@@ -682,6 +691,7 @@ __global__ void __launch_bounds__(kBlock, D == 2 ? 4 : 2) k_advect_tile(Grid<D> 
 #pragma unroll
                 for (int d = 0; d < D; ++d) pq[q][d] = dq[q] >= 0 ? coords.p[d][e] : 0.0;
             }
+            bool missed = false;  // the lane's first entry
 #pragma unroll
             for (int q = 0; q < B; ++q) {
                 if (dq[q] < 0) break;
@@ -694,30 +704,41 @@ __global__ void __launch_bounds__(kBlock, D == 2 ? 4 : 2) k_advect_tile(Grid<D> 
                 for (int d = 0; d < D; ++d) cell[d] = (int)(J[d] - t0[d]);
                 advect_rk<D, M>(P, pq[q], out, interp);
                 if (!win) {
+                    if (q == 0) missed = true;
                     atomicOr(&s_miss[wbase + (dq[q] & 63)], 1ull << (k0 + (dq[q] >> 6)));
                     continue;
                 }
 #pragma unroll
                 for (int d = 0; d < D; ++d) coords.p[d][e] = out[d];
             }
+            // most first entries missed: the other slots would too
+            if (2 * __popcll(__ballot(missed)) > (n < 64 ? n : 64)) {
+                if (k0 + B < 64) s_miss[tid] |= act & ~((1ull << (k0 + B)) - 1);
+                break;
+            }
         }
     };
     if (refined) chunks(std::true_type{});
     else chunks(std::false_type{});
-    __syncthreads();
-    uint64_t miss = inside ? s_miss[tid] : 0;
-    if (!miss) return;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (the words are the wavefront's own)
+    const uint64_t miss = s_miss[tid];
+    if (!__any(miss != 0)) return;
     AxisGuess<D> Gs;
     axis_guess<D>(vg, Gs);
-    while (miss) {
-        const int64_t e = c + C * __builtin_ctzll(miss);
-        miss &= miss - 1;
-        double p0[D], out[D];
+    for (int k0 = kb; k0 < ke; k0 += B) {
+        const int n = list(miss, k0);
+        for (int i = lane; i < n; i += 64) {
+            const int item = items[i];
+            int64_t J[D];
+            cell_of(wbase + (item & 63), J);
+            const int64_t e = lin<D>(g.ni, J) + C * (k0 + (item >> 6));
+            double p0[D], out[D];
 #pragma unroll
-        for (int d = 0; d < D; ++d) p0[d] = coords.p[d][e];
-        advect_slot<D, M, S>(Gs, vg, V, P, p0, I, out);
+            for (int d = 0; d < D; ++d) p0[d] = coords.p[d][e];
+            advect_slot<D, M, S>(Gs, vg, V, P, p0, J, out);
 #pragma unroll
-        for (int d = 0; d < D; ++d) coords.p[d][e] = out[d];
+            for (int d = 0; d < D; ++d) coords.p[d][e] = out[d];
+        }
     }
 }
 
