@@ -271,19 +271,23 @@ __device__ inline void adv_split_tile(const SGrid<D>& g, const SVelIn<D>& V, con
     s_miss[tid][0] = s_miss[tid][1] = 0;
     int n = 0;  // entries waiting
     int k0 = kb;
+    // the entries of the set bits of slots k .. k + CH - 1, from items[n]
+    auto list = [&](uint64_t bits, int k) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            const bool a = k + j < 64 && ((bits >> (k + j)) & 1);
+            const uint64_t bal = __ballot(a);
+            const int below = (int)__builtin_amdgcn_mbcnt_hi(
+                (uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
+            if (a) items[n + below] = (uint16_t)(((k + j) << 6) | lane);
+            n += __popcll(bal);
+        }
+    };
     // the next groups: their entries and positions (past the end the last entry,
     // whose result is not stored)
     auto next = [&](int (&dq)[G], float (&uq)[G][D]) __attribute__((always_inline)) {
         while (n < 64 * G && k0 < ke) {
-#pragma unroll
-            for (int j = 0; j < CH; ++j) {
-                const bool a = k0 + j < 64 && ((act >> (k0 + j)) & 1);
-                const uint64_t bal = __ballot(a);
-                const int below = (int)__builtin_amdgcn_mbcnt_hi(
-                    (uint32_t)(bal >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)bal, 0u));
-                if (a) items[n + below] = (uint16_t)(((k0 + j) << 6) | lane);
-                n += __popcll(bal);
-            }
+            list(act, k0);
             k0 += CH;
         }
         const int take = n < 64 * G ? n : 64 * G;
@@ -303,11 +307,20 @@ __device__ inline void adv_split_tile(const SGrid<D>& g, const SVelIn<D>& V, con
     float uq[G][D], un[G][D];
     int dq[G], dn[G];
     int take = __any(act != 0) ? next(dq, uq) : 0;
+    auto missed = [&](int item) __attribute__((always_inline)) {
+        atomicOr(&s_miss[wave * 64 + (item & 63)][item >> 11], 1u << ((item >> 6) & 31));
+    };
     while (take) {
         const int then = next(dn, un);
+        bool far = false;  // most of the first 64 missed: the others would too
 #pragma unroll
         for (int q = 0; q < G; ++q) {
             if (64 * q >= take) break;
+            const bool mine = lane + 64 * q < take;
+            if (far) {
+                if (mine) missed(dq[q]);
+                continue;
+            }
             const int l = dq[q] & 63;
             int J[D];
             J[0] = w[0] + l % N0;
@@ -318,15 +331,26 @@ __device__ inline void adv_split_tile(const SGrid<D>& g, const SVelIn<D>& V, con
             float out[D];
             const bool ok = advect_split_one<D, M>(WindowVelocity<D, TS>{sV, W, J, cm}, P, uq[q],
                                                    out);
-            if (lane + 64 * q < take) {
+            if (q == 0) far = 2 * __popcll(__ballot(mine && !ok)) > (take < 64 ? take : 64);
+            if (mine) {
                 if (ok) {
                     const uint64_t e = at(dq[q]);
 #pragma unroll
                     for (int d = 0; d < D; ++d) base[d][e] = out[d];
                 } else {
-                    atomicOr(&s_miss[tid - lane + l][dq[q] >> 11], 1u << ((dq[q] >> 6) & 31));
+                    missed(dq[q]);
                 }
             }
+        }
+        if (far) {
+#pragma unroll
+            for (int q = 0; q < G; ++q)
+                if (lane + 64 * q < then) missed(dn[q]);
+            for (int i = lane; i < n; i += 64) missed(items[i]);
+            const uint64_t rest = k0 < 64 ? act & ~((1ull << k0) - 1) : 0ull;
+            if ((uint32_t)rest) atomicOr(&s_miss[tid][0], (uint32_t)rest);
+            if (rest >> 32) atomicOr(&s_miss[tid][1], (uint32_t)(rest >> 32));
+            break;
         }
         take = then;
 #pragma unroll
@@ -336,25 +360,37 @@ __device__ inline void adv_split_tile(const SGrid<D>& g, const SVelIn<D>& V, con
             for (int d = 0; d < D; ++d) uq[q][d] = un[q][d];
         }
     }
-    // those, each by its cell's lane (inside the loop above, the global path took
-    // half its code and a quarter of its registers: 104 for 78)
-    uint64_t miss = ((uint64_t)s_miss[tid][1] << 32) | s_miss[tid][0];
-    while (miss) {
-        const int k = __builtin_ctzll(miss);
-        miss &= miss - 1;
-        int J[D];
-        J[0] = w[0] + lane % N0;
-        J[1] = w[1] + lane / N0;
-        if constexpr (D == 3) J[2] = w[2];
-        CellMap<D> cm;
-        cell_map<D, STD>(m, J, cm);
-        const uint64_t e = at((k << 6) | lane);
-        float u[D], out[D];
+    // those, dealt in the same way, each stage from the windows where they hold it
+    // (inside the loop above, the global path took half its code and a quarter of its
+    // registers: 104 for 78).  Steps of 6 cells, RK4 at 512^2: 101 us (each cell's
+    // particles one after the other by its own lane, whole steps from global memory,
+    // the windows tried for all: 194).
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (the words are the wavefront's own)
+    const uint64_t miss = ((uint64_t)s_miss[tid][1] << 32) | s_miss[tid][0];
+    if (!__any(miss != 0)) return;
+    for (k0 = kb; k0 < ke; k0 += CH) {
+        n = 0;
+        list(miss, k0);
+        for (int i = lane; i < n; i += 64) {
+            const int item = items[i], l = item & 63;
+            int J[D];
+            J[0] = w[0] + l % N0;
+            J[1] = w[1] + l / N0;
+            if constexpr (D == 3) J[2] = w[2];
+            CellMap<D> cm;
+            cell_map<D, STD>(m, J, cm);
+            const uint64_t e = at(item);
+            float u[D], out[D];
 #pragma unroll
-        for (int d = 0; d < D; ++d) u[d] = base[d][e];
-        advect_split_one<D, M>(GlobalVelocity<D>{V, sc, J, cm}, P, u, out);
+            for (int d = 0; d < D; ++d) u[d] = base[d][e];
+            const WindowVelocity<D, TS> near{sV, W, J, cm};
+            const GlobalVelocity<D> any{V, sc, J, cm};
+            advect_split_one<D, M>(
+                [&](const float (&p)[D], float (&v)[D]) { return near(p, v) || any(p, v); }, P, u,
+                out);
 #pragma unroll
-        for (int d = 0; d < D; ++d) base[d][e] = out[d];
+            for (int d = 0; d < D; ++d) base[d][e] = out[d];
+        }
     }
 }
 
