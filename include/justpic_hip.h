@@ -114,10 +114,10 @@ void* jp_ctx_stream(jp_ctx* ctx);
  *   JP_OPT_MOVE_PHASES  the 2D move's colour phases: 0 (default) all nine in
  *                       one launch over tiles of cells, 1 one launch per
  *                       phase (the form the 3D move always takes).
- *   JP_OPT_ADVECT_SLOTS the FP64 advection with the linear interpolation: 0
- *                       (default) tiles of cells with the velocity staged
- *                       in LDS, 1 one thread per slot gathering from global
- *                       memory (the form the MQS and LinP schemes take).
+ *   JP_OPT_ADVECT_SLOTS the FP64 advection: 0 (default) tiles of cells with
+ *                       the velocity staged in LDS (MQS and LinP: on grids
+ *                       with enough slots), 1 one thread per slot gathering
+ *                       from global memory.
  * No reference counterpart (the KernelAbstractions launch sizes of the
  * reference are chosen by its backend). */
 #define JP_OPT_SLOT_SPAN 1

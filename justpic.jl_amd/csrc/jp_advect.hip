@@ -834,7 +834,14 @@ Vel<D> to_vel(const jp_velgrid* vg) {
 template <int D, int M, int S>
 int launch(jp_ctx* ctx, const Grid<D>& G, const Vel<D>& vg, const VPtrs<D>& V, Ptr3 cp,
            const uint8_t* index, const RKParams& P) {
-    if (!ctx->opt_advect_slots) {
+    // MQS and LinP: a thread per slot where the slots are few (a wavefront per row of 64
+    // cells and slot plane, up to 40 per CU, more than it holds at once); a tile's chain
+    // of windows and chunks is then longer than the gathers from global memory.  Tiles
+    // and slots, MQS RK2 in us: 64^2 cells of 48 slots (3072 wavefronts) 22 and 7, 96^2
+    // (9216) 26 and 22, 128^2 (12288) 30 and 29, 160^2 (23040) 35 and 52; 3D 20^3 of 24
+    // (9600) 53 and 40, 12^3 of 54 (7776) 44 and 49, 20^3 of 54 (21600) 60 and 104.
+    const bool few = S != kLinear && row_count<D>(G) * G.K <= (int64_t)40 * ctx->num_cu;
+    if (!ctx->opt_advect_slots && !few) {
         int64_t tiles = 1;
         for (int d = 0; d < D; ++d)
             tiles *= (G.ni[d] + F64Tile<D>::n[d] - 1) / F64Tile<D>::n[d];
