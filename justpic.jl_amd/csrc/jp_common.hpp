@@ -241,8 +241,21 @@ __device__ inline uint64_t active_slots_in(const uint8_t* __restrict__ index, in
 }
 
 // ---- grid to particles: a thread takes kSlots8 slots of its cell (grid2particle_flip!,
-// with more values per slot, half of them)
+// with more values per slot, half of them; on small grids 2)
 constexpr int kSlots8 = 8;
+
+// Active slots kb .. kb + N - 1 of cell c, bit j slot kb + j.
+template <int N>
+__device__ inline uint32_t slots_on(const uint8_t* __restrict__ index, int64_t c, int64_t C,
+                                    int kb, int K) {
+    const int ke = kb + N < K ? kb + N : K;
+    if constexpr (N >= 4) return (uint32_t)(active_slots_in(index, c, C, kb, ke) >> kb);
+    uint32_t bits = 0;
+#pragma unroll
+    for (int j = 0; j < N; ++j)
+        bits |= (uint32_t)(index[c + C * (kb + j < ke ? kb + j : ke - 1)] != 0 && kb + j < ke) << j;
+    return bits;
+}
 
 // The positions (or any D arrays) of slots kb.. of cell c, those of a slot plane
 // in which the wavefront has an active slot: unguarded but for that (uniform), so

@@ -194,6 +194,16 @@ inline int slot_span(const jp_ctx* ctx, int64_t blocks, int K, int64_t target = 
 
 int check_grid(jp_ctx* ctx, const jp_cellgrid* g);
 
+// Slots per thread of the grid-to-particle kernels: kSlots8, or 2 where that would
+// leave fewer than 12 wavefronts per CU (6 of 48 slots at 128^2 cells: with 8 and 2
+// grid2particle 5.5 and 4.9 us, split 6.2 and 4.8, centroid2particle 7.6 and 7.0; at
+// 512 x 384, 72 wavefronts per CU, 8 take 40 for 52 of a thread per slot)
+template <int D>
+inline int slots_per_thread(const jp_ctx* ctx, const Grid<D>& g) {
+    const int64_t waves = row_count<D>(g) * ((g.K + kSlots8 - 1) / kSlots8);
+    return waves < (int64_t)12 * ctx->num_cu ? 2 : kSlots8;
+}
+
 template <int D>
 Grid<D> to_grid(const jp_cellgrid* g) {
     Grid<D> G;

@@ -333,13 +333,13 @@ __global__ void __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, 
 // takes 8 slots of its cell (blockIdx.y): the cell's corners and vertices are read
 // once, and the slots' loads are in flight together (bound by the slots' bytes:
 // 512 x 384 cells of 48 slots 52 us with a thread per slot, now 40).
-template <int D>
+template <int D, int NS>
 __global__ void __launch_bounds__(kBlock) k_g2p(Grid<D> g, double* __restrict__ Fp,
                                                 const double* __restrict__ F, CPtr3 coords,
                                                 const uint8_t* __restrict__ index) {
     int64_t c, I[D];
     if (!row_cell<D>(g, c, I)) return;
-    const int kb = (int)blockIdx.y * kSlots8, ke = kb + kSlots8 < g.K ? kb + kSlots8 : g.K;
+    const int kb = (int)blockIdx.y * NS;
     double v[1 << D], x[D], ix[D];
     cell_corners<D>(g, F, I, v);
 #pragma unroll
@@ -347,11 +347,11 @@ __global__ void __launch_bounds__(kBlock) k_g2p(Grid<D> g, double* __restrict__ 
         x[d] = g.xv[d].x[I[d]];
         ix[d] = g.xv[d].idx[I[d]];
     }
-    const uint32_t on = (uint32_t)(active_slots_in(index, c, g.C, kb, ke) >> kb);
-    double p[kSlots8][D];
-    load_slots<D, kSlots8>(coords, c, g.C, kb, on, p);
+    const uint32_t on = slots_on<NS>(index, c, g.C, kb, g.K);
+    double p[NS][D];
+    load_slots<D, NS>(coords, c, g.C, kb, on, p);
 #pragma unroll
-    for (int j = 0; j < kSlots8; ++j) {
+    for (int j = 0; j < NS; ++j) {
         if (!((on >> j) & 1)) continue;
         double t[D];
 #pragma unroll
@@ -547,8 +547,12 @@ template <int D>
 int run_g2p(jp_ctx* ctx, const jp_cellgrid* g, double* Fp, const double* F,
             const double* const* coords, const uint8_t* index) {
     Grid<D> G = to_grid<D>(g);
-    const dim3 grid((unsigned)row_blocks<D>(G), (unsigned)((G.K + kSlots8 - 1) / kSlots8));
-    k_g2p<D><<<grid, kBlock, 0, ctx->stream>>>(G, Fp, F, cptr3(coords, D), index);
+    const int ns = slots_per_thread(ctx, G);
+    const dim3 grid((unsigned)row_blocks<D>(G), (unsigned)((G.K + ns - 1) / ns));
+    if (ns == 2)
+        k_g2p<D, 2><<<grid, kBlock, 0, ctx->stream>>>(G, Fp, F, cptr3(coords, D), index);
+    else
+        k_g2p<D, kSlots8><<<grid, kBlock, 0, ctx->stream>>>(G, Fp, F, cptr3(coords, D), index);
     JP_LAUNCHED(ctx);
     return finish(ctx);
 }

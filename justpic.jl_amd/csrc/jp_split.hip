@@ -587,20 +587,20 @@ __global__ void __launch_bounds__(kBlock) k_p2g_split_nodes(Grid<D> gg, SGrid<D>
 }
 
 // ------------------------------------------------------------ grid2particle
-template <int D>
+template <int D, int NS>
 __global__ void __launch_bounds__(kBlock) k_g2p_split(Grid<D> g, double* __restrict__ Fp,
                                                       const double* __restrict__ F, FPtr3 off,
                                                       const uint8_t* __restrict__ index) {
     int64_t c, I[D];
     if (!row_cell<D>(g, c, I)) return;
-    const int kb = (int)blockIdx.y * kSlots8, ke = kb + kSlots8 < g.K ? kb + kSlots8 : g.K;
+    const int kb = (int)blockIdx.y * NS;
     double v[1 << D];
     cell_corners<D>(g, F, I, v);
-    const uint32_t on = (uint32_t)(active_slots_in(index, c, g.C, kb, ke) >> kb);
-    float u[kSlots8][D];
-    load_slots<D, kSlots8>(off, c, g.C, kb, on, u);
+    const uint32_t on = slots_on<NS>(index, c, g.C, kb, g.K);
+    float u[NS][D];
+    load_slots<D, NS>(off, c, g.C, kb, on, u);
 #pragma unroll
-    for (int j = 0; j < kSlots8; ++j) {
+    for (int j = 0; j < NS; ++j) {
         if (!((on >> j) & 1)) continue;
         double t[D];
 #pragma unroll
@@ -930,8 +930,12 @@ template <int D>
 int run_g2p(jp_ctx* ctx, const jp_cellgrid* gc, double* Fp, const double* F, float* const* off,
             const uint8_t* index) {
     Grid<D> G = to_grid<D>(gc);
-    const dim3 grid((unsigned)row_blocks<D>(G), (unsigned)((G.K + kSlots8 - 1) / kSlots8));
-    k_g2p_split<D><<<grid, kBlock, 0, ctx->stream>>>(G, Fp, F, fptr3<D>(off), index);
+    const int ns = slots_per_thread(ctx, G);
+    const dim3 grid((unsigned)row_blocks<D>(G), (unsigned)((G.K + ns - 1) / ns));
+    if (ns == 2)
+        k_g2p_split<D, 2><<<grid, kBlock, 0, ctx->stream>>>(G, Fp, F, fptr3<D>(off), index);
+    else
+        k_g2p_split<D, kSlots8><<<grid, kBlock, 0, ctx->stream>>>(G, Fp, F, fptr3<D>(off), index);
     JP_LAUNCHED(ctx);
     return finish(ctx);
 }

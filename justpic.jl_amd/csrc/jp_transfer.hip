@@ -72,8 +72,8 @@ __global__ void __launch_bounds__(kBlock) k_g2p_flip(Grid<D> g, int nf, ArgPtrs 
                                                      const double* __restrict__ h) {
     int64_t c, I[D];
     if (!row_cell<D>(g, c, I)) return;
-    const int kb = (int)blockIdx.y * kSlotsFlip, ke = kb + kSlotsFlip < g.K ? kb + kSlotsFlip : g.K;
-    const uint32_t on = (uint32_t)(active_slots_in(index, c, g.C, kb, ke) >> kb);
+    const int kb = (int)blockIdx.y * kSlotsFlip;
+    const uint32_t on = slots_on<kSlotsFlip>(index, c, g.C, kb, g.K);
     if (!__ballot(on != 0)) return;
     double t[kSlotsFlip][D];
     load_slots<D, kSlotsFlip>(coords, c, g.C, kb, on, t);
@@ -189,15 +189,15 @@ __global__ void __launch_bounds__(kBlock) k_p2c(Grid<D> g, CAxes<D> xc, int nf, 
 // takes 8 slots of its cell; shifted_index against xci[I], clamped to 1..ni-1
 // (1-based), lerp of the centred field's corners (512 x 384 cells of 48 slots: a
 // thread per slot 67 us, 51)
-template <int D>
+template <int D, int NS>
 __global__ void __launch_bounds__(kBlock) k_c2p(Grid<D> g, CAxes<D> xc, int nf, ArgPtrs Fp,
                                                 FieldPtrs F, CPtr3 coords) {
     int64_t c, I[D];
     if (!row_cell<D>(g, c, I)) return;
-    const int kb = (int)blockIdx.y * kSlots8;
-    double p[kSlots8][D];
+    const int kb = (int)blockIdx.y * NS;
+    double p[NS][D];
 #pragma unroll
-    for (int j = 0; j < kSlots8; ++j) {
+    for (int j = 0; j < NS; ++j) {
         const int64_t e = c + g.C * (kb + j < g.K ? kb + j : g.K - 1);
 #pragma unroll
         for (int d = 0; d < D; ++d) p[j][d] = coords.p[d][e];
@@ -219,7 +219,7 @@ __global__ void __launch_bounds__(kBlock) k_c2p(Grid<D> g, CAxes<D> xc, int nf, 
         }
     }
 #pragma unroll
-    for (int j = 0; j < kSlots8; ++j) {
+    for (int j = 0; j < NS; ++j) {
         bool nan = kb + j >= g.K;
 #pragma unroll
         for (int d = 0; d < D; ++d) nan = nan || p[j][d] != p[j][d];
@@ -293,6 +293,20 @@ int run_flip(jp_ctx* ctx, const jp_cellgrid* gc, int nf, double* const* Fp, cons
     return finish(ctx);
 }
 
+template <int D>
+void launch_c2p(jp_ctx* ctx, const jp_cellgrid* gc, const jp_axis* xc, int nf, double* const* Fp,
+                const double* const* F, const double* const* coords) {
+    const Grid<D> G = to_grid<D>(gc);
+    const int ns = slots_per_thread(ctx, G);
+    const dim3 grid((unsigned)row_blocks<D>(G), (unsigned)((G.K + ns - 1) / ns));
+    if (ns == 2)
+        k_c2p<D, 2><<<grid, kBlock, 0, ctx->stream>>>(G, caxes<D>(xc), nf, argptrs(Fp, nf),
+                                                      fieldptrs(F, nf), cptr3(coords, D));
+    else
+        k_c2p<D, kSlots8><<<grid, kBlock, 0, ctx->stream>>>(G, caxes<D>(xc), nf, argptrs(Fp, nf),
+                                                            fieldptrs(F, nf), cptr3(coords, D));
+}
+
 }  // namespace
 
 extern "C" {
@@ -349,15 +363,10 @@ int jp_centroid2particle(jp_ctx* ctx, const jp_cellgrid* g, const jp_axis* xc, i
     if ((rc = check_arrays(ctx, g->ndim, (const void* const*)coords, "coords"))) return rc;
     if ((rc = check_arrays(ctx, nfields, (const void* const*)F, "F"))) return rc;
     if ((rc = check_arrays(ctx, nfields, (const void* const*)Fp, "Fp"))) return rc;
-    if (g->ndim == 2) {
-        Grid<2> G = to_grid<2>(g);
-        k_c2p<2><<<dim3((unsigned)row_blocks<2>(G), (unsigned)((G.K + kSlots8 - 1) / kSlots8)), kBlock, 0, ctx->stream>>>(
-            G, caxes<2>(xc), nfields, argptrs(Fp, nfields), fieldptrs(F, nfields), cptr3(coords, 2));
-    } else {
-        Grid<3> G = to_grid<3>(g);
-        k_c2p<3><<<dim3((unsigned)row_blocks<3>(G), (unsigned)((G.K + kSlots8 - 1) / kSlots8)), kBlock, 0, ctx->stream>>>(
-            G, caxes<3>(xc), nfields, argptrs(Fp, nfields), fieldptrs(F, nfields), cptr3(coords, 3));
-    }
+    if (g->ndim == 2)
+        launch_c2p<2>(ctx, g, xc, nfields, Fp, F, coords);
+    else
+        launch_c2p<3>(ctx, g, xc, nfields, Fp, F, coords);
     JP_LAUNCHED(ctx);
     return finish(ctx);
 }
