@@ -180,6 +180,9 @@ __device__ inline bool interp_window(const float (*sV)[TS::size()], const SWindo
 #pragma unroll
     for (int d = 1; d < D; ++d) far += fabsf(u[d]);
     bool ok = far < 1.0e5f;
+    float q0[D];  // (what the conversions below are defined for)
+#pragma unroll
+    for (int d = 0; d < D; ++d) q0[d] = ok ? u[d] : 0.0f;
     int b[D];
     float t[D][D];
 #pragma unroll
@@ -187,7 +190,7 @@ __device__ inline bool interp_window(const float (*sV)[TS::size()], const SWindo
         int k[D];
 #pragma unroll
         for (int d = 0; d < D; ++d) {
-            const float s = fmaf(u[d], cm.r[c][d], cm.ef[c][d]);
+            const float s = fmaf(q0[d], cm.r[c][d], cm.ef[c][d]);
             const float fl = floorf(s);
             t[c][d] = s - fl;
             k[d] = (I[d] - W.w0[c][d]) + cm.ei[c][d] + (int)fl;
