@@ -517,8 +517,9 @@ int run_p2g(jp_ctx* ctx, const jp_cellgrid* g, int nf, double* const* F, const d
     // with R = 1): 187, 180, 157, 190 us; 389 x 211, three fields (1292): 104,
     // 77, 118, 216; 61 x 47 x 74, two fields (1744): 509, 383, 542, 965; 32^2
     // (18): 31, 51, 91, 172.
+    const int64_t want = (int64_t)ctx->num_cu * 4 * 9 / 16 * 64;  // threads
     int R = 1;
-    while (R < 16 && cols * ((G.ni[D - 1] + 2 * R) / (2 * R)) >= (int64_t)576 * 64) R *= 2;
+    while (R < 16 && cols * ((G.ni[D - 1] + 2 * R) / (2 * R)) >= want) R *= 2;
     const int64_t threads = cols * ((G.ni[D - 1] + R) / R);
     // up to three fields per launch (their sums are independent: every launch
     // computes the same weights); four would spill
