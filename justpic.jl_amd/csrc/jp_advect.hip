@@ -377,9 +377,11 @@ __global__ void __launch_bounds__(kBlock) k_advect_slot(Grid<D> g, Vel<D> vg, VP
 // coordinates and inverse spacings are staged too.  A bracket, and the nodal
 // values, come from the window when they lie in it and from global memory
 // otherwise, with the same tests and the same values as the slot kernel, so
-// the results are identical.  Bound by FP64 issue and LDS reads: RK2 98 us at
-// 512^2, RK4 594 us at 61 x 47 x 74; MQS RK2 88 us at 300 x 431 (the slot
-// kernel, which gathers its stencils from global memory: 191).
+// the results are identical.  Bound by latency, of LDS reads and dependent FP64
+// operations: the VALUs are busy 43% of the time at 512^2 (RK2, 98 us, 2.9
+// wavefronts per SIMD) and 41% at 61 x 47 x 74 (RK4, 594 us, 1.7: 173 registers
+// and 60 KB of LDS).  MQS RK2 85 us at 300 x 431 (the slot kernel, which gathers
+// its stencils from global memory: 191).
 template <int D>
 struct F64Tile;
 template <>

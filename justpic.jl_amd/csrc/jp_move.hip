@@ -467,8 +467,9 @@ struct alignas(16) NbEntry {
 // loop over the mover bits with two dependent LDS reads, arrival words updated
 // per mover and an origin stored for every processing took 105 us for the
 // tiled 2D phases at 512^2 (32^2: 87, 3D 128^3: 30.9 per phase), this one 51
-// (38, 26.6).  Of that, origins stored for the tile's own cells only: 74 -> 58,
-// in 16 bits: 58 -> 51 (scattered stores, each a cache line).
+// (38; 3D 22.6, 4 of it by loading the neighbours' words in one round).  Of
+// that, origins stored for the tile's own cells only: 74 -> 58, in 16 bits:
+// 58 -> 51 (scattered stores, each a cache line).
 //
 // at(code): the entry of a code's destination.
 template <int D, bool STATS, typename At>

@@ -169,7 +169,7 @@ __device__ inline void window_limits(const SVelIn<D>& V, SWindow<D>& W) {
 // The velocity at cell I + offset u from the windows; false unless they hold every
 // corner of every component.  One test of all and no branch before it: component
 // by component with early returns, an RK2 step in 3D spent 700 vector
-// instructions on a particle and as many scalar ones on execution masks, now 300
+// instructions on a particle and 400 scalar ones on execution masks, now 400 and 90
 // (128^3: advection 993 us -> 800, where 2.8 GB of slots take 610; 512^2: 62 -> 46).
 template <int D, class TS>
 __device__ inline bool interp_window(const float (*sV)[TS::size()], const SWindow<D>& W,
